@@ -57,6 +57,33 @@ def test_rmsnorm_rows_forward_backward(hip_device, dtype, w_dtype, N, d, rows):
         assert_close(np64(dw), rdw, **TOL[w_dtype], what="dw")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,chunks", [(3, 65), (3, 129), (3, 256), (3, 257), (5, 513), (5, 1025), (2, 2048),
+                                      (2100, 65), (1030, 257)])
+def test_rmsnorm_rows_layout_edges(hip_device, dtype, n, chunks):
+    """Each row layout (one wave or four per row, 1 to 8 chunks a thread) at its first and last
+    width, more rows than one sweep of the backward's blocks, and a weight whose storage does not
+    start on 16 bytes (the scalar weight loads)."""
+    from zmoe import ops
+
+    d = chunks * (16 // dtype.itemsize)
+    X, w, _ = _inputs(n, d, None, dtype, dtype, seed=n + chunks)
+    wd = torch.empty(d + 1, dtype=dtype, device=hip_device)[1:]
+    wd.copy_(w)
+    for wt in (w.to(hip_device), wd):
+        Y, rstd = ops.rmsnorm_rows(X.to(hip_device), wt, 1e-6)
+        ry, rr = O.zc_rmsnorm_rows(np64(X), np64(w), 1e-6)
+        assert_close(np64(Y), ry, **TOL[dtype], what="y")
+        dY = torch.randn(n, d, generator=gen(n * 7 + d)).to(dtype)
+        dX, dw = ops.rmsnorm_rows_backward(dY.to(hip_device), X.to(hip_device), None, rstd, wt)
+        rdX, rdw = O.zc_rmsnorm_rows_backward(np64(dY), np64(X), np64(w), rr)
+        assert_close(np64(dX), rdX, **TOL[dtype], what="dX")
+        if dtype == torch.float32 and n >= 256:  # fp32 sums over hundreds of rows: norm-wise (helpers.TOL)
+            assert_close_fro(np64(dw), rdw, what="dw")
+        else:
+            assert_close(np64(dw), rdw, **TOL[dtype], what="dw")
+
+
 def test_rmsnorm_rows_out_of_range_and_empty(hip_device):
     from zmoe import ops
 
