@@ -2,7 +2,8 @@
 
     python architecture-zarelga-superposition_amd/build_lib.py [-v] [--asan]
 
-Objects go to ``_build/`` next to this file; the library to ``zmoe/libzmoe_hip.so``.
+Objects go to ``_build/`` next to this file; the library to ``zmoe/libzmoe_hip.so``, and the
+torch dispatcher kernels over it (csrc/eager_ops.cpp) to ``zmoe/libzmoe_eager.so``.
 ``--asan``: the host-sanitized build for the CPU tests, ``_build/asan/libzmoe_hip_asan.so``.
 """
 
@@ -22,6 +23,7 @@ INCLUDE = os.path.join(REPO, "include")
 BUILD = os.path.join(HERE, "_build")
 GEN = os.path.join(BUILD, "gen")
 LIB = os.path.join(HERE, "zmoe", "libzmoe_hip.so")
+EAGER_LIB = os.path.join(HERE, "zmoe", "libzmoe_eager.so")
 ARCH = os.environ.get("ZMOE_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (the host pass warns that
@@ -118,7 +120,34 @@ def build(verbose: bool = False, jobs: int | None = None, asan: bool = False) ->
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + res.stdout + res.stderr)
     os.replace(tmp, lib)
+    if not asan:
+        build_eager_ops(verbose)
     return lib
+
+
+def build_eager_ops(verbose: bool = False) -> str:
+    """csrc/eager_ops.cpp (host code against torch's headers) into zmoe/libzmoe_eager.so, linked to
+    the C ABI library next to it."""
+    import torch
+    from torch.utils import cpp_extension
+
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    rocm = os.path.dirname(os.path.dirname(hipcc()))
+    tmp = EAGER_LIB + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE,
+           *(arg for path in cpp_extension.include_paths() for arg in ("-isystem", path)),
+           "-isystem", os.path.join(rocm, "include"), os.path.join(CSRC, "eager_ops.cpp"), "-o", tmp,
+           "-L", torch_lib, "-lc10", "-lc10_hip", "-ltorch_cpu", "-L", os.path.dirname(LIB), "-lzmoe_hip",
+           "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("eager ops failed to build:\n" + res.stdout + res.stderr)
+    os.replace(tmp, EAGER_LIB)
+    return EAGER_LIB
 
 
 if __name__ == "__main__":

@@ -13,6 +13,7 @@ from typing import Optional
 import torch
 
 from zmoe import ops as _z
+from zmoe.library import layer_op
 
 BLOCK_M = 128  # kept for API compatibility (reference ops.py:6); tiles are chosen per launch
 
@@ -29,7 +30,7 @@ def rowwise_sum_product(A, B, dtype=None):
     return output
 
 
-@torch.library.custom_op("zmoe::rowwise_sum_product", mutates_args={"output"})
+@layer_op("rowwise_sum_product", mutates_args=("output",))
 def rowwise_sum_product_compileable(output: torch.Tensor, A: torch.Tensor, B: torch.Tensor) -> None:
     _z.rowwise_sum_product(A, B, out=output)
 
@@ -57,7 +58,7 @@ def scatter2scatter(X, W, sorted_expert_idxs, sorted_scattered_idxs, k, b=None, 
     return output
 
 
-@torch.library.custom_op("zmoe::scatter2scatter", mutates_args={"output"})
+@layer_op("scatter2scatter", mutates_args=("output",))
 def scatter2scatter_compileable(output: torch.Tensor, W: torch.Tensor, X: torch.Tensor, k: int,
                                 sorted_expert_idxs: torch.Tensor, sorted_scattered_idxs: torch.Tensor,
                                 b: Optional[torch.Tensor], x_grouped: bool, y_grouped: bool,
@@ -81,7 +82,7 @@ def group_bwd_W(DY, X, expert_offsets, E, has_bias=False):
     return DW, Db
 
 
-@torch.library.custom_op("zmoe::groupXtY", mutates_args={"DW", "Db"})
+@layer_op("groupXtY", mutates_args=("DW", "Db",))
 def groupXtY_compileable(E: int, DW: torch.Tensor, Db: Optional[torch.Tensor], DY: torch.Tensor, X: torch.Tensor,
                          expert_offsets: torch.Tensor) -> None:
     DWt = DW.permute(0, 2, 1)
@@ -105,7 +106,7 @@ def group(A, sorted_expert_idxs, coeff=None, fan_out=1, out=None):
     return Y
 
 
-@torch.library.custom_op("zmoe::group", mutates_args={"Y"})
+@layer_op("group", mutates_args=("Y",))
 def group_compileable(A: torch.Tensor, K: int, N: int, Y: torch.Tensor, coeff: Optional[torch.Tensor],
                       has_coeff: bool, fan_out: int, sorted_expert_idxs: torch.Tensor) -> None:
     _z.group(A, sorted_expert_idxs, coeff=coeff if has_coeff else None, fan_out=fan_out, out=Y)

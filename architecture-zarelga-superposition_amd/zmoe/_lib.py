@@ -12,6 +12,7 @@ import threading
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libzmoe_hip.so")
+EAGER_PATH = os.path.join(_HERE, "libzmoe_eager.so")  # torch dispatcher kernels over the C ABI
 
 DTYPE_F32 = 0
 DTYPE_BF16 = 1

@@ -13,14 +13,90 @@ ctypes) on the current stream.
 
 from __future__ import annotations
 
+import functools
+import inspect
+import os
+import threading
 from typing import List, Optional
 
 import torch
 
+from . import _lib as L
 from . import ops as _z
+from . import profiling
 
 _I64 = torch.int64
 _F32 = torch.float32
+
+_eager_fakes = []   # (name, fake implementation) to register once the native ops are loaded
+_eager_lock = threading.Lock()
+
+
+def _load_eager():
+    """The native ops (csrc/eager_ops.cpp), loaded once; there is no fallback if they are missing."""
+    global _eager_fakes
+    with _eager_lock:
+        if _eager_fakes is not None:
+            L.load()  # the C ABI library they call
+            if not os.path.exists(L.EAGER_PATH):
+                raise ImportError(f"{os.path.basename(L.EAGER_PATH)} not found at {L.EAGER_PATH}; build it first "
+                                  "(python architecture-zarelga-superposition_amd/build_lib.py)")
+            torch.ops.load_library(L.EAGER_PATH)
+            for name, fake in _eager_fakes:
+                torch.library.register_fake(f"zmoe_eager::{name}", fake)
+            _eager_fakes = None
+
+
+def layer_op(name: str, mutates_args=()):
+    """``torch.library.custom_op("zmoe::<name>")``, with the native ``zmoe_eager::<name>`` of
+    csrc/eager_ops.cpp for eager calls with gradients off.
+
+    The layer calls its ops from inside autograd functions, where grad mode is off and there is
+    nothing to record; a small layer's step is bound by the host time of its ~25 calls, most of
+    it custom_op's Python (autograd kernel, redispatch, alias check) and the wrapper's. The
+    native op is an ordinary dispatcher kernel, so modes, fake tensors and profilers see it. With
+    grad mode on (a caller outside an autograd function, or a backward with create_graph) the
+    call goes to the custom_op, which refuses a backward through it; while compiling too, so
+    compiled graphs hold the zmoe:: names, with a symbolic size (the native ops take integers),
+    and while zmoe.profiling times single launches."""
+
+    def wrap(fn):
+        custom = torch.library.custom_op(f"zmoe::{name}", mutates_args=mutates_args)(fn)
+        params = tuple(inspect.signature(fn).parameters)
+        mutated = tuple(params.index(m) for m in mutates_args)
+        native = None
+
+        @functools.wraps(fn)
+        def call(*args, **kwargs):
+            nonlocal native
+            if (kwargs or torch.is_grad_enabled() or torch.compiler.is_compiling() or profiling.active()
+                    or torch.SymInt in map(type, args)):
+                return custom(*args, **kwargs)
+            if native is None:
+                _load_eager()
+                native = getattr(torch.ops.zmoe_eager, name).default
+            out = native(*args)
+            for i in mutated:  # as custom_op does: autograd sees that the tensor changed
+                if i < len(args) and args[i] is not None:
+                    torch.autograd.graph.increment_version(args[i])
+            return out
+
+        def register_fake(fake):
+            custom.register_fake(fake)
+            with _eager_lock:
+                if _eager_fakes is None:  # the native ops are loaded already
+                    torch.library.register_fake(f"zmoe_eager::{name}", fake)
+                else:
+                    _eager_fakes.append((name, fake))
+            return fake
+
+        call.register_fake = register_fake
+        for method in ("register_kernel", "register_autograd", "register_vmap", "register_torch_dispatch",
+                       "set_kernel_enabled"):
+            setattr(call, method, getattr(custom, method))
+        return call
+
+    return wrap
 
 
 def _empty(shape, like: torch.Tensor, dtype=None):
@@ -28,7 +104,7 @@ def _empty(shape, like: torch.Tensor, dtype=None):
 
 
 # ------------------------------------------------------------------ routing
-@torch.library.custom_op("zmoe::route_topk", mutates_args=())
+@layer_op("route_topk")
 def route_topk(logits: torch.Tensor, expert_biases: torch.Tensor, k: int,
                round_probs_bf16: bool) -> List[torch.Tensor]:
     """moe_gate.py:27-34 from the logits: [idx int64, weight f32, prob f32], each [T, k]."""
@@ -41,7 +117,7 @@ def _(logits, expert_biases, k, round_probs_bf16):
     return [_empty((T, k), logits, _I64), _empty((T, k), logits, _F32), _empty((T, k), logits, _F32)]
 
 
-@torch.library.custom_op("zmoe::swiglu_route_backward", mutates_args=())
+@layer_op("swiglu_route_backward")
 def swiglu_route_backward(dAs: torch.Tensor, Hs: torch.Tensor, d_gates: torch.Tensor, topk_prob: torch.Tensor,
                           topk_idx: torch.Tensor, num_experts: int) -> torch.Tensor:
     """[swiglu_backward(dAs, Hs) | d_logits] side by side in one [T, 2f + E] buffer: the
@@ -58,7 +134,7 @@ def _(dAs, Hs, d_gates, topk_prob, topk_idx, num_experts):
     return _empty((Hs.shape[0], Hs.shape[1] + num_experts), Hs)
 
 
-@torch.library.custom_op("zmoe::route_topk_backward", mutates_args=())
+@layer_op("route_topk_backward")
 def route_topk_backward(d_weight: torch.Tensor, topk_prob: torch.Tensor, topk_idx: torch.Tensor, num_experts: int,
                         like: torch.Tensor) -> torch.Tensor:
     """d_logits [T, E] in ``like``'s dtype."""
@@ -71,7 +147,7 @@ def _(d_weight, topk_prob, topk_idx, num_experts, like):
 
 
 # ------------------------------------------------------------------ sort
-@torch.library.custom_op("zmoe::flatten_sort_count", mutates_args=())
+@layer_op("flatten_sort_count")
 def flatten_sort_count(expert_idxs: torch.Tensor, num_experts: int) -> List[torch.Tensor]:
     """parallel_experts.py:21-28: [sorted_expert_idxs, sorted_scattered_idxs, expert_offsets,
     inverse int32]."""
@@ -86,7 +162,7 @@ def _(expert_idxs, num_experts):
 
 
 # ------------------------------------------------------------------ grouped GEMMs
-@torch.library.custom_op("zmoe::glu_w1_forward", mutates_args=())
+@layer_op("glu_w1_forward")
 def glu_w1_forward(x: torch.Tensor, W1: torch.Tensor, sorted_expert_idxs: torch.Tensor,
                    sorted_scattered_idxs: torch.Tensor, expert_offsets: torch.Tensor, k: int,
                    row_scale: Optional[torch.Tensor]) -> List[torch.Tensor]:
@@ -103,7 +179,7 @@ def _(x, W1, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, row_s
     return [_empty((R, two_f), x), _empty((R, two_f // 2), x)]
 
 
-@torch.library.custom_op("zmoe::grouped_mm", mutates_args=())
+@layer_op("grouped_mm")
 def grouped_mm(X: torch.Tensor, W: torch.Tensor, sorted_expert_idxs: torch.Tensor,
                sorted_scattered_idxs: torch.Tensor, k: int, x_grouped: bool, y_grouped: bool,
                expert_offsets: torch.Tensor, region: str) -> torch.Tensor:
@@ -117,7 +193,7 @@ def _(X, W, sorted_expert_idxs, sorted_scattered_idxs, k, x_grouped, y_grouped, 
     return _empty((sorted_expert_idxs.shape[0], W.shape[2]), X)
 
 
-@torch.library.custom_op("zmoe::glu_w2_backward_dh", mutates_args=())
+@layer_op("glu_w2_backward_dh")
 def glu_w2_backward_dh(dYg: torch.Tensor, W2: torch.Tensor, H: torch.Tensor, sorted_expert_idxs: torch.Tensor,
                        expert_offsets: torch.Tensor) -> torch.Tensor:
     """dH [T*k, 2f]: the W2 input-grad GEMM with the SwiGLU backward epilogue."""
@@ -133,7 +209,7 @@ def _wdt(DY: torch.Tensor, out_f32: bool) -> torch.dtype:
     return torch.float32 if out_f32 else DY.dtype
 
 
-@torch.library.custom_op("zmoe::group_bwd_w", mutates_args=())
+@layer_op("group_bwd_w")
 def group_bwd_w(DY: torch.Tensor, X: torch.Tensor, expert_offsets: torch.Tensor, num_experts: int,
                 x_gather: Optional[torch.Tensor], x_div: int, out_f32: bool = False) -> torch.Tensor:
     """group_bwd_W (ops.py:263-271): DWt [E, N, K] (the parameter layout); ``out_f32``: fp32
@@ -147,7 +223,7 @@ def _(DY, X, expert_offsets, num_experts, x_gather, x_div, out_f32=False):
     return _empty((num_experts, DY.shape[1], X.shape[1]), DY, _wdt(DY, out_f32))
 
 
-@torch.library.custom_op("zmoe::group_bwd_w_bias", mutates_args=())
+@layer_op("group_bwd_w_bias")
 def group_bwd_w_bias(DY: torch.Tensor, X: torch.Tensor, expert_offsets: torch.Tensor, num_experts: int,
                      x_gather: Optional[torch.Tensor], x_div: int) -> List[torch.Tensor]:
     """group_bwd_W with has_bias (ops.py:263-271, :430-438): [DWt [E, N, K], Db [E, N]]."""
@@ -159,7 +235,7 @@ def _(DY, X, expert_offsets, num_experts, x_gather, x_div):
     return [_empty((num_experts, DY.shape[1], X.shape[1]), DY), _empty((num_experts, DY.shape[1]), DY)]
 
 
-@torch.library.custom_op("zmoe::group_bwd_w_gather_dy", mutates_args=())
+@layer_op("group_bwd_w_gather_dy")
 def group_bwd_w_gather_dy(DY: torch.Tensor, dy_gather: torch.Tensor, dy_div: int, X: torch.Tensor,
                           expert_offsets: torch.Tensor, num_experts: int, out_f32: bool = False) -> torch.Tensor:
     """Weight grads with DY's rows gathered in the kernel: DWt [E, N, K]."""
@@ -172,7 +248,7 @@ def _(DY, dy_gather, dy_div, X, expert_offsets, num_experts, out_f32=False):
     return _empty((num_experts, DY.shape[1], X.shape[1]), DY, _wdt(DY, out_f32))
 
 
-@torch.library.custom_op("zmoe::dense_wgrad", mutates_args=())
+@layer_op("dense_wgrad")
 def dense_wgrad(DY: torch.Tensor, X: torch.Tensor, out_f32: bool = False) -> torch.Tensor:
     """DW [N, K] = DY^T X (the F.linear weight grad, split-K)."""
     return _z.dense_wgrad(DY, X, out_dtype=_wdt(DY, out_f32))
@@ -184,7 +260,7 @@ def _(DY, X, out_f32=False):
 
 
 # ------------------------------------------------------------------ row passes
-@torch.library.custom_op("zmoe::combine", mutates_args=())
+@layer_op("combine")
 def combine(Y: torch.Tensor, gates: Optional[torch.Tensor], k: int, addend: Optional[torch.Tensor],
             out_rows: Optional[torch.Tensor], out_total: int) -> torch.Tensor:
     """out[t] = addend[t] + sum_j gates[t, j] Y[t*k + j] ([T, d], or the padded [out_total, d]
@@ -199,7 +275,7 @@ def _(Y, gates, k, addend, out_rows, out_total):
     return _empty((rows, Y.shape[1]), Y)
 
 
-@torch.library.custom_op("zmoe::combine_backward", mutates_args=())
+@layer_op("combine_backward")
 def combine_backward(Y: torch.Tensor, grad_out: torch.Tensor, gates: torch.Tensor, inverse: torch.Tensor,
                      grad_rows: Optional[torch.Tensor]) -> List[torch.Tensor]:
     """[d_gates [T, k] f32, gate-scaled grad rows [T*k, d] in sorted order]."""
@@ -212,7 +288,7 @@ def _(Y, grad_out, gates, inverse, grad_rows):
     return [_empty((T, k), gates, _F32), _empty((T * k, Y.shape[-1]), Y)]
 
 
-@torch.library.custom_op("zmoe::sum_k", mutates_args=())
+@layer_op("sum_k")
 def sum_k(Xe: torch.Tensor, k: int, add0: Optional[torch.Tensor], out_f32: bool = False) -> torch.Tensor:
     """out[t] = sum_j Xe[t*k + j] (+ add0[t]) (parallel_experts.py:125); ``out_f32``: the fp32
     sum unrounded."""
@@ -224,7 +300,7 @@ def _(Xe, k, add0, out_f32=False):
     return _empty((Xe.shape[0] // k, Xe.shape[1]), Xe, torch.float32 if out_f32 else None)
 
 
-@torch.library.custom_op("zmoe::cast_bf16", mutates_args=())
+@layer_op("cast_bf16")
 def cast_bf16(src: torch.Tensor) -> torch.Tensor:
     """The bf16 compute copy of an fp32 tensor (fp32 master weights under bf16 autocast)."""
     return _z.cast_bf16(src).clone() if src.dtype == torch.bfloat16 else _z.cast_bf16(src)
@@ -235,7 +311,7 @@ def _(src):
     return _empty(src.shape, src, torch.bfloat16)
 
 
-@torch.library.custom_op("zmoe::swiglu", mutates_args=())
+@layer_op("swiglu")
 def swiglu(H: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up for H = [up | gate] (mlp.py:86, expert_layer.py:23-24)."""
     return _z.swiglu(H)
@@ -246,7 +322,7 @@ def _(H):
     return _empty((H.shape[0], H.shape[1] // 2), H)
 
 
-@torch.library.custom_op("zmoe::swiglu_backward", mutates_args=())
+@layer_op("swiglu_backward")
 def swiglu_backward(dA: torch.Tensor, H: torch.Tensor) -> torch.Tensor:
     return _z.swiglu_backward(dA, H)
 
@@ -256,7 +332,7 @@ def _(dA, H):
     return _empty(H.shape, H)
 
 
-@torch.library.custom_op("zmoe::swiglu_backward_gates", mutates_args=())
+@layer_op("swiglu_backward_gates")
 def swiglu_backward_gates(dA: torch.Tensor, H: torch.Tensor, row_scale: torch.Tensor,
                           slot_of_row: torch.Tensor) -> List[torch.Tensor]:
     """[dH [R, 2f], d_gates [R] f32 in slot order] of gate-scaled rows."""
@@ -268,7 +344,7 @@ def _(dA, H, row_scale, slot_of_row):
     return [_empty(H.shape, H), _empty((H.shape[0],), H, _F32)]
 
 
-@torch.library.custom_op("zmoe::rmsnorm_rows", mutates_args=())
+@layer_op("rmsnorm_rows")
 def rmsnorm_rows(X: torch.Tensor, weight: torch.Tensor, eps: float, rows: Optional[torch.Tensor]) -> List[torch.Tensor]:
     """[Y [n, d], rstd [n] f32]: zRMSNorm.py:10-17 on rows ``rows`` of X."""
     return list(_z.rmsnorm_rows(X, weight, eps, rows))
@@ -280,7 +356,7 @@ def _(X, weight, eps, rows):
     return [_empty((n, X.shape[1]), X), _empty((n,), X, _F32)]
 
 
-@torch.library.custom_op("zmoe::rmsnorm_rows_backward", mutates_args=())
+@layer_op("rmsnorm_rows_backward")
 def rmsnorm_rows_backward(dY: torch.Tensor, X: torch.Tensor, rows: Optional[torch.Tensor], rstd: torch.Tensor,
                           weight: torch.Tensor) -> List[torch.Tensor]:
     """[dX [N, d] (zeros outside ``rows``), dweight]."""

@@ -34,6 +34,11 @@ def region(name: str, dev):
     return _timed(name, dev) if name in _enabled else _NULL
 
 
+def active() -> bool:
+    """Whether any launch is being timed (the layer's ops then run their Python wrappers)."""
+    return bool(_enabled)
+
+
 def enable(*names: str) -> None:
     _enabled.update(names)
 
