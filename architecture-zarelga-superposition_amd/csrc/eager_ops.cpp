@@ -2,7 +2,7 @@
 // zmoe/library.py run with gradients off. Each takes the operands that the layer itself passes
 // (device tensors of one device, bf16 or f32 rows, int64 indices), allocates its outputs with
 // torch and makes one C-ABI call on torch's current stream. Everything else (other dtypes and
-// devices, widths the kernels do not take, bad sizes) goes to the op's general form, the Python
+// devices, strides the kernels do not take, bad sizes) goes to the op's general form, the Python
 // wrapper registered as zmoe::<name>, which converts, pads or raises.
 //
 // Why native: a training step of a small layer is bound by its host work. An op costs ~20-40 us
@@ -15,7 +15,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
-#include <initializer_list>
+#include <algorithm>
 #include <limits>
 #include <optional>
 #include <string>
@@ -66,6 +66,27 @@ Tensor workspace(size_t bytes, const Tensor& like) {
 template <typename T> T* ptr(const Tensor& t) { return static_cast<T*>(t.data_ptr()); }
 void* raw(const Tensor& t) { return t.data_ptr(); }
 const int64_t* ids(const Tensor& t) { return ptr<const int64_t>(t); }
+
+// ------------------------------------------------------------------ padded copies
+// Widths that are not whole 16-byte chunks go through zero-padded copies, as in zmoe.ops.
+int64_t vec(const Tensor& t) { return 16 / (int64_t)t.element_size(); }
+int64_t up(int64_t n, const Tensor& like) { return (n + vec(like) - 1) / vec(like) * vec(like); }
+
+// src [r, c] or [b, r, c] (unit last stride) -> dst [rows, cols] or [b, rows, cols], cut or
+// zero-filled; false on an error.
+bool copy_pad_into(const Tensor& src, const Tensor& dst) {
+  const int64_t nd = src.dim();
+  const int64_t rows = dst.size(-2), cols = dst.size(-1);
+  return zmoe_copy_pad(raw(src), nd == 3 ? src.stride(0) : 0, src.stride(-2), nd == 3 ? src.size(0) : 1,
+                       std::min(rows, src.size(-2)), std::min(cols, src.size(-1)), code(src), raw(dst), rows, cols,
+                       stream_of(src)) == ZMOE_OK;
+}
+// The padded copy, or src itself where it has that size (undefined on an error).
+Tensor padded(const Tensor& src, int64_t rows, int64_t cols) {
+  if (src.size(-2) == rows && src.size(-1) == cols) return src;
+  Tensor dst = src.dim() == 3 ? empty({src.size(0), rows, cols}, src) : empty({rows, cols}, src);
+  return copy_pad_into(src, dst) ? dst : Tensor();
+}
 
 // ------------------------------------------------------------------ routing and sort
 Tensors route_topk(const Tensor& logits, const Tensor& bias, int64_t k, bool round) {
@@ -172,6 +193,19 @@ bool grouped_into(const Tensor& X, const Tensor& W, const Opt& b, const Tensor& 
   const int64_t M = X.size(0), E = W.size(0), K = W.size(1), N = W.size(2), R = M * k;
   if (!(index(se, X, R) && index(ss, X, R) && index(off, X, E) && out.size(0) == R && out.size(1) == N)) return false;
   if (b && !(flat(*b, X, X.scalar_type()) && b->dim() == 2 && b->size(0) == E && b->size(1) == N)) return false;
+  const int64_t Kp = up(K, X), Np = up(N, X);
+  if (Kp != K || Np != N) {
+    if (!out.is_contiguous()) return false;
+    const Tensor Xp = padded(X, M, Kp);
+    // in its storage order: unit stride along K (the nn.Linear layout) or along N
+    Tensor Wp = W.stride(1) == 1 ? padded(W.permute({0, 2, 1}), Np, Kp) : padded(W, Kp, Np);
+    const Tensor bp = b ? padded(*b, E, Np) : Tensor();
+    if (!Xp.defined() || !Wp.defined() || (b && !bp.defined())) return false;
+    if (W.stride(1) == 1) Wp = Wp.permute({0, 2, 1});
+    const Tensor Y = Np == N ? out : empty({R, Np}, X);
+    return grouped_into(Xp, Wp, b ? Opt(bp) : std::nullopt, se, ss, k, xg, yg, off, Y) &&
+           (Np == N || copy_pad_into(Y, out));
+  }
   return zmoe_scatter2scatter(raw(X), X.stride(0), raw(W), W.stride(0), W.stride(1), W.stride(2), b ? raw(*b) : nullptr,
                               b ? b->stride(0) : 0, ids(se), ids(ss), ids(off), M, K, N, (int)E, (int)k, xg, yg,
                               code(X), raw(out), out.stride(0), stream_of(X)) == ZMOE_OK;
@@ -223,6 +257,14 @@ bool wgrad_into(const Tensor& DY, const Tensor& X, const Tensor& off, int64_t E,
   if (!(DY.is_cuda() && known(DY) && rows2(DY, DY) && rows2(X, DY) && index(off, DY, E) && fits_int(E) &&
         fits_int(div) && (gather ? index(*gather, DY, DY.size(0)) : X.size(0) == DY.size(0))))
     return false;
+  const int64_t N = DY.size(1), K = X.size(1), Np = up(N, DY), Kp = up(K, X);
+  if (Np != N || Kp != K) {
+    const Tensor DYp = padded(DY, DY.size(0), Np), Xp = padded(X, X.size(0), Kp);
+    if (!DYp.defined() || !Xp.defined()) return false;
+    const Tensor dWp = empty({E, Np, Kp}, dW), dbp = db && Np != N ? empty({E, Np}, *db) : Tensor();
+    return wgrad_into(DYp, Xp, off, E, gather, div, dWp, dbp.defined() ? Opt(dbp) : db) && copy_pad_into(dWp, dW) &&
+           (!dbp.defined() || copy_pad_into(dbp, *db));
+  }
   return zmoe_group_bwd_w(raw(DY), DY.stride(0), raw(X), X.stride(0), gather ? ids(*gather) : nullptr, (int)div,
                           ids(off), DY.size(0), DY.size(1), X.size(1), (int)E, code(DY), code(dW), raw(dW),
                           db ? raw(*db) : nullptr, stream_of(DY)) == ZMOE_OK;
@@ -316,6 +358,15 @@ Tensor combine(const Tensor& Y, const Opt& gates, int64_t k, const Opt& addend, 
         (!addend || (flat(*addend, Y, Y.scalar_type()) && addend->numel() == T * d)) &&
         (!out_rows || (index(*out_rows, Y, T) && out_total >= 0))) {
       const c10::DeviceGuard guard(Y.device());
+      if (const int64_t dp = up(d, Y); dp != d) {
+        const Tensor Yp = padded(Y, T * k, dp);
+        const Tensor ap = addend ? padded(addend->view({T, d}), T, dp) : Tensor();
+        if (Yp.defined() && (!addend || ap.defined())) {
+          const Tensor full = combine(Yp, gates, k, addend ? Opt(ap) : std::nullopt, out_rows, out_total);
+          Tensor out = empty({full.size(0), d}, Y);
+          if (copy_pad_into(full, out)) return out;
+        }
+      }
       const float* g = gates ? ptr<const float>(*gates) : nullptr;
       const void* add = addend ? raw(*addend) : nullptr;
       if (!out_rows) {
@@ -363,6 +414,14 @@ Tensor sum_k(const Tensor& Xe, int64_t k, const Opt& add0, bool out_f32) {
     const int64_t T = Xe.size(0) / k, d = Xe.size(1);
     if (!add0 || (flat(*add0, Xe, Xe.scalar_type()) && add0->numel() == T * d)) {
       const c10::DeviceGuard guard(Xe.device());
+      if (const int64_t dp = up(d, Xe); dp != d) {
+        const Tensor Xp = padded(Xe, T * k, dp), ap = add0 ? padded(add0->view({T, d}), T, dp) : Tensor();
+        if (Xp.defined() && (!add0 || ap.defined())) {
+          const Tensor full = sum_k(Xp, k, add0 ? Opt(ap) : std::nullopt, out_f32);
+          Tensor out = empty({T, d}, full);
+          if (copy_pad_into(full, out)) return out;
+        }
+      }
       Tensor out = empty({T, d}, Xe, wgrad_dtype(Xe, out_f32));
       if (zmoe_sum_k(raw(Xe), T, (int)k, d, code(Xe), add0 ? raw(*add0) : nullptr, nullptr, code(out), raw(out),
                      stream_of(Xe)) == ZMOE_OK)
@@ -473,18 +532,29 @@ void rowwise_sum_product(const Tensor& out, const Tensor& A, const Tensor& B) {
   op.call(out, A, B);
 }
 
-void group(const Tensor& A, int64_t K, int64_t N, const Tensor& Y, const Opt& coeff, bool has_coeff, int64_t fan_out,
-           const Tensor& idx) {
+// Y = the grouped rows; false where the general form has to run.
+bool group_into(const Tensor& A, const Tensor& Y, const Opt& coeff, bool has_coeff, int64_t fan_out,
+                const Tensor& idx) {
   const bool use = has_coeff && coeff;
   if (A.is_cuda() && known(A) && rows2(A, A) && fan_out > 0 && fits_int(fan_out) &&
       index(idx, A, A.size(0) * fan_out) && rows2(Y, A) && Y.size(0) == idx.numel() && Y.size(1) == A.size(1) &&
       (!use || (on(*coeff, A) && known(*coeff) && coeff->is_contiguous() && coeff->numel() == idx.numel()))) {
     const c10::DeviceGuard guard(A.device());
-    if (zmoe_group(raw(A), A.stride(0), A.size(1), code(A), ids(idx), idx.numel(), (int)fan_out,
-                   use ? raw(*coeff) : nullptr, use ? code(*coeff) : ZMOE_DTYPE_F32, raw(Y), Y.stride(0),
-                   stream_of(A)) == ZMOE_OK)
-      return;
+    if (const int64_t Kp = up(A.size(1), A); Kp != A.size(1)) {
+      if (!Y.is_contiguous()) return false;
+      const Tensor Ap = padded(A, A.size(0), Kp), Yp = empty({Y.size(0), Kp}, Y);
+      return Ap.defined() && group_into(Ap, Yp, coeff, has_coeff, fan_out, idx) && copy_pad_into(Yp, Y);
+    }
+    return zmoe_group(raw(A), A.stride(0), A.size(1), code(A), ids(idx), idx.numel(), (int)fan_out,
+                      use ? raw(*coeff) : nullptr, use ? code(*coeff) : ZMOE_DTYPE_F32, raw(Y), Y.stride(0),
+                      stream_of(A)) == ZMOE_OK;
   }
+  return false;
+}
+
+void group(const Tensor& A, int64_t K, int64_t N, const Tensor& Y, const Opt& coeff, bool has_coeff, int64_t fan_out,
+           const Tensor& idx) {
+  if (group_into(A, Y, coeff, has_coeff, fan_out, idx)) return;
   static const auto op = general<void(const Tensor&, c10::SymInt, c10::SymInt, const Tensor&, const Opt&, bool,
                                       c10::SymInt, const Tensor&)>("zmoe::group");
   op.call(A, K, N, Y, coeff, has_coeff, fan_out, idx);

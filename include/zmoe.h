@@ -311,6 +311,14 @@ int zmoe_sum_k(const void* Xe, int64_t T, int k, int64_t d, int dtype,
  * even, NaN kept. src and dst 16-byte aligned. */
 int zmoe_cast_f32_bf16(const float* src, int64_t n, void* dst, void* stream);
 
+/* dst [batch, dst_rows, dst_cols] (contiguous) = src[b, r, c] where r < rows and c < cols, else
+ * 0; src has strides (src_stride_b, src_stride_r, 1). The padded copies that rows of a width
+ * the other entry points do not take (not whole 16-byte chunks) go through, and back. Pointers
+ * and strides need the element's alignment only. */
+int zmoe_copy_pad(const void* src, int64_t src_stride_b, int64_t src_stride_r, int64_t batch,
+                  int64_t rows, int64_t cols, int dtype, void* dst, int64_t dst_rows,
+                  int64_t dst_cols, void* stream);
+
 /* scattermoe/mlp.py:86 stand-alone (shapes the fused kernels reject):
  * A = silu(H[:, f:]) * H[:, :f]; and its backward dH from (dA, H), rows of dH
  * ld_dh >= 2f elements apart (2f for a packed [R, 2f]). */

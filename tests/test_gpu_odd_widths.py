@@ -154,3 +154,42 @@ def test_moe_layer_odd_hidden_size(hip_device):
         # the composition rounds a few more intermediates than the oracle models (torch's silu
         # and product as separate bf16 ops): two rss allowances, as for the two-path comparison
         assert_close(np64(p.grad), g[keys[n]], **tol, what=n, rss=2 * g["rss"][keys[n]])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("batch,rows,cols,drows,dcols", [
+    (1, 5, 1, 5, 8), (1, 1, 1031, 1, 1032), (3, 7, 513, 9, 516), (2, 6, 40, 5, 33), (1, 4, 512, 4, 511),
+    (1, 0, 9, 3, 9), (2, 3, 0, 3, 4), (1, 300001, 3, 300002, 8), (3, 100001, 5, 100000, 3)])
+def test_copy_pad(hip_device, dtype, batch, rows, cols, drows, dcols):
+    """The padded copy at its edges: one element, partial last chunks on either side, zero rows and
+    columns, cuts, more rows than one launch takes; a source that is a view starting off a 16-byte
+    boundary with rows further apart than they are long, into a NaN-filled output."""
+    from zmoe import ops
+
+    wide = torch.randn(batch, rows + 1, cols + 3, generator=gen(rows + cols)).to(dtype).to(hip_device)
+    src = wide[:, 1:, 1:cols + 1]
+    out = torch.full((batch, drows, dcols), float("nan"), dtype=dtype, device=hip_device)
+    ops.copy_pad(src, drows, dcols, out)
+    ref = torch.zeros(batch, drows, dcols, dtype=dtype, device=hip_device)
+    r, c = min(rows, drows), min(cols, dcols)
+    ref[:, :r, :c] = src[:, :r, :c]
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N", [8, 32, 40, 64, 136])
+def test_bias_grad_row_counts(hip_device, dtype, N):
+    """The bias grad where its rows are split differently: no rows, one, around the 128 row slots
+    of a block and the four rows a slot loads at once; column counts around a block's 128 bytes."""
+    from zmoe import ops
+
+    counts = [0, 1, 127, 128, 129, 0, 511, 513, 1300]
+    off = torch.tensor(np.cumsum(counts), device=hip_device)
+    g = gen(N)
+    DY = torch.randn(sum(counts), N, generator=g).to(dtype)
+    X = torch.randn(sum(counts), 16, generator=g).to(dtype)
+    _, Db = ops.group_bwd_w(DY.to(hip_device), X.to(hip_device), off, len(counts), has_bias=True)
+    ref = np.stack([r.sum(0) for r in np.split(np64(DY), np.cumsum(counts)[:-1])])
+    # fp32 sums of up to 1300 terms ~ N(0, 1): 1300 * 2^-24 * sum|terms| bounds any order
+    atol = max(TOL[dtype]["atol"], 1300 * 2.0 ** -24 * float(np.abs(np64(DY)).sum(0).max()))
+    assert_close(np64(Db), ref, rtol=TOL[dtype]["rtol"], atol=atol, what="bias grad")
