@@ -38,8 +38,8 @@
 //     for weight grads and for rows launches under skewed routing, slabs of 32
 //     consecutive tiles dealt to the XCDs in turn so that uneven per-tile costs
 //     even out (xcd_logical_tile, slab_logical_tile).
-// The f32 kernels use the same tiling with VGPR-staged loads, 32-deep stages and
-// v_mfma_f32_32x32x2f32 (four per 16-byte fragment).
+// The f32 kernels use the same tiling (128 x 128 or, where those are few, 64-row tiles) with
+// VGPR-staged loads, 32-deep stages and v_mfma_f32_32x32x2f32 (four per 16-byte fragment).
 #include <mutex>
 #include <type_traits>
 #include <unordered_set>
@@ -2619,6 +2619,20 @@ int launch_stream_rows(const RowsParams& p, hipStream_t s) {
   return check_launch("grouped rows streaming kernel");
 }
 
+// Tiles of BM rows that R rows in E experts come to, about (half a partial tile per expert).
+inline int64_t rows_tiles(int64_t R, int E, int BM) { return cdiv(R, BM) + (R < E ? R : E) / 2; }
+
+// f32 tiles of 64 rows (64 x 64, one 32 x 32 block per wave; 64 x 128 for SwiGLU) where 128 x 128
+// ones are fewer than about two per CU: a tile's time is then the latency of its own K loop
+// (register-staged loads, one stage ahead), and more, shorter tiles per CU overlap theirs.
+// Measured, us, 128 x 128 against 64 (tile counts of the former): T = 2048 d = 256 E = 8 k = 2
+// f = 512: W1 46 / 39 (320), W2 45 / 27 (72), its input grad 35 / 26 (144), dW2 68 / 35 (64), dW1
+// 93 / 60 (128), W1 input grad 87 / 53 (72); T = 8192 d = 512 E = 32 f = 160: W1 78 / 62 (432),
+// dW1 176 / 148 (384). Past that the larger tiles' reuse wins: T = 8192 d = 384 E = 16 f = 640:
+// dW1 268 / 309 (480); d = 512 E = 32 f = 160: W1 input grad 59 / 66 (576).
+constexpr int64_t kF32SmallTiles = 448;
+inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
+
 template <bool B_KN, int EPI>
 int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipStream_t s) {
   // n_tiles: along N (or along pair columns for SwiGLU, BN/2 pairs per tile)
@@ -2638,6 +2652,12 @@ int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipS
     }
     p.n_tiles = (int)cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128);
     return launch_rows_bf16<128, 128, B_KN, EPI>(p, R, s);
+  }
+  // SwiGLU pairs 32-column blocks inside a wave, so its tile stays 128 columns (64 pairs) wide
+  constexpr int BN = EPI == EPI_SWIGLU ? 128 : 64;
+  if (f32_small_tiles(rows_tiles(R, p.E, 128) * cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128))) {
+    p.n_tiles = (int)cdiv(bn_for_tiles_div, 64);
+    return launch_rows_f32<64, BN, B_KN, EPI>(p, R, s);
   }
   p.n_tiles = (int)cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128);
   return launch_rows_f32<128, 128, B_KN, EPI>(p, R, s);
@@ -3106,8 +3126,11 @@ extern "C" int zmoe_group_bwd_w(const void* DY, int64_t dy_stride_m, const void*
   if (dtype == ZMOE_DTYPE_BF16) {
     rc = group_bwd_w_bf16_out<false>(p, M, E, N, K, out_dtype, s);
   } else {
-    rc = launch_wgrad_kernel(grouped_wgrad_kernel<float, 128, 128>, rows_lds_bytes<float, 128, 128>(), 128, 128, p,
-                             s);
+    if (f32_small_tiles(E * cdiv(N, 128) * cdiv(K, 128)))
+      rc = launch_wgrad_kernel(grouped_wgrad_kernel<float, 64, 64>, rows_lds_bytes<float, 64, 64>(), 64, 64, p, s);
+    else
+      rc = launch_wgrad_kernel(grouped_wgrad_kernel<float, 128, 128>, rows_lds_bytes<float, 128, 128>(), 128, 128, p,
+                               s);
   }
   if (rc || Db == nullptr) return rc;
   const dim3 grid((unsigned)cdiv(N, 8 * v), (unsigned)E), block(kBiasThreads);

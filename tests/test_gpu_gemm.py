@@ -523,3 +523,45 @@ def test_dense_wgrad_f32(hip_device):
     X = torch.randn(777, 96, generator=g)
     DW = ops.dense_wgrad(DY.to(hip_device), X.to(hip_device), splits=4)
     assert_close_fro(np64(DW), np64(DY).T @ np64(X), what="dense_wgrad f32")  # 777-row fp32 sums
+
+
+@pytest.mark.parametrize("d,f", [(72, 136), (72, 2200)])  # under / over 448 tiles of 128 x 128 in every launch
+def test_f32_tile_sizes(hip_device, d, f):
+    """The f32 kernels with 64-row and with 128 x 128 tiles: row counts around both sizes, partial
+    column and K tiles, every operand form (gathered or grouped A, B along K or N, SwiGLU forward
+    and backward, weight grads with X gathered or not)."""
+    from zmoe import ops
+
+    counts, k = np.array([0, 1, 31, 63, 64, 65, 127, 128, 129, 300, 0, 192]), 2
+    E, R = len(counts), int(counts.sum())
+    se, ss, off = _fixed_routing(counts, k, hip_device, seed=19)
+    sn, en, on = ss.cpu().numpy(), se.cpu().numpy(), off.cpu().numpy()
+    g = gen(d + f)
+    x = torch.randn(R // k, d, generator=g)
+    W1 = torch.randn(E, 2 * f, d, generator=g) / d ** 0.5
+    W2 = torch.randn(E, d, f, generator=g) / f ** 0.5
+    H, A = ops.glu_w1_forward(x.to(hip_device), W1.to(hip_device), se, ss, off, k)
+    tol = TOL[torch.float32]
+    assert_close(np64(H), O.scatter2scatter(np64(x), np64(W1).transpose(0, 2, 1), en, sn, k, x_grouped=False,
+                                            y_grouped=True), **tol, what="H")
+    assert_close(np64(A), O.swiglu(np64(H)), **tol, what="A")
+    dY = torch.randn(R, d, generator=g)
+    dH = ops.glu_w2_backward_dh(dY.to(hip_device), W2.to(hip_device), H, se, off)
+    dA = O.scatter2scatter(np64(dY), np64(W2), en, sn, 1, x_grouped=True, y_grouped=True)
+    rdH = O.swiglu_backward(dA, np64(H))
+    assert_close(np64(dH), rdH, **tol, what="dH")
+    Y = ops.scatter2scatter(A, W2.to(hip_device).permute(0, 2, 1), se, ss, 1, x_grouped=True, expert_offsets=off)
+    # fp32 sums of f products: f * 2^-24 * sum|terms| bounds any order, ~ sqrt(f) of it is met
+    assert_close_fro(np64(Y), O.scatter2scatter(np64(A), np64(W2).transpose(0, 2, 1), en, sn, 1, x_grouped=True,
+                                                y_grouped=False), what="Y")
+    dx = ops.scatter2scatter(dH, W1.to(hip_device), se, ss, 1, x_grouped=True, expert_offsets=off)
+    assert_close_fro(np64(dx), O.scatter2scatter(np64(dH), np64(W1), en, sn, 1, x_grouped=True, y_grouped=False),
+                     what="dx")
+    dW1, _ = ops.group_bwd_w(dH, x.to(hip_device), off, E, x_gather=ss, x_div=k)
+    ref, _ = O.group_bwd_w(np64(dH), O.group(np64(x), sn, fan_out=k), on, E)
+    assert_close_fro(np64(dW1), ref.transpose(0, 2, 1), what="dW1")
+    dW2, _ = ops.group_bwd_w(dY.to(hip_device), A, off, E)
+    ref, _ = O.group_bwd_w(np64(dY), np64(A), on, E)
+    assert_close_fro(np64(dW2), ref.transpose(0, 2, 1), what="dW2")
+    for e in np.nonzero(counts == 0)[0]:
+        assert not dW1[e].any() and not dW2[e].any()
