@@ -1403,6 +1403,86 @@ __device__ __forceinline__ void kloop_small(int nk, lds_char* lds, int wm0, int 
   __builtin_amdgcn_s_waitcnt(vm_wait(0));  // loads past the end (zeros) are done before LDS is reused
 }
 
+// Stages of the ring K loop for a tile size of the rows kernel, 0: the double-buffered loops.
+constexpr int ring_stages(int BM, int BN, int NW) {
+  return (BM == 64 && BN == 128 && NW == 4) || (BM == 128 && BN == 256 && NW == 8) ? 3 : 0;
+}
+
+// The K loop of the tiles for experts of few rows (64 x 128 on 4 waves, two workgroups per CU, and
+// 128 x 256 on 8 waves): such launches stream every expert's weights for little MFMA work, so what
+// counts is how many bytes a CU keeps in flight. NS LDS stages, NS - 1 of them in flight while one
+// is read: per stage, wait for this wave's loads of it, barrier (every wave's loads are in, and
+// every wave is done with the stage before), issue the loads of the stage NS - 1 ahead into that
+// one's buffer, then read both 32-deep k-steps' fragments and multiply. Accumulators as in
+// kloop64_m16; dma_a / dma_b as in kloop_small.
+template <int NS, int NQA, int NQB, int MI, int NI, bool B_T, int BM, int BN, typename DmaA, typename DmaB,
+          typename Hook>
+__device__ __forceinline__ void kloop_ring(int nk, lds_char* lds, int wm0, int wn0, f32x4_t (&acc)[MI][NI][4],
+                                           DmaA dma_a, DmaB dma_b, Hook after_prologue_loads) {
+  constexpr int KS = 64;
+  constexpr int kA = BM * KS * 2;
+  constexpr int kS = kA + BN * KS * 2;
+  constexpr int AR = Frag16<false>::kReads, BR = Frag16<B_T>::kReads;
+  constexpr int NR = 2 * MI * AR + 2 * NI * BR;  // fragment reads per k-step
+  auto issue = [&](int buf, int kt, bool on) {
+    lds_char* st = lds + buf * kS;
+#pragma unroll
+    for (int q = 0; q < NQA; ++q) dma_a(q, st, kt, on);
+#pragma unroll
+    for (int q = 0; q < NQB; ++q) dma_b(q, st + kA, kt, on);
+  };
+  if (nk <= 0) {
+    after_prologue_loads();
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i) issue(i, i, nk > i);
+  after_prologue_loads();
+  Frag16<false> fa[2][MI][2];
+  Frag16<B_T> fb[2][NI][2];
+  int cur = 0;  // buffer of stage kt
+  for (int kt = 0; kt < nk; ++kt) {
+    __builtin_amdgcn_s_waitcnt(vm_wait((NS - 2) * (NQA + NQB)));  // stage kt has landed
+    asm volatile("s_barrier" ::: "memory");
+    issue(cur == 0 ? NS - 1 : cur - 1, kt + NS - 1, kt + NS - 1 < nk);
+    const lds_char* st = lds + cur * kS;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int f = 0; f < 2 * MI; ++f)
+#pragma unroll
+        for (int q = 0; q < AR; ++q) fa[j][f >> 1][f & 1].template read_piece<BM, KS>(st, wm0 + 16 * f, j, q);
+#pragma unroll
+      for (int f = 0; f < 2 * NI; ++f)
+#pragma unroll
+        for (int q = 0; q < BR; ++q) fb[j][f >> 1][f & 1].template read_piece<BN, KS>(st + kA, wn0 + 16 * f, j, q);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      if (j == 0) asm_wait_lgkm<NR>();  // (reads return in order; at most NR of the second k-step's are out)
+      else asm_wait_lgkm<0>();
+#pragma unroll
+      for (int f = 0; f < 2 * MI; ++f) fa[j][f >> 1][f & 1].tie();
+#pragma unroll
+      for (int f = 0; f < 2 * NI; ++f) fb[j][f >> 1][f & 1].tie();
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+              acc[mi][ni][2 * a + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  fb[j][ni][b].value(), fa[j][mi][a].value(), acc[mi][ni][2 * a + b], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    cur = cur == NS - 1 ? 0 : cur + 1;
+  }
+  __builtin_amdgcn_s_waitcnt(vm_wait(0));  // loads past the end (zeros) are done before LDS is reused
+}
+
 // Epilogues: each wave stages its own WM x WN accumulator block in its own LDS area
 // (bf16, rows of WN * 2 + 16 bytes) and writes it out row-contiguously, 16 bytes
 // per lane, so every store instruction covers whole 128-byte lines. The MFMA layout
@@ -1511,14 +1591,16 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
     // staged columns per 64: [h 32 | gate 32] for pair columns jj0 + 32 pb + 0..31;
     // A = silu(gate) * h from the bf16-rounded h and gate, as stored in H
     constexpr int PB = NI / 2, CPP = 32 / VEC;  // pair blocks, chunks per 32 columns
-    constexpr int ITERS = 16 * MI * PB * CPP / 64;
+    constexpr int PARTS = MI % 2 == 0 ? 2 : 1;  // row parts: 3 outputs per pair need room
+    constexpr int PROWS = 32 * MI / PARTS;      // rows per part
+    constexpr int ITERS = PROWS * PB * CPP / 64;
     constexpr int B = ITERS < EPI_BATCH ? ITERS : EPI_BATCH;
     static_assert(ITERS % B == 0, "batches tile the staged block");
     uint16_t* A2 = reinterpret_cast<uint16_t*>(p.c2);
     const int jj0 = nt * (BN / 2) + (wn0 / 64) * 32;
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {  // two halves of the rows: 3 outputs per pair need room
-      wave_stage_bf16(st, acc, half * MI / 2, (half + 1) * MI / 2, nullptr);
+    for (int half = 0; half < PARTS; ++half) {
+      wave_stage_bf16(st, acc, half * MI / PARTS, (half + 1) * MI / PARTS, nullptr);
 #pragma unroll
       for (int i0 = 0; i0 < ITERS; i0 += B) {
         uint4 hv[B], gv[B];
@@ -1530,14 +1612,14 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
           const int pb = rem / CPP, cc = rem % CPP;
           hv[u] = *reinterpret_cast<const uint4*>(st + rr * S::PITCH + (pb * 64 + cc * VEC) * 2);
           gv[u] = *reinterpret_cast<const uint4*>(st + rr * S::PITCH + (pb * 64 + 32 + cc * VEC) * 2);
-          orow[u] = row_table[wm0 + half * 16 * MI + rr];
+          orow[u] = row_table[wm0 + half * PROWS + rr];
         }
 #pragma unroll
         for (int u = 0; u < B; ++u) {
           const int idx = lane + 64 * (i0 + u);
           const int rr = idx / (PB * CPP), rem = idx % (PB * CPP);
           const int pb = rem / CPP, cc = rem % CPP;
-          const int rl = wm0 + half * 16 * MI + rr;
+          const int rl = wm0 + half * PROWS + rr;
           const int jj = jj0 + pb * 32 + cc * VEC;
           if (rl < rows && jj < p.half) {
             float h[VEC], gt[VEC], a[VEC];
@@ -1838,15 +1920,18 @@ struct WaveGrid {
 // the wave staging areas after the K loop, then the rows kernel's output-row table.
 template <int BM, int BN, int NW = 4>
 constexpr int bf16_stage_bytes() {
-  constexpr int loop = 2 * (BM + BN) * 64 * 2;
+  constexpr int loop = (ring_stages(BM, BN, NW) > 0 ? ring_stages(BM, BN, NW) : 2) * (BM + BN) * 64 * 2;
   constexpr int small = (BM == 256 && NW == 8) ? 3 * (kSmallRows + BN) * 64 * 2 : 0;
   constexpr int epi = NW * WaveGrid<BM, BN, NW>::WM * WaveStage<WaveGrid<BM, BN, NW>::WN>::PITCH;
   constexpr int ops = loop > small ? loop : small;
   return ops > epi ? ops : epi;
 }
 
+// (the 4-wave ring kernels state their two workgroups per CU: left to the compiler, its
+// accumulators moved through AGPRs in the loop)
 template <int BM, int BN, bool B_T, int EPI, int NW = 4>
-__global__ __launch_bounds__(NW * 64) void rows_bf16_kernel(RowsParams p) {
+__global__ __launch_bounds__(NW * 64, (NW == 4 && ring_stages(BM, BN, NW) > 0 ? 2 : 1)) void rows_bf16_kernel(
+    RowsParams p) {
   extern __shared__ __align__(16) char smem[];
   constexpr int KS = 64;
   using WG = WaveGrid<BM, BN, NW>;
@@ -1938,7 +2023,8 @@ __global__ __launch_bounds__(NW * 64) void rows_bf16_kernel(RowsParams p) {
   // 8 waves run the 16 x 16 x 32 K loop (kloop64_m16; the C3 step 2.8% faster than on 32 x 32 x 16
   // MFMAs, the Newton-Schulz pass 2.5%), except with the SwiGLU-backward epilogue, which has no
   // registers left for its extra fragments
-  constexpr bool M16 = EPI != EPI_SWIGLU_BWD && NW == 8;
+  constexpr int RING = ring_stages(BM, BN, NW);
+  constexpr bool M16 = RING > 0 || (EPI != EPI_SWIGLU_BWD && NW == 8);
   using Acc = typename std::conditional<M16, f32x4_t[4], f32x16_t>::type;
   Acc acc[MI][NI];
 #pragma unroll
@@ -1977,7 +2063,9 @@ __global__ __launch_bounds__(NW * 64) void rows_bf16_kernel(RowsParams p) {
       if constexpr (EPI == EPI_SWIGLU_BWD || EPI == EPI_SWIGLU) scale_table[threadIdx.x] = scale_v;
     }
   };
-  if constexpr (M16) {
+  if constexpr (RING > 0) {
+    kloop_ring<RING, NQA, LPS - NQA, MI, NI, B_T, BM, BN>(nk, lds, wm0, wn0, acc, dma_a, dma_b, hook);
+  } else if constexpr (M16) {
     // a tile of at most kSmallRows rows streams its weight block three stages deep
     if (BM == 256 && __builtin_amdgcn_readfirstlane(rows) <= kSmallRows)
       kloop_small<NQA, LPS - NQA, MI, NI, B_T, BN>(nk, lds, wm0, wn0, acc, dma_a, dma_b, hook);
@@ -2449,7 +2537,7 @@ constexpr int kBigWaves = 8;
 
 template <int BM, int BN, bool B_KN, int EPI>
 int launch_rows_bf16(const RowsParams& p, int64_t R, hipStream_t s) {
-  constexpr int NW = BM == 256 ? kBigWaves : 4;
+  constexpr int NW = BN == 256 ? kBigWaves : 4;
   return launch_rows_kernel(rows_bf16_kernel<BM, BN, B_KN, EPI, NW>, bf16_lds_bytes<BM, BN, NW>(), BM, p, R, s,
                             NW * 64);
 }
@@ -2633,6 +2721,35 @@ inline int64_t rows_tiles(int64_t R, int E, int BM) { return cdiv(R, BM) + (R < 
 constexpr int64_t kF32SmallTiles = 448;
 inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
 
+// Tile size of a bf16 rows launch from its rows per expert (R / E on average) and its column
+// tiles of 256 and of 128 (nt256, nt128 per expert). All figures in us.
+//  * Up to 52 rows nearly every expert is one tile of 64, and the launch streams weights: 64 x 128
+//    ring tiles, two workgroups per CU, keep more of them in flight (E = 128, d = 2048, f = 768,
+//    against 128 x 128: at 32 rows W1 174 / 198, W2 86 / 96, dA 78 / 90; at 64 rows, where half the
+//    experts take two tiles, W1 192 / 205, but d = 1024, E = 64, f = 512: 37 / 29). With B read
+//    along N and K > 2048 they lose 1-6% (d = 7168, E = 64, f = 2048: dA 337 / 317 at 24 rows).
+//  * From 112 rows most experts still are one tile of 256 but two of 128: 256 x 256 (d = 7168, 160
+//    rows: W1 897 / 1238, dA 430 / 619; d = 2048, 126 rows: W1 227 / 250, W1 input grad 204 / 229;
+//    but at 96: 222 / 210). Between the two, 128 x 256 ring tiles (d = 7168, 96 rows: W1 682 / 742
+//    on 128 x 128, W1 input grad 686 / 752). Both need enough tiles: d = 1024, E = 64 has 256
+//    (expert, 256-column) pairs for W1, and under a Zipf(1.1) skew at 126 rows 256 x 256 takes 61,
+//    128 x 128 49.
+//  * From 256 rows on, whichever needs less time in whole rounds over the CUs (one 256 x 256 or two
+//    128 x 128 workgroups each, a round of the former 1.45x the latter's): d = 512, E = 32, f = 160,
+//    410 rows: W1 21 / 17 on 128 x 128; d = 2048, E = 32, f = 768: dA 93 / 73 at 600 rows, but
+//    51 / 65 at 410; from a few rounds on 256 x 256, whose loads have twice the reuse.
+enum RowsForm { ROWS_128x128, ROWS_64x128, ROWS_128x256, ROWS_256x256 };
+inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t nt256, int64_t nt128, bool b_kn) {
+  if (R >= (int64_t)E * 256 && N >= 256) {
+    const int64_t r256 = cdiv(rows_tiles(R, E, 256) * nt256, 256), r128 = cdiv(rows_tiles(R, E, 128) * nt128, 512);
+    return 20 * r128 < 29 * r256 ? ROWS_128x128 : ROWS_256x256;
+  }
+  const bool many = N >= 256 && E * nt256 >= 384;
+  if (many && R >= (int64_t)E * 112) return ROWS_256x256;
+  if (R <= (int64_t)E * 52 && !(b_kn && K > 2048)) return ROWS_64x128;
+  return many ? ROWS_128x256 : ROWS_128x128;
+}
+
 template <bool B_KN, int EPI>
 int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipStream_t s) {
   // n_tiles: along N (or along pair columns for SwiGLU, BN/2 pairs per tile)
@@ -2646,12 +2763,16 @@ int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipS
     // contiguous the n-tiles are, so the tiles sharing B columns run together (measured
     // at C3: W2 forward 3%, W1 input grad 2% faster; n-major W1 forward 1% slower)
     p.n_major = p.a_rows == nullptr ? 1 : 0;
-    if (use_big_tiles(R, p.E, p.N)) {
-      p.n_tiles = (int)cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 128 : 256);
-      return launch_rows_bf16<256, 256, B_KN, EPI>(p, R, s);
+    const int64_t nt256 = cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 128 : 256);
+    const int64_t nt128 = cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128);
+    const RowsForm form = rows_form(R, p.E, p.N, p.K, nt256, nt128, B_KN);
+    p.n_tiles = (int)(form == ROWS_256x256 || form == ROWS_128x256 ? nt256 : nt128);
+    switch (form) {
+      case ROWS_256x256: return launch_rows_bf16<256, 256, B_KN, EPI>(p, R, s);
+      case ROWS_128x256: return launch_rows_bf16<128, 256, B_KN, EPI>(p, R, s);
+      case ROWS_64x128: return launch_rows_bf16<64, 128, B_KN, EPI>(p, R, s);
+      default: return launch_rows_bf16<128, 128, B_KN, EPI>(p, R, s);
     }
-    p.n_tiles = (int)cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128);
-    return launch_rows_bf16<128, 128, B_KN, EPI>(p, R, s);
   }
   // SwiGLU pairs 32-column blocks inside a wave, so its tile stays 128 columns (64 pairs) wide
   constexpr int BN = EPI == EPI_SWIGLU ? 128 : 64;
@@ -2979,9 +3100,23 @@ extern "C" int zmoe_glu_w2_backward_dh_gates(const void* dout, int64_t T, int k,
 namespace {
 // bf16 weight grads: 256 x 256 tiles when the experts are large enough, 128 x 128 otherwise,
 // and the small experts split off under a skewed routing. DYG: the gather is on DY's rows.
+// 256 x 256 weight-grad tiles (with the few-rows form for experts of at most 64 rows) rather than
+// 128 x 128. A tile's time is mostly its fixed cost (decode, first loads, output) unless its expert
+// has many rows, so the larger tile wins whenever the launch has several per CU, whatever the rows
+// (us, 256 / 128: E = 128, d = 2048, f = 768, 32 rows an expert: dW1 204 / 270, dW2 107 / 134; d =
+// 7168, E = 64, f = 2048, 126 rows: dW1 1291 / 1686; d = 1024, E = 64, f = 512, 16 rows: dW1, 1024
+// tiles, 31 / 42, but dW2, 512 tiles, 44 / 35 at 126 skewed rows). From 256 rows on it needs more
+// than half a tile per CU, or a popular expert's few tiles run long alone (d = 512, E = 32, f =
+// 160, 410 rows: dW1, 128 tiles, 18 / 17, under a Zipf(1) skew 58 / 43; f = 320, 192 tiles: 20 /
+// 25 and 58 / 52).
+inline bool use_big_wgrad(int64_t M, int E, int64_t N, int64_t K) {
+  const int64_t tiles = (int64_t)E * cdiv(N, 256) * cdiv(K, 256);
+  return N >= 256 && K >= 256 && (tiles >= 1024 || (M >= (int64_t)E * 256 && tiles > 128));
+}
+
 template <bool DYG, bool OUT_F32 = false>
 int group_bwd_w_bf16(WgradParams p, int64_t M, int E, int64_t N, int64_t K, hipStream_t s) {
-  const bool big = use_big_tiles(M, E, N) && K >= 256;
+  const bool big = use_big_wgrad(M, E, N, K);
   const int gather = p.x_rows ? (p.x_div_shift >= 0 ? 1 : 2) : 0;
   if (DYG && gather == 0) return zmoe::set_error(ZMOE_ERR_NULL, "group_bwd_w: the DY gather needs indices");
   auto small_tiles = [&](const WgradParams& q) -> int {

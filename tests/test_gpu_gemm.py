@@ -565,3 +565,95 @@ def test_f32_tile_sizes(hip_device, d, f):
     assert_close_fro(np64(dW2), ref.transpose(0, 2, 1), what="dW2")
     for e in np.nonzero(counts == 0)[0]:
         assert not dW1[e].any() and not dW2[e].any()
+
+
+# (rows per expert, N, f): each tile size of the bf16 rows launches at its own row counts, K of 1, 2
+# and 4 stages (the 3-stage rings' edges)
+_FORM_COUNTS = {
+    "64x128": (np.array([0, 1, 17, 63, 64, 65, 127, 128, 129, 0, 5, 8]), 264, 200),       # <= 52 rows on average
+    "128x256": (np.array([0, 1, 63, 64, 65, 127, 128, 129, 257, 60, 40, 30] * 8), 1000, 504),  # 52-112, >= 384 pairs
+    "256x256 few rows": (np.array([0, 3, 64, 65, 128, 129, 255, 256, 257, 190, 120, 100] * 8), 1000, 504),
+    "256x256": (SMALL_TILE_COUNTS, 1928, 960),  # one round of 256 x 256, two of 128 x 128
+}
+
+
+@pytest.mark.parametrize("K", [64, 120, 200])
+@pytest.mark.parametrize("form", list(_FORM_COUNTS))
+def test_rows_tile_forms(hip_device, form, K):
+    """bf16 rows launches at sizes that the dispatch sends to each tile size: both weight layouts,
+    gathered and grouped A, scattered output, bias, the (scaled) SwiGLU forward and its backward."""
+    from zmoe import ops
+
+    counts, N, f = _FORM_COUNTS[form]
+    k, dt = 2, torch.bfloat16
+    if counts.sum() % k:
+        counts = counts.copy()
+        counts[-1] += 1
+    E, R = len(counts), int(counts.sum())
+    se, ss, off = _fixed_routing(counts, k, hip_device, seed=23)
+    sn, en = ss.cpu().numpy(), se.cpu().numpy()
+    g = gen(R + N + K)
+    x = torch.randn(R // k, K, generator=g).to(dt)
+    Xg = torch.randn(R, K, generator=g).to(dt)
+    W = (torch.randn(E, N, K, generator=g) / K ** 0.5).to(dt)
+    b = (torch.randn(E, N, generator=g) * 0.3).to(dt)
+    Wp, W64 = W.to(hip_device).permute(0, 2, 1), np64(W).transpose(0, 2, 1)
+    tol = TOL[dt]
+    for layout in (Wp, Wp.contiguous()):
+        Y = ops.scatter2scatter(x.to(hip_device), layout, se, ss, k, b=b.to(hip_device), y_grouped=True,
+                                expert_offsets=off)
+        assert_close(np64(Y), O.scatter2scatter(np64(x), W64, en, sn, k, b=np64(b), x_grouped=False, y_grouped=True),
+                     **tol, what="gathered A, bias")
+        Y = ops.scatter2scatter(Xg.to(hip_device), layout, se, ss, 1, x_grouped=True, expert_offsets=off)
+        assert_close(np64(Y), O.scatter2scatter(np64(Xg), W64, en, sn, 1, x_grouped=True, y_grouped=False), **tol,
+                     what="grouped A, scattered")
+    W1 = (torch.randn(E, 2 * f, K, generator=g) / K ** 0.5).to(dt)
+    rs = torch.rand(R, generator=g) + 0.05
+    H, A = ops.glu_w1_forward(x.to(hip_device), W1.to(hip_device), se, ss, off, k, row_scale=rs.to(hip_device))
+    assert_close(np64(H), O.scatter2scatter(np64(x), np64(W1).transpose(0, 2, 1), en, sn, k, x_grouped=False,
+                                            y_grouped=True), **tol, what="H")
+    assert_close(np64(A), np64(rs)[:, None] * O.swiglu(np64(H)), **tol, what="A")
+    # W2's input grad with the SwiGLU backward epilogue: [R, K] x [K, f]
+    W2 = (torch.randn(E, K, f, generator=g) / f ** 0.5).to(dt)
+    dH = ops.glu_w2_backward_dh(Xg.to(hip_device), W2.to(hip_device), H, se, off)
+    dA = O.scatter2scatter(np64(Xg), np64(W2), en, sn, 1, x_grouped=True, y_grouped=True)
+    dA = O.bf16_round(dA.astype(np.float32)).astype(np.float64)  # dA is stored in bf16 before the epilogue
+    assert_close(np64(dH), O.swiglu_backward(dA, np64(H)), **tol, what="dH")
+
+
+@pytest.mark.parametrize("out_f32", [False, True])
+@pytest.mark.parametrize("gather", [None, "x", "dy"])
+@pytest.mark.parametrize("few", [False, True])
+def test_group_bwd_w_large_tiles_by_count(hip_device, few, gather, out_f32):
+    """Weight grads on 256 x 256 tiles because a launch has many of them: more than 128 at 256 rows
+    an expert or more, and at least 1024 below that (few), with the few-rows form and the zero
+    fillers or the separate few-rows launch. The output starts as NaN."""
+    from zmoe import ops
+
+    counts = np.array([0, 0, 1, 64, 65, 700, 0, 2400, 3, 0, 0, 300, 0])
+    if few:
+        counts = np.concatenate([counts, np.array([9, 30, 0, 16, 17] * 11)])
+    E, k, N, K = len(counts), 3, 1000, 776
+    R, dt = int(counts.sum()), torch.bfloat16
+    assert E * 16 >= 1024 if few else R >= 256 * E
+    off = torch.from_numpy(np.cumsum(counts)).to(hip_device)
+    g = gen(R + 9)
+    ss = torch.from_numpy(np.random.default_rng(12).permutation(R)).to(hip_device)
+    od = torch.float32 if out_f32 else None
+    DWt = torch.full((E, N, K), float("nan"), dtype=od or dt, device=hip_device)
+    DY = torch.randn(R // k + 1 if gather == "dy" else R, N, generator=g).to(dt)
+    X = torch.randn(R // k + 1 if gather == "x" else R, K, generator=g).to(dt)
+    DYg = O.group(np64(DY), ss.cpu().numpy(), fan_out=k) if gather == "dy" else np64(DY)
+    Xg = O.group(np64(X), ss.cpu().numpy(), fan_out=k) if gather == "x" else np64(X)
+    if gather == "dy":
+        ops.group_bwd_w_gather_dy(DY.to(hip_device), ss, k, X.to(hip_device), off, E, out=DWt, out_dtype=od)
+    else:
+        ops.group_bwd_w(DY.to(hip_device), X.to(hip_device), off, E, x_gather=ss if gather else None, x_div=k,
+                        out=DWt, out_dtype=od)
+    ref, _ = O.group_bwd_w(DYg, Xg, off.cpu().numpy(), E)
+    if out_f32:
+        assert_close_fro(np64(DWt), ref.transpose(0, 2, 1), what="group_bwd_w f32")
+    else:
+        assert_close(np64(DWt), ref.transpose(0, 2, 1), **TOL[dt], what="group_bwd_w")
+    for e in np.nonzero(counts == 0)[0]:
+        assert (DWt[e] == 0).all(), f"empty expert {e} must get exact zeros"
