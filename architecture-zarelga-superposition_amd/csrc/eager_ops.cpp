@@ -159,7 +159,52 @@ Tensors flatten_sort_count(const Tensor& e, int64_t E) {
   return op.call(e, E);
 }
 
+Tensors flatten_sort_count_weights(const Tensor& e, const Tensor& w, int64_t E) {
+  if (e.is_cuda() && e.scalar_type() == at::kLong && e.is_contiguous() && E >= 0 && fits_int(E) &&
+      flat(w, e, at::kFloat) && w.numel() == e.numel()) {
+    const c10::DeviceGuard guard(e.device());
+    const int64_t R = e.numel();
+    const size_t bytes = zmoe_sort_workspace_bytes(R, (int)E);
+    Tensor se = empty({R}, e), ss = empty({R}, e), off = empty({E}, e), inv = empty({R}, e, at::kInt),
+           sw = empty({R}, e, at::kFloat), ws = workspace(bytes, e);
+    if (zmoe_flatten_sort_count_weights(ids(e), ptr<const float>(w), R, (int)E, ptr<int64_t>(se), ptr<int64_t>(ss),
+                                        ptr<int64_t>(off), ptr<int32_t>(inv), ptr<float>(sw), raw(ws), bytes,
+                                        stream_of(e)) == ZMOE_OK)
+      return {se, ss, off, inv, sw};
+  }
+  static const auto op = general<Tensors(const Tensor&, const Tensor&, c10::SymInt)>("zmoe::flatten_sort_count_weights");
+  return op.call(e, w, E);
+}
+
 // ------------------------------------------------------------------ grouped GEMMs
+Tensors glu_shared_forward(const Tensor& x, const Tensor& W1, const Tensor& W2, const Tensor& ss, const Tensor& off,
+                           int64_t k, const Tensor& scale, const Tensor& Wu, const Tensor& Wg, const Tensor& Wd) {
+  const auto bf = at::kBFloat16;
+  if (x.is_cuda() && x.dim() == 2 && flat(x, x, bf) && flat(W1, x, bf) && flat(W2, x, bf) && flat(Wu, x, bf) &&
+      flat(Wg, x, bf) && flat(Wd, x, bf) && W1.dim() == 3 && W2.dim() == 3 && Wu.dim() == 2 && Wg.dim() == 2 &&
+      Wd.dim() == 2 && k > 0 && fits_int(k) && W1.size(1) % 2 == 0 && fits_int(W1.size(0))) {
+    const int64_t T = x.size(0), d = x.size(1), E = W1.size(0), f = W1.size(1) / 2, fs = Wu.size(0), R = T * k;
+    if (W1.size(2) == d && W2.size(0) == E && W2.size(1) == d && W2.size(2) == f && Wu.size(1) == d &&
+        Wg.size(0) == fs && Wg.size(1) == d && Wd.size(0) == d && Wd.size(1) == fs && index(ss, x, R) &&
+        index(off, x, E) && flat(scale, x, at::kFloat) && scale.numel() == R &&
+        zmoe_glu_stream_shared_ok(T, d, f, fs, (int)E, (int)k)) {
+      const c10::DeviceGuard guard(x.device());
+      Tensor H = empty({R, 2 * f}, x), A = empty({R, f}, x), Y = empty({R, d}, x), Hs = empty({T, 2 * fs}, x),
+             As = empty({T, fs}, x), S = empty({T, d}, x);
+      if (zmoe_glu_w1_forward_shared(raw(x), raw(W1), ids(ss), ids(off), T, d, f, (int)E, (int)k,
+                                     ptr<const float>(scale), raw(H), raw(A), raw(Wu), raw(Wg), fs, raw(Hs), raw(As),
+                                     stream_of(x)) == ZMOE_OK &&
+          zmoe_glu_w2_forward_shared(raw(A), raw(W2), ids(ss), ids(off), T, d, f, (int)E, (int)k, raw(Y), raw(As),
+                                     raw(Wd), fs, raw(S), stream_of(x)) == ZMOE_OK)
+        return {H, A, Y, Hs, As, S};
+    }
+  }
+  static const auto op =
+      general<Tensors(const Tensor&, const Tensor&, const Tensor&, const Tensor&, const Tensor&, c10::SymInt,
+                      const Tensor&, const Tensor&, const Tensor&, const Tensor&)>("zmoe::glu_shared_forward");
+  return op.call(x, W1, W2, ss, off, k, scale, Wu, Wg, Wd);
+}
+
 Tensors glu_w1_forward(const Tensor& x, const Tensor& W1, const Tensor& se, const Tensor& ss, const Tensor& off,
                        int64_t k, const Opt& scale) {
   if (x.is_cuda() && known(x) && rows2(x, x) && flat(W1, x, x.scalar_type()) && W1.dim() == 3 && k > 0 && fits_int(k) &&
@@ -587,6 +632,10 @@ TORCH_LIBRARY(zmoe_eager, m) {
   ZMOE_EAGER(route_topk_backward,
              "(Tensor d_weight, Tensor topk_prob, Tensor topk_idx, int num_experts, Tensor like) -> Tensor");
   ZMOE_EAGER(flatten_sort_count, "(Tensor expert_idxs, int num_experts) -> Tensor[]");
+  ZMOE_EAGER(flatten_sort_count_weights, "(Tensor expert_idxs, Tensor weights, int num_experts) -> Tensor[]");
+  ZMOE_EAGER(glu_shared_forward,
+             "(Tensor x, Tensor W1, Tensor W2, Tensor sorted_scattered_idxs, Tensor expert_offsets, int k, "
+             "Tensor row_scale, Tensor W_up, Tensor W_gate, Tensor W_down) -> Tensor[]");
   ZMOE_EAGER(glu_w1_forward,
              "(Tensor x, Tensor W1, Tensor sorted_expert_idxs, Tensor sorted_scattered_idxs, Tensor expert_offsets, "
              "int k, Tensor? row_scale) -> Tensor[]");

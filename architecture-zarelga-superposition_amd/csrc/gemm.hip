@@ -2589,51 +2589,105 @@ inline int wgrad_small_rows(int64_t R, int E) { return R < (int64_t)E * 1024 ? k
 // ==================================================================== small-M streaming path
 // Forward rows GEMMs when the experts hold few rows (the small-batch regime, e.g. a
 // decode step): the weights are then the only large operand and the GEMM is bound by
-// streaming them from HBM. Each wave owns 32 weight rows (16 SwiGLU pairs: their h and
-// gate rows) and streams them from HBM straight into MFMA operand registers (no LDS, no
-// barriers), kStreamDepth 64-deep stages ahead, multiplying them with up to 32 of the
+// streaming them from HBM. A tile is 32 weight rows (16 SwiGLU pairs: their h and
+// gate rows), streamed from HBM straight into MFMA operand registers (no LDS),
+// kStreamDepth 64-deep stages ahead, and multiplied with up to 32 of the
 // expert's rows per pass, which come from L2. v_mfma_f32_32x32x16_bf16 takes the weight
 // fragment as its first operand, so lane (r, g) ends up with 4 consecutive output
 // columns (weight rows 8 q + 4 g .. + 3) of expert row r.
 // Measured at d = 2048, E = 128, k = 8 (W1 with SwiGLU + W2): 219 vs 237 us for the tiled
 // kernels at T = 32, even at T = 128, slower from T = 256 on; depths 2, 3 and 4 time the same.
+//
+// KSPLIT = 1: a wave owns a tile and walks the whole reduction (no barriers). KSPLIT = 4: the four
+// waves of a block take a quarter of the reduction each and wave 0 adds their sums (in wave order,
+// through LDS) and writes the outputs: with few experts touched there are too few tiles for the
+// loads in flight to cover HBM's latency (T = 4 at the shapes above: ~30 experts, 1440 waves of 128
+// KB each; W1 59.6 -> 38.3 us, W2 24.5 -> 22.2 us, the shared expert below included).
+//
+// StreamShared: a dense expert beside the routed ones, in the same launch (the layer's shared
+// expert, whose rows are all T tokens): its blocks come first, one per tile (or four tiles) and 32
+// tokens. On their own its three products took two library GEMMs, a concatenation of their weights
+// and an elementwise pass (27 us and four launches of a 139 us forward at T = 4).
 constexpr int kStreamDepth = 2;
 constexpr int kStreamRowsPerExpert = 8;  // dispatch bound on R / E
 
-template <int EPI>
-__global__ __launch_bounds__(256) void stream_rows_kernel(RowsParams p, int wtiles_per_e) {
-  const int lane = (int)(threadIdx.x & 63);
-  const int wpe = (wtiles_per_e + 3) / 4;  // workgroups per expert
-  const int e = (int)blockIdx.x / wpe;
-  const int wt = ((int)blockIdx.x % wpe) * 4 + (int)(threadIdx.x >> 6);
-  if (e >= p.E || wt >= wtiles_per_e) return;  // (waves are independent: no barriers)
-  const int64_t e_begin = e ? p.offsets[e - 1] : 0;
-  const int64_t count = p.offsets[e] - e_begin;
-  if (count <= 0) return;
-  const int r = lane & 31, g = lane >> 5;
-  int n;
-  bool nok;
-  if constexpr (EPI == EPI_SWIGLU) {
-    const int jj = wt * 16 + (r & 15);
-    nok = jj < p.half;
-    n = (r & 16) ? p.half + jj : jj;
+struct StreamShared {
+  const void* b0;       // weight rows: up (SwiGLU) or [N][K]
+  const void* b1;       // gate rows (SwiGLU)
+  const void* a;        // rows x K, rows lda apart
+  void *c, *c2;         // outputs as RowsParams'
+  int64_t lda, ldc, ldc2;
+  uint32_t a_bytes;
+  int K, width, rows;   // width: SwiGLU pairs or output columns
+  int blocks_per_group; // blocks of one group of 32 rows
+  int blocks;           // 0: none
+};
+
+template <int EPI, int KSPLIT>
+__global__ __launch_bounds__(256, (KSPLIT > 1 ? 4 : 1)) void stream_rows_kernel(RowsParams p, StreamShared sh, int wtiles_per_e) {
+  __shared__ f32x4_t red[KSPLIT > 1 ? 3 : 1][4][64];
+  const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
+  const int tpb = KSPLIT == 1 ? 4 : 1;  // tiles per block
+  const bool shared = (int)blockIdx.x < sh.blocks;  // uniform
+  int64_t e_begin, count;
+  const char *w0, *w1 = nullptr;
+  int wt, K, width;
+  int64_t ldb, lda, ldc, ldc2;
+  uint16_t *C, *C2;
+  __amdgpu_buffer_rsrc_t ars;
+  if (shared) {
+    const int group = (int)blockIdx.x / sh.blocks_per_group;
+    wt = ((int)blockIdx.x % sh.blocks_per_group) * tpb;
+    e_begin = (int64_t)group * 32;
+    count = sh.rows - e_begin < 32 ? sh.rows - e_begin : 32;
+    w0 = static_cast<const char*>(sh.b0);
+    w1 = static_cast<const char*>(sh.b1);
+    K = sh.K;
+    width = sh.width;
+    ldb = sh.K;
+    lda = sh.lda;
+    ldc = sh.ldc;
+    ldc2 = sh.ldc2;
+    C = static_cast<uint16_t*>(sh.c);
+    C2 = static_cast<uint16_t*>(sh.c2);
+    ars = make_rsrc(sh.a, sh.a_bytes);
   } else {
-    n = wt * 32 + r;
-    nok = n < p.N;
+    const int wpe = (wtiles_per_e + tpb - 1) / tpb;  // blocks per expert
+    const int b = (int)blockIdx.x - sh.blocks;
+    const int e = b / wpe;
+    if (e >= p.E) return;
+    wt = (b % wpe) * tpb;
+    e_begin = e ? p.offsets[e - 1] : 0;
+    count = p.offsets[e] - e_begin;
+    if (count <= 0) return;
+    w0 = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(p.b) + (int64_t)e * p.b_estride);
+    K = p.K;
+    width = EPI == EPI_SWIGLU ? p.half : p.N;
+    ldb = p.ldb;
+    if constexpr (EPI == EPI_SWIGLU) w1 = w0 + (int64_t)p.half * ldb * 2;
+    lda = p.lda;
+    ldc = p.ldc;
+    ldc2 = p.ldc2;
+    C = static_cast<uint16_t*>(p.c);
+    C2 = static_cast<uint16_t*>(p.c2);
+    ars = make_rsrc(p.a, p.a_bytes);
   }
-  const char* b_base = reinterpret_cast<const char*>(reinterpret_cast<const uint16_t*>(p.b) + (int64_t)e * p.b_estride);
-  const __amdgpu_buffer_rsrc_t brs = make_rsrc(b_base, p.b_bytes);
-  const __amdgpu_buffer_rsrc_t ars = make_rsrc(p.a, p.a_bytes);
-  // offsets of this lane's 16 bytes at k = 0 (kOOB: reads zero); + 128 per 64-deep stage, + 32 per step
-  const uint32_t boff = nok ? (uint32_t)((int64_t)n * p.ldb * 2) + 16u * (uint32_t)g : kOOB;
-  const int nkc = p.K / 64;
-  uint16_t* C = reinterpret_cast<uint16_t*>(p.c);
+  if constexpr (KSPLIT == 1) {
+    wt += wave;
+    if (wt * (EPI == EPI_SWIGLU ? 16 : 32) >= width) return;  // (waves are independent: no barriers)
+  }
+  const int r = lane & 31, g = lane >> 5;
+  // this lane's weight row (rows past the width: the last one; their products are not stored)
+  const int n = wt * (EPI == EPI_SWIGLU ? 16 : 32) + (EPI == EPI_SWIGLU ? r & 15 : r);
+  const char* wp = (EPI == EPI_SWIGLU && (r & 16) ? w1 : w0) + (int64_t)(n < width ? n : width - 1) * ldb * 2 + 16 * g;
+  const int nkc = K / 64;
+  const int k0 = KSPLIT == 1 ? 0 : nkc * wave / KSPLIT, k1 = KSPLIT == 1 ? nkc : nkc * (wave + 1) / KSPLIT;
   for (int64_t mb = 0; mb < count; mb += 32) {
-    uint32_t aoff = kOOB;
+    uint32_t aoff = kOOB;  // (rows past the count read zeros)
     if (mb + r < count) {
       int64_t src = e_begin + mb + r;
-      if (p.a_rows != nullptr) src = reinterpret_cast<const int*>(p.a_rows)[2 * src] / p.a_div;
-      aoff = (uint32_t)(src * p.lda * 2) + 16u * (uint32_t)g;
+      if (!shared && p.a_rows != nullptr) src = reinterpret_cast<const int*>(p.a_rows)[2 * src] / p.a_div;
+      aoff = (uint32_t)(src * lda * 2) + 16u * (uint32_t)g;
     }
     f32x16_t acc;
 #pragma unroll
@@ -2643,68 +2697,104 @@ __global__ __launch_bounds__(256) void stream_rows_kernel(RowsParams p, int wtil
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         const uint32_t ko = (uint32_t)kc * 128u + 32u * (uint32_t)s;
-        wf[buf][s] = __builtin_bit_cast(v4i32_t, __builtin_amdgcn_raw_buffer_load_b128(brs, boff + ko, 0, 0));
+        wf[buf][s] = *reinterpret_cast<const v4i32_t*>(wp + ko);
         xf[buf][s] = __builtin_bit_cast(v4i32_t, __builtin_amdgcn_raw_buffer_load_b128(ars, aoff + ko, 0, 0));
       }
     };
 #pragma unroll
     for (int u = 0; u < kStreamDepth; ++u)
-      if (u < nkc) load(u, u);
-    for (int kc = 0; kc < nkc; kc += kStreamDepth) {
+      if (k0 + u < k1) load(u, k0 + u);
+    for (int kc = k0; kc < k1; kc += kStreamDepth) {
 #pragma unroll
       for (int u = 0; u < kStreamDepth; ++u) {
-        if (kc + u < nkc) {
+        if (kc + u < k1) {
 #pragma unroll
           for (int s = 0; s < 4; ++s)
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, wf[u][s]),
                                                           __builtin_bit_cast(bf16x8_t, xf[u][s]), acc, 0, 0, 0);
-          if (kc + u + kStreamDepth < nkc) load(u, kc + u + kStreamDepth);
+          if (kc + u + kStreamDepth < k1) load(u, kc + u + kStreamDepth);
         }
       }
     }
-    if (mb + r >= count) continue;
-    const int64_t i = e_begin + mb + r;  // sorted row
-    const int64_t o = p.c_rows ? reinterpret_cast<const int*>(p.c_rows)[2 * i] : i;
-    if constexpr (EPI == EPI_SWIGLU) {
-      // acc[4 q + u]: h of pair wt 16 + 8 q + 4 g + u for q = 0, 1; its gate at q + 2
-      uint16_t* A2 = reinterpret_cast<uint16_t*>(p.c2);
-      const float rs = p.row_scale != nullptr ? p.row_scale[i] : 1.f;
+    if constexpr (KSPLIT > 1) {
+      if (mb > 0) __syncthreads();  // wave 0 has read the sums of the rows before
+      if (wave > 0) {
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        const int pr = wt * 16 + 8 * q + 4 * g;
-        if (pr >= p.half) continue;
-        float h[4], gt[4], a[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          h[u] = to_f32(bf16_bits(acc[4 * q + u]));
-          gt[u] = to_f32(bf16_bits(acc[4 * (q + 2) + u]));
-          a[u] = rs * (silu_f(gt[u]) * h[u]);
-        }
-        *reinterpret_cast<uint2*>(C + o * p.ldc + pr) = pack4_bf16(h);
-        *reinterpret_cast<uint2*>(C + o * p.ldc + p.half + pr) = pack4_bf16(gt);
-        *reinterpret_cast<uint2*>(A2 + o * p.ldc2 + pr) = pack4_bf16(a);
+        for (int q = 0; q < 4; ++q)
+          red[wave - 1][q][lane] = f32x4_t{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
       }
-    } else {
+      __syncthreads();
+      if (wave > 0) continue;
+#pragma unroll 1
+      for (int w = 0; w < 3; ++w)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int c0 = wt * 32 + 8 * q + 4 * g;
-        if (c0 >= p.N) continue;
-        float v[4];
+        for (int q = 0; q < 4; ++q) {
+          const f32x4_t v = red[w][q][lane];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = acc[4 * q + u];
-        *reinterpret_cast<uint2*>(C + o * p.ldc + c0) = pack4_bf16(v);
+          for (int u = 0; u < 4; ++u) acc[4 * q + u] += v[u];
+        }
+    }
+    if (mb + r < count) {
+      const int64_t i = e_begin + mb + r;  // sorted row
+      const int64_t o = !shared && p.c_rows ? reinterpret_cast<const int*>(p.c_rows)[2 * i] : i;
+      if constexpr (EPI == EPI_SWIGLU) {
+        // acc[4 q + u]: h of pair wt 16 + 8 q + 4 g + u for q = 0, 1; its gate at q + 2
+        const float rs = !shared && p.row_scale != nullptr ? p.row_scale[i] : 1.f;
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const int pr = wt * 16 + 8 * q + 4 * g;
+          if (pr >= width) continue;
+          float h[4], gt[4], a[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            h[u] = to_f32(bf16_bits(acc[4 * q + u]));
+            gt[u] = to_f32(bf16_bits(acc[4 * (q + 2) + u]));
+            a[u] = rs * (silu_f(gt[u]) * h[u]);
+          }
+          *reinterpret_cast<uint2*>(C + o * ldc + pr) = pack4_bf16(h);
+          *reinterpret_cast<uint2*>(C + o * ldc + width + pr) = pack4_bf16(gt);
+          *reinterpret_cast<uint2*>(C2 + o * ldc2 + pr) = pack4_bf16(a);
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int c0 = wt * 32 + 8 * q + 4 * g;
+          if (c0 >= width) continue;
+          float v[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) v[u] = acc[4 * q + u];
+          *reinterpret_cast<uint2*>(C + o * ldc + c0) = pack4_bf16(v);
+        }
       }
     }
   }
 }
 
+// Waves that a launch needs for its loads in flight to cover HBM's latency: 16 per CU.
+constexpr int64_t kStreamWaves = 4096;
+
 template <int EPI>
-int launch_stream_rows(const RowsParams& p, hipStream_t s) {
-  const int wtiles = EPI == EPI_SWIGLU ? (int)cdiv(p.half, 16) : (int)cdiv(p.N, 32);
-  const int64_t blocks = (int64_t)p.E * cdiv(wtiles, 4);
+int launch_stream_rows(const RowsParams& p, int64_t R, hipStream_t s, StreamShared sh = {}) {
+  constexpr int TILE = EPI == EPI_SWIGLU ? 16 : 32;
+  const int wtiles = (int)cdiv(EPI == EPI_SWIGLU ? p.half : p.N, TILE);
+  const bool split = (R < p.E ? R : p.E) * wtiles < kStreamWaves && p.K >= 256;
+  const int tpb = split ? 1 : 4;
+  if (sh.rows > 0) {
+    sh.blocks_per_group = (int)cdiv(cdiv(sh.width, TILE), tpb);
+    sh.blocks = sh.blocks_per_group * (int)cdiv(sh.rows, 32);
+  }
+  const int64_t blocks = (int64_t)p.E * cdiv(wtiles, tpb) + sh.blocks;
   ZMOE_REQUIRE(blocks < (int64_t)0x7fffffff, ZMOE_ERR_SHAPE, "grouped gemm: too many tiles");
-  hipLaunchKernelGGL(stream_rows_kernel<EPI>, dim3((unsigned)blocks), dim3(256), 0, s, p, wtiles);
+  if (split)
+    hipLaunchKernelGGL((stream_rows_kernel<EPI, 4>), dim3((unsigned)blocks), dim3(256), 0, s, p, sh, wtiles);
+  else
+    hipLaunchKernelGGL((stream_rows_kernel<EPI, 1>), dim3((unsigned)blocks), dim3(256), 0, s, p, sh, wtiles);
   return check_launch("grouped rows streaming kernel");
+}
+
+// Few rows per expert: stream the weights (the K loop takes whole 64-deep stages).
+inline bool use_stream(int64_t R, int64_t E, int64_t K) {
+  return R <= kStreamRowsPerExpert * E && K % 64 == 0;
 }
 
 // Tiles of BM rows that R rows in E experts come to, about (half a partial tile per expert).
@@ -2755,8 +2845,7 @@ int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipS
   // n_tiles: along N (or along pair columns for SwiGLU, BN/2 pairs per tile)
   if (dtype == ZMOE_DTYPE_BF16) {
     if constexpr (!B_KN && (EPI == EPI_STORE || EPI == EPI_SWIGLU)) {
-      // few rows per expert: stream the weights (the K loop takes whole 64-deep stages)
-      if (R <= (int64_t)kStreamRowsPerExpert * p.E && p.K % 64 == 0) return launch_stream_rows<EPI>(p, s);
+      if (use_stream(R, p.E, p.K)) return launch_stream_rows<EPI>(p, R, s);
     }
     // tile order within an expert: the tiles that share the gathered operand run
     // together. With A rows gathered (W1 forward, dA) the m-tiles are outer; with A
@@ -2970,6 +3059,99 @@ extern "C" int zmoe_glu_w1_forward_scaled(const void* X, int64_t x_stride_m, con
   ZMOE_REQUIRE(T <= 0 || k <= 0 || row_scale != nullptr, ZMOE_ERR_NULL, "glu_w1_forward_scaled: null row_scale");
   return glu_w1_forward_impl(X, x_stride_m, W1, sorted_scattered_idxs, expert_offsets, T, d, f, E, k, dtype,
                              row_scale, H, A, stream);
+}
+
+extern "C" int zmoe_glu_stream_shared_ok(int64_t T, int64_t d, int64_t f, int64_t fs, int E, int k) {
+  if (T < 1 || d < 64 || f < 64 || fs < 64 || E < 1 || E > kGemmMaxE || k < 1 || T >= kMaxRows / k) return 0;
+  if (d >= (1 << 24) || f >= (1 << 24) || fs >= (1 << 24)) return 0;
+  const int64_t R = T * k;
+  // every operand a whole number of 64-deep stages, its rows within a buffer's range
+  return use_stream(R, E, d) && f % 64 == 0 && fs % 64 == 0 && T * d * 2 <= kMaxSpan && R * f * 2 <= kMaxSpan &&
+         T * fs * 2 <= kMaxSpan && 2 * f * d * 2 <= kMaxSpan;
+}
+
+extern "C" int zmoe_glu_w1_forward_shared(const void* X, const void* W1, const int64_t* sorted_scattered_idxs,
+                                          const int64_t* expert_offsets, int64_t T, int64_t d, int64_t f, int E,
+                                          int k, const float* row_scale, void* H, void* A, const void* W_up,
+                                          const void* W_gate, int64_t fs, void* Hs, void* As, void* stream) {
+  ZMOE_REQUIRE(zmoe_glu_stream_shared_ok(T, d, f, fs, E, k), ZMOE_ERR_SHAPE,
+               "glu_w1_forward_shared: sizes outside the streaming path");
+  ZMOE_REQUIRE(X && W1 && sorted_scattered_idxs && expert_offsets && row_scale && H && A && W_up && W_gate && Hs && As,
+               ZMOE_ERR_NULL, "glu_w1_forward_shared: null pointer");
+  ZMOE_REQUIRE(aligned16(X) && aligned16(W1) && aligned16(H) && aligned16(A) && aligned16(W_up) && aligned16(W_gate) &&
+                   aligned16(Hs) && aligned16(As),
+               ZMOE_ERR_ALIGN, "glu_w1_forward_shared: pointers must be 16-byte aligned");
+  RowsParams p{};
+  p.a = X;
+  p.lda = d;
+  p.a_rows = sorted_scattered_idxs;
+  p.a_div = k;
+  p.b = W1;
+  p.b_estride = 2 * f * d;
+  p.ldb = d;
+  p.c = H;
+  p.ldc = 2 * f;
+  p.c2 = A;
+  p.ldc2 = f;
+  p.offsets = expert_offsets;
+  p.K = (int)d;
+  p.N = (int)(2 * f);
+  p.E = E;
+  p.half = (int)f;
+  p.a_bytes = (uint32_t)(T * d * 2);
+  p.row_scale = row_scale;
+  StreamShared sh{};
+  sh.b0 = W_up;
+  sh.b1 = W_gate;
+  sh.a = X;
+  sh.c = Hs;
+  sh.c2 = As;
+  sh.lda = d;
+  sh.ldc = 2 * fs;
+  sh.ldc2 = fs;
+  sh.a_bytes = p.a_bytes;
+  sh.K = (int)d;
+  sh.width = (int)fs;
+  sh.rows = (int)T;
+  return launch_stream_rows<EPI_SWIGLU>(p, T * k, as_stream(stream), sh);
+}
+
+extern "C" int zmoe_glu_w2_forward_shared(const void* A, const void* W2, const int64_t* sorted_scattered_idxs,
+                                          const int64_t* expert_offsets, int64_t T, int64_t d, int64_t f, int E,
+                                          int k, void* Y, const void* As, const void* W_down, int64_t fs, void* S,
+                                          void* stream) {
+  ZMOE_REQUIRE(zmoe_glu_stream_shared_ok(T, d, f, fs, E, k), ZMOE_ERR_SHAPE,
+               "glu_w2_forward_shared: sizes outside the streaming path");
+  ZMOE_REQUIRE(A && W2 && sorted_scattered_idxs && expert_offsets && Y && As && W_down && S, ZMOE_ERR_NULL,
+               "glu_w2_forward_shared: null pointer");
+  ZMOE_REQUIRE(aligned16(A) && aligned16(W2) && aligned16(Y) && aligned16(As) && aligned16(W_down) && aligned16(S),
+               ZMOE_ERR_ALIGN, "glu_w2_forward_shared: pointers must be 16-byte aligned");
+  RowsParams p{};
+  p.a = A;
+  p.lda = f;
+  p.a_div = 1;
+  p.b = W2;
+  p.b_estride = d * f;
+  p.ldb = f;
+  p.c = Y;
+  p.ldc = d;
+  p.c_rows = sorted_scattered_idxs;
+  p.offsets = expert_offsets;
+  p.K = (int)f;
+  p.N = (int)d;
+  p.E = E;
+  p.a_bytes = (uint32_t)(T * k * f * 2);
+  StreamShared sh{};
+  sh.b0 = W_down;
+  sh.a = As;
+  sh.c = S;
+  sh.lda = fs;
+  sh.ldc = d;
+  sh.a_bytes = (uint32_t)(T * fs * 2);
+  sh.K = (int)fs;
+  sh.width = (int)d;
+  sh.rows = (int)T;
+  return launch_stream_rows<EPI_STORE>(p, T * k, as_stream(stream), sh);
 }
 
 extern "C" int zmoe_glu_w2_backward_dh(const void* dYg, const void* W2, const void* H,

@@ -74,22 +74,30 @@ class _FusedMoELayer(torch.autograd.Function):
         # bf16 compute copies of fp32 operands (one HIP pass each)
         cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731
         x, W1, W2 = cast(x), cast(W1), cast(W2)
-        # [up | gate | router] rows in one operand (cast with the concatenation)
-        W3 = torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf)  # [2fs + E, d]; rows :2fs = [up | gate]
         Ws_down = Ws_down.to(bf)
         fs = Ws_up.shape[0]
-        logits = F.linear(x, W3[2 * fs:])                                            # moe_gate.py:26
-        idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
-        Hs = F.linear(x, W3[:2 * fs])
-        As = _zl.swiglu(Hs)
-        S = F.linear(As, Ws_down)                                                    # expert_layer.py:23-24
-        se, ss, off, inv = _zl.flatten_sort_count(idx, E)                            # mlp.py:76-77
-        w_sorted = w.reshape(-1).index_select(0, ss)
-        H, A_s = _zl.glu_w1_forward(x, W1, se, ss, off, k, w_sorted)                 # A_s = w * A
-        Y_s = _zl.grouped_mm(A_s, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
-                             "scatter2scatter")                                      # = w * Y
+        if _zl.glu_stream_shared_ok(x.shape[0], x.shape[1], W2.shape[2], fs, E, k):
+            # few rows per expert: the launches stream weights, and the shared expert's products
+            # ride in the routed experts' two (W3 below is only formed if there is a backward)
+            w3 = (Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf))
+            logits = F.linear(x, w3[2])                                              # moe_gate.py:26
+            idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
+            se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
+            H, A_s, Y_s, Hs, As, S = _zl.glu_shared_forward(x, W1, W2, ss, off, k, w_sorted, w3[0], w3[1], Ws_down)
+        else:
+            # [up | gate | router] rows in one operand (cast with the concatenation)
+            w3 = (torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf),)  # [2fs + E, d]; rows :2fs = [up | gate]
+            logits = F.linear(x, w3[0][2 * fs:])                                     # moe_gate.py:26
+            idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
+            Hs = F.linear(x, w3[0][:2 * fs])
+            As = _zl.swiglu(Hs)
+            S = F.linear(As, Ws_down)                                                # expert_layer.py:23-24
+            se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
+            H, A_s = _zl.glu_w1_forward(x, W1, se, ss, off, k, w_sorted)             # A_s = w * A
+            Y_s = _zl.grouped_mm(A_s, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
+                                 "scatter2scatter")                                  # = w * Y
         out = _zl.combine(Y_s, None, k, S, pad_rows, pad_total)                      # moe_layer.py:48-56
-        ctx.save_for_backward(x, W1, W2, W3, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows)
+        ctx.save_for_backward(x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3)
         ctx.k, ctx.E, ctx.fs = k, E, fs
         ctx.mark_non_differentiable(idx, off)
         ctx.set_materialize_grads(False)  # no zero-filled grads for idx and off (two fill launches)
@@ -99,7 +107,8 @@ class _FusedMoELayer(torch.autograd.Function):
     def backward(ctx, dout, d_idx, d_off):
         if dout is None:  # out took no part in the loss
             return (None,) * 12
-        x, W1, W2, W3, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows = ctx.saved_tensors
+        x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3 = ctx.saved_tensors
+        W3 = w3[0] if len(w3) == 1 else torch.cat(w3, dim=0)  # [up | gate | router]
         k, E, fs = ctx.k, ctx.E, ctx.fs
         need = ctx.needs_input_grad
         f32 = ctx.f32_grads  # fp32 weight grads from the accumulators (fp32 master weights)

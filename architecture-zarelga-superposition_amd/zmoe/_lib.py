@@ -42,6 +42,7 @@ SIGNATURES = {
     "zmoe_bincount": (I32, [P, I64, I32, P, P]),
     "zmoe_sort_workspace_bytes": (SZ, [I64, I32]),
     "zmoe_flatten_sort_count": (I32, [P, I64, I32, P, P, P, P, P, SZ, P]),
+    "zmoe_flatten_sort_count_weights": (I32, [P, P, I64, I32, P, P, P, P, P, P, SZ, P]),
     "zmoe_sort_error_flag": (P, [P]),
     "zmoe_flatten_sort_count_noalloc": (I32, [P, I64, I32, P, P, P, P, P, P]),
     "zmoe_offsets_from_sorted": (I32, [P, I64, I32, P, P]),
@@ -55,6 +56,9 @@ SIGNATURES = {
     "zmoe_rowwise_sum_product": (I32, [P, I32, P, I32, I64, I32, I64, P, I32, P]),
     "zmoe_glu_w1_forward": (I32, [P, I64, P, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P]),
     "zmoe_glu_w1_forward_scaled": (I32, [P, I64, P, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P, P]),
+    "zmoe_glu_stream_shared_ok": (I32, [I64, I64, I64, I64, I32, I32]),
+    "zmoe_glu_w1_forward_shared": (I32, [P, P, P, P, I64, I64, I64, I32, I32, P, P, P, P, P, I64, P, P, P]),
+    "zmoe_glu_w2_forward_shared": (I32, [P, P, P, P, I64, I64, I64, I32, I32, P, P, P, I64, P, P]),
     "zmoe_glu_w2_backward_dh": (I32, [P, P, P, P, P, I64, I64, I64, I32, I32, P, P]),
     "zmoe_glu_w2_backward_dh_gates_workspace_bytes": (SZ, [I64, I64]),
     "zmoe_glu_w2_backward_dh_gates": (I32, [P, I64, I32, P, P, P, P, P, P, I64, I64, I32, I32, P, P, P, SZ, P]),

@@ -161,7 +161,43 @@ def _(expert_idxs, num_experts):
             _empty((num_experts,), expert_idxs, _I64), _empty((R,), expert_idxs, torch.int32)]
 
 
+@layer_op("flatten_sort_count_weights")
+def flatten_sort_count_weights(expert_idxs: torch.Tensor, weights: torch.Tensor,
+                               num_experts: int) -> List[torch.Tensor]:
+    """flatten_sort_count's four, and the routing weights in sorted order."""
+    return list(_z.flatten_sort_count_weights(expert_idxs, weights, num_experts))
+
+
+@flatten_sort_count_weights.register_fake
+def _(expert_idxs, weights, num_experts):
+    R = expert_idxs.numel()
+    return [_empty((R,), expert_idxs, _I64), _empty((R,), expert_idxs, _I64),
+            _empty((num_experts,), expert_idxs, _I64), _empty((R,), expert_idxs, torch.int32),
+            _empty((R,), expert_idxs, _F32)]
+
+
 # ------------------------------------------------------------------ grouped GEMMs
+glu_stream_shared_ok = _z.glu_stream_shared_ok
+
+
+@layer_op("glu_shared_forward")
+def glu_shared_forward(x: torch.Tensor, W1: torch.Tensor, W2: torch.Tensor, sorted_scattered_idxs: torch.Tensor,
+                       expert_offsets: torch.Tensor, k: int, row_scale: torch.Tensor, W_up: torch.Tensor,
+                       W_gate: torch.Tensor, W_down: torch.Tensor) -> List[torch.Tensor]:
+    """Few rows per expert: the routed and shared experts' forward in two launches:
+    [H, A, Y (slot order), Hs, As, S]."""
+    return list(_z.glu_shared_forward(x, W1, W2, sorted_scattered_idxs, expert_offsets, k, row_scale, W_up, W_gate,
+                                      W_down))
+
+
+@glu_shared_forward.register_fake
+def _(x, W1, W2, sorted_scattered_idxs, expert_offsets, k, row_scale, W_up, W_gate, W_down):
+    T, d = x.shape
+    R, two_f, fs = T * k, W1.shape[1], W_up.shape[0]
+    return [_empty((R, two_f), x), _empty((R, two_f // 2), x), _empty((R, d), x), _empty((T, 2 * fs), x),
+            _empty((T, fs), x), _empty((T, d), x)]
+
+
 @layer_op("glu_w1_forward")
 def glu_w1_forward(x: torch.Tensor, W1: torch.Tensor, sorted_expert_idxs: torch.Tensor,
                    sorted_scattered_idxs: torch.Tensor, expert_offsets: torch.Tensor, k: int,

@@ -193,6 +193,28 @@ def flatten_sort_count(expert_idxs: torch.Tensor, num_experts: int, return_works
     return se, ss, off, inv
 
 
+def flatten_sort_count_weights(expert_idxs: torch.Tensor, weights: torch.Tensor, num_experts: int):
+    """flatten_sort_count with the routing weights (f32, slot order) put in sorted order by the same
+    launches: (sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, inverse, sorted_weights)."""
+    dev = _require_cuda(expert_idxs, weights)
+    flat = _idx64(expert_idxs)
+    R = flat.numel()
+    w = weights.reshape(-1).to(torch.float32).contiguous()
+    if w.numel() != R:
+        raise ValueError("flatten_sort_count_weights: one weight per slot")
+    se = torch.empty(R, dtype=torch.int64, device=dev)
+    ss = torch.empty(R, dtype=torch.int64, device=dev)
+    off = torch.empty(num_experts, dtype=torch.int64, device=dev)
+    inv = torch.empty(R, dtype=torch.int32, device=dev)
+    ws = torch.empty(R, dtype=torch.float32, device=dev)
+    nbytes = L.load().zmoe_sort_workspace_bytes(R, num_experts)
+    work = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+    with profiling.region("flatten_sort_count", dev):
+        L.call("zmoe_flatten_sort_count_weights", _ptr(flat), _ptr(w), R, num_experts, _ptr(se), _ptr(ss), _ptr(off),
+               _ptr(inv), _ptr(ws), _ptr(work), nbytes, _stream(dev))
+    return se, ss, off, inv, ws
+
+
 def sort_out_of_range(workspace: torch.Tensor) -> bool:
     """Host check (synchronises) of the sort's out-of-range flag."""
     return bool(workspace[:4].view(torch.int32)[0].item())
@@ -435,6 +457,44 @@ def glu_w1_forward(x: torch.Tensor, W1: torch.Tensor, sorted_expert_idxs, sorted
                    _ptr(sorted_scattered_idxs), _ptr(expert_offsets), T, d, f, E, k, _dtype_code(x),
                    _ptr(rs.contiguous()), _ptr(H), _ptr(A), _stream(dev))
     return H, A
+
+
+def glu_stream_shared_ok(T: int, d: int, f: int, fs: int, E: int, k: int) -> bool:
+    """Whether ``glu_shared_forward`` takes these sizes (zmoe_glu_stream_shared_ok, in Python so that
+    tracing can follow it): bf16 layers of few rows per expert."""
+    span = 0x7fff0000 // 2
+    return (T >= 1 and T * k <= 8 * E and d % 64 == 0 and f % 64 == 0 and fs % 64 == 0
+            and max(T * d, T * k * f, T * fs, 2 * f * d) <= span and max(d, f, fs) < 1 << 24)
+
+
+def glu_shared_forward(x: torch.Tensor, W1: torch.Tensor, W2: torch.Tensor, sorted_scattered_idxs: torch.Tensor,
+                       expert_offsets: torch.Tensor, k: int, row_scale: torch.Tensor, W_up: torch.Tensor,
+                       W_gate: torch.Tensor, W_down: torch.Tensor):
+    """The routed and the shared experts' forward on the weight-streaming path, two launches (bf16,
+    sizes of ``glu_stream_shared_ok``): (H [R, 2f], A [R, f] scaled by ``row_scale``, Y [R, d] in slot
+    order, Hs [T, 2fs] = [up | gate], As [T, fs], S [T, d])."""
+    dev = _require_cuda(x, W1, W2, sorted_scattered_idxs, expert_offsets, row_scale, W_up, W_gate, W_down)
+    x, W1, W2 = x.contiguous(), W1.contiguous(), W2.contiguous()
+    W_up, W_gate, W_down = W_up.contiguous(), W_gate.contiguous(), W_down.contiguous()
+    if any(t.dtype != torch.bfloat16 for t in (x, W1, W2, W_up, W_gate, W_down)):
+        raise ValueError("glu_shared_forward: bf16 operands only")
+    T, d = x.shape
+    E, two_f, _ = W1.shape
+    f, fs, R = two_f // 2, W_up.shape[0], T * k
+    rs = row_scale.reshape(-1).to(torch.float32).contiguous()
+    ss, off = _idx64(sorted_scattered_idxs), _idx64(expert_offsets)
+    if (W1.shape[2] != d or W2.shape != (E, d, f) or W_up.shape != (fs, d) or W_gate.shape != (fs, d)
+            or W_down.shape != (d, fs) or rs.numel() != R or ss.numel() != R or off.numel() != E):
+        raise ValueError("glu_shared_forward: operand shapes do not match")
+    new = lambda *s: torch.empty(s, dtype=x.dtype, device=dev)  # noqa: E731
+    H, A, Y, Hs, As, S = new(R, two_f), new(R, f), new(R, d), new(T, 2 * fs), new(T, fs), new(T, d)
+    with profiling.region("glu_w1_forward", dev):
+        L.call("zmoe_glu_w1_forward_shared", _ptr(x), _ptr(W1), _ptr(ss), _ptr(off), T, d, f, E, k, _ptr(rs), _ptr(H),
+               _ptr(A), _ptr(W_up), _ptr(W_gate), fs, _ptr(Hs), _ptr(As), _stream(dev))
+    with profiling.region("scatter2scatter", dev):
+        L.call("zmoe_glu_w2_forward_shared", _ptr(A), _ptr(W2), _ptr(ss), _ptr(off), T, d, f, E, k, _ptr(Y), _ptr(As),
+               _ptr(W_down), fs, _ptr(S), _stream(dev))
+    return H, A, Y, Hs, As, S
 
 
 def glu_w2_backward_dh(dYg: torch.Tensor, W2: torch.Tensor, H: torch.Tensor, sorted_expert_idxs, expert_offsets):

@@ -96,6 +96,14 @@ int zmoe_flatten_sort_count(const int64_t* expert_idxs, int64_t R, int E,
                             int64_t* expert_offsets, int32_t* inverse,
                             void* workspace, size_t workspace_bytes, void* stream);
 
+/* The same, and with `weights` (f32 [R] in slot order, or NULL) sorted_weights[i] =
+ * weights[sorted_scattered_idxs[i]], the routing weights in sorted order. */
+int zmoe_flatten_sort_count_weights(const int64_t* expert_idxs, const float* weights, int64_t R,
+                                    int E, int64_t* sorted_expert_idxs,
+                                    int64_t* sorted_scattered_idxs, int64_t* expert_offsets,
+                                    int32_t* inverse, float* sorted_weights, void* workspace,
+                                    size_t workspace_bytes, void* stream);
+
 /* Device address of the out-of-range flag inside a sort workspace. */
 const int32_t* zmoe_sort_error_flag(const void* workspace);
 
@@ -237,6 +245,22 @@ int zmoe_glu_w1_forward_scaled(const void* X, int64_t x_stride_m, const void* W1
                                const int64_t* expert_offsets, int64_t T, int64_t d,
                                int64_t f, int E, int k, int dtype, const float* row_scale,
                                void* H, void* A, void* stream);
+
+/* Small batches (few rows per expert, bf16): the two forward launches of the routed experts with
+ * the shared expert's products (expert_layer.py:23-24) in the same launches. ok returns 1 for the
+ * sizes they take (T * k <= 8 E; d, f and fs multiples of 64), else 0 and they return
+ * ZMOE_ERR_SHAPE. Contiguous operands: X [T, d], W_up and W_gate [fs, d], W_down [d, fs]; H, A, Y as
+ * zmoe_glu_w1_forward_scaled's and zmoe_scatter2scatter's (Y in slot order); Hs [T, 2 fs] = [up |
+ * gate], As [T, fs] = silu(gate) * up, S [T, d] = As W_down^T. */
+int zmoe_glu_stream_shared_ok(int64_t T, int64_t d, int64_t f, int64_t fs, int E, int k);
+int zmoe_glu_w1_forward_shared(const void* X, const void* W1, const int64_t* sorted_scattered_idxs,
+                               const int64_t* expert_offsets, int64_t T, int64_t d, int64_t f, int E,
+                               int k, const float* row_scale, void* H, void* A, const void* W_up,
+                               const void* W_gate, int64_t fs, void* Hs, void* As, void* stream);
+int zmoe_glu_w2_forward_shared(const void* A, const void* W2, const int64_t* sorted_scattered_idxs,
+                               const int64_t* expert_offsets, int64_t T, int64_t d, int64_t f, int E,
+                               int k, void* Y, const void* As, const void* W_down, int64_t fs, void* S,
+                               void* stream);
 
 /* scattermoe/parallel_experts.py:112-120 (W2 input grad, x_grouped and
  * y_grouped) fused with the backward of silu(gates) * h (mlp.py:86):

@@ -31,6 +31,7 @@ def _ops(dev, dtype, d, f):
         "route_topk": (logits, r(E, dt=torch.float32), K2, dtype == torch.bfloat16),
         "route_topk_backward": (w, p, idx, E, x),
         "flatten_sort_count": (idx, E),
+        "flatten_sort_count_weights": (idx, w, E),
         "grouped_mm": (A, W2.permute(0, 2, 1), se, ss, 1, True, False, off, "scatter2scatter"),
         "group_bwd_w": (Y, wide, off, E, ss, K2, False),
         "group_bwd_w_bias": (Y, x, off, E, ss, K2),
@@ -54,6 +55,11 @@ def _ops(dev, dtype, d, f):
         ops["cast_bf16"] = (x,)
     elif d % 8 == 0 and f % 8 == 0:
         ops["glu_w1_forward_scaled"] = (x, W1, se, ss, off, K2, w.reshape(-1)[ss])
+        xs, ws, fs = r(8, 128), [r(E, 128, 128), r(E, 128, 64)], 192   # streaming sizes: 8 tokens, 2 of 8 experts
+        i8 = idx[:8].contiguous()
+        _, s8, o8, _ = torch.ops.zmoe.flatten_sort_count(i8, E)
+        ops["glu_shared_forward"] = (xs, *ws, s8, o8, K2, torch.rand(8 * K2, generator=g).to(dev), r(fs, 128),
+                                     r(fs, 128), r(128, fs))
         ops["group_bwd_w_f32"] = (Y, x, off, E, ss, K2, True)
         ops["group_bwd_w_gather_dy"] = (x, ss, K2, A, off, E, True)
         ops["dense_wgrad_f32"] = (r(5000, d), r(5000, f), True)

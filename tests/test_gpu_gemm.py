@@ -657,3 +657,77 @@ def test_group_bwd_w_large_tiles_by_count(hip_device, few, gather, out_f32):
         assert_close(np64(DWt), ref.transpose(0, 2, 1), **TOL[dt], what="group_bwd_w")
     for e in np.nonzero(counts == 0)[0]:
         assert (DWt[e] == 0).all(), f"empty expert {e} must get exact zeros"
+
+
+# (T, d, f, fs, E, k): the reduction split over a block's waves (few weight tiles) and not, one and
+# several groups of 32 tokens for the shared expert, experts past 32 rows (skewed), partial tiles
+STREAM_SHARED = [(1, 256, 64, 64, 8, 2), (4, 512, 192, 320, 16, 8), (33, 256, 128, 192, 64, 4),
+                 (100, 192, 64, 64, 50, 4), (150, 256, 576, 128, 150, 8), (70, 64, 64, 64, 72, 8)]
+
+
+@pytest.mark.parametrize("skew", [0.0, 2.0])
+@pytest.mark.parametrize("T,d,f,fs,E,k", STREAM_SHARED)
+def test_glu_shared_forward(hip_device, T, d, f, fs, E, k, skew):
+    """The weight-streaming launches with the shared expert in them, against the oracle at the
+    path's rounding points."""
+    from zmoe import ops
+
+    assert ops.glu_stream_shared_ok(T, d, f, fs, E, k)
+    dt = torch.bfloat16
+    idx, se, ss, off, _ = _routing(T, E, k, skew, hip_device, seed=T + f)
+    sn, en = ss.cpu().numpy(), se.cpu().numpy()
+    g = gen(T + d + f)
+    x = torch.randn(T, d, generator=g).to(dt)
+    W1 = (torch.randn(E, 2 * f, d, generator=g) / d ** 0.5).to(dt)
+    W2 = (torch.randn(E, d, f, generator=g) / f ** 0.5).to(dt)
+    Wu, Wg = ((torch.randn(fs, d, generator=g) / d ** 0.5).to(dt) for _ in range(2))
+    Wd = (torch.randn(d, fs, generator=g) / fs ** 0.5).to(dt)
+    rs = torch.rand(T * k, generator=g) + 0.05
+    H, A, Y, Hs, As, S = ops.glu_shared_forward(*(t.to(hip_device) for t in (x, W1, W2)), ss, off, k,
+                                                *(t.to(hip_device) for t in (rs, Wu, Wg, Wd)))
+    tol = TOL[dt]
+    assert_close(np64(H), O.scatter2scatter(np64(x), np64(W1).transpose(0, 2, 1), en, sn, k, x_grouped=False,
+                                            y_grouped=True), **tol, what="H")
+    assert_close(np64(A), np64(rs)[:, None] * O.swiglu(np64(H)), **tol, what="A")
+    assert_close(np64(Y), O.scatter2scatter(np64(A), np64(W2).transpose(0, 2, 1), en, sn, 1, x_grouped=True,
+                                            y_grouped=False), **tol, what="Y")
+    assert_close(np64(Hs), np.concatenate([np64(x) @ np64(Wu).T, np64(x) @ np64(Wg).T], axis=1), **tol, what="Hs")
+    assert_close(np64(As), O.swiglu(np64(Hs)), **tol, what="As")
+    assert_close(np64(S), np64(As) @ np64(Wd).T, **tol, what="S")
+
+
+def test_glu_shared_forward_sizes(hip_device):
+    """The Python rule equals the library's, and other sizes are refused."""
+    import itertools
+
+    from zmoe import _lib as L
+    from zmoe import ops
+
+    lib = L.load()
+    for T, d, f, fs, E, k in itertools.product([0, 1, 64, 65, 1 << 20], [0, 64, 100, 1 << 24], [32, 64, 1 << 20],
+                                               [63, 128], [0, 1, 64, 1024, 2000], [0, 1, 8]):
+        if E >= 1 and k >= 1 and E <= 1024 and min(d, f, fs) >= 64:
+            assert bool(lib.zmoe_glu_stream_shared_ok(T, d, f, fs, E, k)) == ops.glu_stream_shared_ok(T, d, f, fs, E, k)
+    z = lambda *s: torch.zeros(s, dtype=torch.bfloat16, device=hip_device)  # noqa: E731
+    ss = torch.arange(20, device=hip_device)
+    off = torch.tensor([10, 20], device=hip_device)
+    with pytest.raises(ValueError):   # 10 rows per expert
+        ops.glu_shared_forward(z(20, 64), z(2, 128, 64), z(2, 64, 64), ss, off, 1, torch.ones(20, device=hip_device),
+                               z(64, 64), z(64, 64), z(64, 64))
+
+
+@pytest.mark.parametrize("K,N,E,R", [(256, 264, 600, 1200), (64, 40, 30, 200), (320, 72, 40, 320), (256, 8, 4, 30)])
+def test_stream_reduction_split(hip_device, K, N, E, R):
+    """scatter2scatter on the streaming path, the reduction whole (many weight tiles, or K < 256) or
+    split over a block's four waves; experts of none to more than 32 rows."""
+    from zmoe import ops
+
+    counts = np.random.default_rng(R).multinomial(R, np.arange(E, 0, -1) ** 2.0 / (np.arange(E, 0, -1) ** 2.0).sum())
+    se, ss, off = _fixed_routing(counts, 1, hip_device, seed=31)
+    g = gen(K + N)
+    X = torch.randn(R, K, generator=g).to(torch.bfloat16)
+    Wp = (torch.randn(E, N, K, generator=g) / K ** 0.5).to(torch.bfloat16)
+    Y = ops.scatter2scatter(X.to(hip_device), Wp.to(hip_device).permute(0, 2, 1), se, ss, 1, expert_offsets=off)
+    ref = O.scatter2scatter(np64(X), np64(Wp).transpose(0, 2, 1), se.cpu().numpy(), ss.cpu().numpy(), 1,
+                            x_grouped=False, y_grouped=False)
+    assert_close(np64(Y), ref, **TOL[torch.bfloat16], what="stream")

@@ -207,3 +207,21 @@ def test_bias_update_matches_reference_rule(hip_device):
     b = b0.to(hip_device).clone()
     ops.bias_update_(b, off, 1e-3)
     np.testing.assert_array_equal(b.cpu().numpy(), O.bias_update(b0.numpy(), idx.numpy(), E, 1e-3))
+
+
+@pytest.mark.parametrize("R,E", [(1, 1), (32, 128), (1023, 5), (1024, 1024), (1025, 7), (5000, 40), (300000, 300)])
+def test_sort_weights(hip_device, R, E):
+    """The weights in sorted order, and the single-launch sort of one tile (R <= 1024): stable order,
+    offsets and inverse, with out-of-range ids last."""
+    from zmoe import ops
+
+    g = torch.Generator()
+    g.manual_seed(R + E)
+    idx = torch.randint(0, E, (R,), generator=g)
+    idx[torch.rand(R, generator=g) < 0.01] = E + 3
+    w = torch.rand(R, generator=g).to(hip_device)
+    se, ss, off, inv, ws = ops.flatten_sort_count_weights(idx.to(hip_device), w, E)
+    order = torch.sort(torch.where(idx < E, idx, E), stable=True).indices
+    assert torch.equal(ss.cpu(), order) and torch.equal(se.cpu(), idx[order])
+    assert torch.equal(off.cpu(), torch.cumsum(torch.bincount(idx[idx < E], minlength=E), 0))
+    assert torch.equal(ws, w[ss]) and torch.equal(inv.long()[ss].cpu(), torch.arange(R))
