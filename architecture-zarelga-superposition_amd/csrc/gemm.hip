@@ -55,8 +55,8 @@ constexpr int kXcds = 8;
 
 // EPI_STORE_BIAS: EPI_STORE plus a per-expert bias row (a separate instantiation keeps
 // the bias loads out of the common kernel's register budget). EPI_NS: the Newton-Schulz
-// step outputs (bf16 only): t = bf16(acc); C = bf16(t + bf16(ns_beta * D)) when D
-// (p.aux) is given, else t; C2 = bf16(ns_gamma * t) when C2 is given.
+// step outputs (bf16 only): t = bf16(ns_gamma * acc); C = bf16(t + bf16(ns_beta * D)) when D
+// (p.aux) is given, else t.
 enum Epi { EPI_STORE = 0, EPI_SWIGLU = 1, EPI_SWIGLU_BWD = 2, EPI_STORE_BIAS = 3, EPI_NS = 4 };
 
 __device__ __forceinline__ uint32_t lds_off(int row, int chunk) {
@@ -309,8 +309,9 @@ struct RowsParams {
   const void* aux;        // H for the SwiGLU backward; D for EPI_NS
   int64_t ld_aux;
   float ns_beta, ns_gamma; // EPI_NS scalars
-  int ns_sym_m;            // EPI_NS: > 0 when every expert's output is a symmetric m x m matrix:
-                           // only tiles on or above the diagonal run, and they also write their mirror
+  int ns_m;                // EPI_NS: rows of every expert (offsets unused)
+  int ns_sym;              // EPI_NS: the outputs are symmetric m x m matrices: only tiles on or above
+                           // the diagonal run, and they also write their mirror
   const void* bias;       // [E, N] or null
   int64_t bias_estride;
   const int64_t* offsets; // inclusive expert ends [E]
@@ -374,22 +375,27 @@ struct RowsTile {
 // Map this workgroup to (expert, m-tile, n-tile) of a rows launch; false if it has no tile.
 template <int BM, int NT = kGemmThreads>
 __device__ __forceinline__ bool decode_rows_tile(const RowsParams& p, char* smem, RowsTile& t) {
-  if (p.ns_sym_m > 0) {
-    // m x m outputs, one per expert: the upper-triangle tiles (nt >= mt) in row order
-    const int nm = (p.ns_sym_m + BM - 1) / BM;
-    const int tri = nm * (nm + 1) / 2;
-    const int logical = xcd_logical_tile(p.E * tri);
+  if (p.ns_m > 0) {
+    // equal experts: no offsets to read; symmetric ones run the upper-triangle tiles (nt >= mt)
+    const int nm = (p.ns_m + BM - 1) / BM;
+    const int per = p.ns_sym ? nm * (nm + 1) / 2 : nm * p.n_tiles;
+    const int logical = xcd_logical_tile(p.E * per);
     if (logical < 0) return false;
-    t.e = logical / tri;
-    int r = logical % tri, mt = 0;
-    while (r >= nm - mt) {
-      r -= nm - mt;
-      ++mt;
+    t.e = logical / per;
+    int r = logical % per;
+    if (p.ns_sym) {
+      int mt = 0;
+      while (r >= nm - mt) {
+        r -= nm - mt;
+        ++mt;
+      }
+      t.mt = mt;
+      t.nt = mt + r;
+    } else {
+      expert_tile_order(r, p.n_tiles, nm, t.nt, t.mt);
     }
-    t.mt = mt;
-    t.nt = mt + r;
-    t.row0 = (int64_t)t.e * p.ns_sym_m + (int64_t)mt * BM;
-    t.rows = min(BM, p.ns_sym_m - mt * BM);
+    t.row0 = (int64_t)t.e * p.ns_m + (int64_t)t.mt * BM;
+    t.rows = min(BM, p.ns_m - t.mt * BM);
     return true;
   }
   // One pass over the expert ends: each thread counts the m-tiles of its experts, a
@@ -1514,7 +1520,8 @@ __device__ __forceinline__ void unpack4_bf16(uint2 w, float (&v)[4]) {
 // rounded to bf16 (plus the bias row first, if any: one rounding, as an unfused add would not do)
 template <int MI, int NI>
 __device__ __forceinline__ void wave_stage_bf16(char* st, const f32x16_t (&acc)[MI][NI], int mi0, int mi1,
-                                                const uint16_t* bias_cols = nullptr, int bias_ncols = 0) {
+                                                const uint16_t* bias_cols = nullptr, int bias_ncols = 0,
+                                                float scale = 1.f) {
   constexpr int PITCH = WaveStage<NI * 32>::PITCH;
   const int lane = threadIdx.x & 63;
   const int r = lane & 31, g = lane >> 5;
@@ -1528,7 +1535,7 @@ __device__ __forceinline__ void wave_stage_bf16(char* st, const f32x16_t (&acc)[
         const int col = 32 * ni + 8 * q + 4 * g;
         float v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = acc[mi][ni][4 * q + u];
+        for (int u = 0; u < 4; ++u) v[u] = scale * acc[mi][ni][4 * q + u];
         if (bias_cols != nullptr && col < bias_ncols) {  // (columns past N are never stored)
           float bv[4];
           unpack4_bf16(*reinterpret_cast<const uint2*>(bias_cols + col), bv);
@@ -1544,7 +1551,8 @@ __device__ __forceinline__ void wave_stage_bf16(char* st, const f32x16_t (&acc)[
 // holds, in acc[mi][ni][2 a + b], row 32 mi + 16 a + r, columns 32 ni + 16 b + 4 g + 0..3).
 template <int MI, int NI>
 __device__ __forceinline__ void wave_stage_bf16(char* st, const f32x4_t (&acc)[MI][NI][4], int mi0, int mi1,
-                                                const uint16_t* bias_cols = nullptr, int bias_ncols = 0) {
+                                                const uint16_t* bias_cols = nullptr, int bias_ncols = 0,
+                                                float scale = 1.f) {
   constexpr int PITCH = WaveStage<NI * 32>::PITCH;
   const int lane = threadIdx.x & 63;
   const int r = lane & 15, g = lane >> 4;
@@ -1559,7 +1567,7 @@ __device__ __forceinline__ void wave_stage_bf16(char* st, const f32x4_t (&acc)[M
         const int col = 32 * ni + 16 * b + 4 * g;
         float v[4];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = acc[mi][ni][ab][u];
+        for (int u = 0; u < 4; ++u) v[u] = scale * acc[mi][ni][ab][u];
         if (bias_cols != nullptr && col < bias_ncols) {
           float bv[4];
           unpack4_bf16(*reinterpret_cast<const uint2*>(bias_cols + col), bv);
@@ -1645,7 +1653,7 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
   const uint16_t* bias = nullptr;
   if constexpr (EPI == EPI_STORE_BIAS)
     bias = reinterpret_cast<const uint16_t*>(p.bias) + (int64_t)e * p.bias_estride + ncol0;
-  wave_stage_bf16(st, acc, 0, MI, bias, p.N - ncol0);
+  wave_stage_bf16(st, acc, 0, MI, bias, p.N - ncol0, EPI == EPI_NS ? p.ns_gamma : 1.f);
   // chunk (row, column) of item u of batch i
   auto item_rl = [&](int i, int u) { return wm0 + (lane + 64 * (i * B + u)) / S::CPR; };
   auto item_cc = [&](int i, int u) { return (lane + 64 * (i * B + u)) % S::CPR; };
@@ -1656,6 +1664,7 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
   constexpr bool kGlobal = EPI == EPI_SWIGLU_BWD || EPI == EPI_NS;
   const uint16_t* G = reinterpret_cast<const uint16_t*>(p.aux);
   const bool has_g = kGlobal && G != nullptr;
+  const bool mirror = EPI == EPI_NS && p.ns_sym && nt != mt;
   uint4 g0[2][B], g1[2][B];
   auto load_globals = [&](int i, int buf) {
 #pragma unroll
@@ -1697,24 +1706,17 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
       if constexpr (EPI == EPI_STORE || EPI == EPI_STORE_BIAS) {
         st_out(C + o * p.ldc + col, tv[u]);
       } else if constexpr (EPI == EPI_NS) {
-        // out = t + bf16(beta * D) and out2 = bf16(gamma * t) with t = bf16(acc): the rounding
-        // points of bf16 tensor arithmetic in muon.py:24-27 (each product and sum rounded)
-        uint16_t* C2 = reinterpret_cast<uint16_t*>(p.c2);
-        float t[VEC];
-        unpack_chunk(tv[u], t, uint16_t{});
-        if (C2 != nullptr) {
-          float q[VEC];
-#pragma unroll
-          for (int v = 0; v < VEC; ++v) q[v] = p.ns_gamma * t[v];
-          st_out(C2 + o * p.ldc2 + col, pack_chunk(q, uint16_t{}));
-        }
+        // out = bf16(t + bf16(beta * D)) with t = bf16(gamma * acc): every term and the sum rounded
         uint4 ov = tv[u];
         if (has_g) {
-          float d[VEC], r[VEC];
+          float t[VEC], d[VEC], r[VEC];
+          unpack_chunk(tv[u], t, uint16_t{});
           unpack_chunk(g0[cur][u], d, uint16_t{});
 #pragma unroll
           for (int v = 0; v < VEC; ++v) r[v] = t[v] + to_f32(bf16_bits(p.ns_beta * d[v]));
           ov = pack_chunk(r, uint16_t{});
+          // the mirror below is written from the finished values
+          if (mirror) *reinterpret_cast<uint4*>(st + (item_rl(i, u) - wm0) * S::PITCH + item_cc(i, u) * 16) = ov;
         }
         st_out(C + o * p.ldc + col, ov);
       } else {  // EPI_SWIGLU_BWD: staged dA (bf16, as the unfused path stores it), H rows in sorted order
@@ -1752,67 +1754,33 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
   }
   if constexpr (EPI == EPI_NS) {
     // Symmetric output (the Gram products of the Newton-Schulz step): a tile above the
-    // diagonal also writes its mirror. Output row j of the mirror block is column j of
-    // the staged block, read 8 rows at a time with 16-bit LDS reads.
-    if (p.ns_sym_m > 0 && nt != mt) {
-      constexpr int CPC = 32 * MI / VEC;                 // 16-byte chunks per mirrored row
-      constexpr int MITERS = NI * 32 * CPC / 64;
-      constexpr int MB = MITERS < EPI_BATCH ? MITERS : EPI_BATCH;
-      static_assert(MITERS % MB == 0, "batches tile the mirrored block");
-      const uint16_t* D = reinterpret_cast<const uint16_t*>(p.aux);
-      uint16_t* C2 = reinterpret_cast<uint16_t*>(p.c2);
+    // diagonal also writes its mirror, whose row j is column j of the staged block. A lane
+    // reads the same two columns of 8 staged rows as 32-bit words and splits them into one
+    // 16-byte chunk of each mirrored row; 8 lanes side by side write 128 bytes of a row.
+    if (mirror) {
+      static_assert(MI % 2 == 0, "eight chunks of 8 staged rows at a time");
+      constexpr int JB = NI * 2, RB = MI / 2;            // blocks of 16 columns, of 64 rows
       const int64_t ebase = row0 - (int64_t)mt * BM;     // the expert's first row
-      const int jcol0 = nt * BN + wn0;                   // the block's first column = first mirrored row
+      const int rc = lane & 7, cp = lane >> 3;
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the other lanes' finished values
 #pragma unroll
-      for (int i0 = 0; i0 < MITERS; i0 += MB) {
-        uint4 tv[MB], dv[MB];
+      for (int i = 0; i < JB * RB; ++i) {
+        const int r0 = (i % RB) * 64 + rc * VEC;         // first of the lane's 8 staged rows
+        const int c = (i / RB) * 16 + 2 * cp;            // first of its 2 staged columns
+        uint32_t w[8];
 #pragma unroll
-        for (int u = 0; u < MB; ++u) {
-          const int idx = lane + 64 * (i0 + u);
-          const int c = idx / CPC, rc = idx % CPC;       // staged column, chunk of 8 staged rows
-          uint32_t w[4];
+        for (int q = 0; q < 8; ++q) w[q] = *reinterpret_cast<const uint32_t*>(st + (r0 + q) * S::PITCH + c * 2);
+        uint32_t lo[4], hi[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t lo = *reinterpret_cast<const uint16_t*>(st + (rc * VEC + 2 * q) * S::PITCH + c * 2);
-            const uint32_t hi = *reinterpret_cast<const uint16_t*>(st + (rc * VEC + 2 * q + 1) * S::PITCH + c * 2);
-            w[q] = lo | (hi << 16);
-          }
-          tv[u] = make_uint4(w[0], w[1], w[2], w[3]);
+        for (int q = 0; q < 4; ++q) {
+          lo[q] = (w[2 * q] & 0xffffu) | (w[2 * q + 1] << 16);
+          hi[q] = (w[2 * q] >> 16) | (w[2 * q + 1] & 0xffff0000u);
         }
-        if (D != nullptr) {
-#pragma unroll
-          for (int u = 0; u < MB; ++u) {
-            const int idx = lane + 64 * (i0 + u);
-            const int c = idx / CPC, rc = idx % CPC;
-            if (jcol0 + c < p.N && wm0 + rc * VEC < rows)
-              dv[u] = ldg16(D + (ebase + jcol0 + c) * p.ld_aux + mt * BM + wm0 + rc * VEC);
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < MB; ++u) {
-          const int idx = lane + 64 * (i0 + u);
-          const int c = idx / CPC, rc = idx % CPC;
-          if (jcol0 + c >= p.N || wm0 + rc * VEC >= rows) continue;
-          const int64_t o = ebase + jcol0 + c;
-          const int col = mt * BM + wm0 + rc * VEC;
-          float t[VEC];
-          unpack_chunk(tv[u], t, uint16_t{});
-          if (C2 != nullptr) {
-            float q[VEC];
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) q[v] = p.ns_gamma * t[v];
-            st_out(C2 + o * p.ldc2 + col, pack_chunk(q, uint16_t{}));
-          }
-          uint4 ov = tv[u];
-          if (D != nullptr) {
-            float d[VEC], r[VEC];
-            unpack_chunk(dv[u], d, uint16_t{});
-#pragma unroll
-            for (int v = 0; v < VEC; ++v) r[v] = t[v] + to_f32(bf16_bits(p.ns_beta * d[v]));
-            ov = pack_chunk(r, uint16_t{});
-          }
-          st_out(C + o * p.ldc + col, ov);
-        }
+        const int j = nt * BN + wn0 + c;                 // (N and the rows are multiples of 8)
+        if (j >= p.N || wm0 + r0 >= rows) continue;
+        uint16_t* o = C + (ebase + j) * p.ldc + mt * BM + wm0 + r0;
+        st_out(o, make_uint4(lo[0], lo[1], lo[2], lo[3]));
+        st_out(o + p.ldc, make_uint4(hi[0], hi[1], hi[2], hi[3]));
       }
     }
   }
@@ -2828,11 +2796,14 @@ inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
 //    128 x 128 workgroups each, a round of the former 1.45x the latter's): d = 512, E = 32, f = 160,
 //    410 rows: W1 21 / 17 on 128 x 128; d = 2048, E = 32, f = 768: dA 93 / 73 at 600 rows, but
 //    51 / 65 at 410; from a few rounds on 256 x 256, whose loads have twice the reuse.
+inline bool fewer_rounds_128(int64_t tiles256, int64_t tiles128) {
+  return 20 * cdiv(tiles128, 512) < 29 * cdiv(tiles256, 256);
+}
 enum RowsForm { ROWS_128x128, ROWS_64x128, ROWS_128x256, ROWS_256x256 };
 inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t nt256, int64_t nt128, bool b_kn) {
   if (R >= (int64_t)E * 256 && N >= 256) {
-    const int64_t r256 = cdiv(rows_tiles(R, E, 256) * nt256, 256), r128 = cdiv(rows_tiles(R, E, 128) * nt128, 512);
-    return 20 * r128 < 29 * r256 ? ROWS_128x128 : ROWS_256x256;
+    return fewer_rounds_128(rows_tiles(R, E, 256) * nt256, rows_tiles(R, E, 128) * nt128) ? ROWS_128x128
+                                                                                          : ROWS_256x256;
   }
   const bool many = N >= 256 && E * nt256 >= 384;
   if (many && R >= (int64_t)E * 112) return ROWS_256x256;
@@ -2875,9 +2846,9 @@ int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipS
 
 int ns_gemm(const NsGemm& g, hipStream_t s) {
   ZMOE_REQUIRE(g.E >= 1 && g.E <= kGemmMaxE && g.K >= 8 && g.N >= 8 && g.K % 8 == 0 && g.N % 8 == 0 &&
-                   g.R >= 0 && g.R < 0x7fffffffLL,
+                   g.m >= 1 && (!g.sym || g.N == g.m) && (int64_t)g.E * g.m < 0x7fffffffLL,
                ZMOE_ERR_SHAPE, "ns_gemm: bad sizes");
-  if (g.R == 0) return ZMOE_OK;
+  const int64_t R = (int64_t)g.E * g.m;
   RowsParams p{};
   p.a = g.A;
   p.lda = g.lda;
@@ -2886,30 +2857,36 @@ int ns_gemm(const NsGemm& g, hipStream_t s) {
   p.ldb = g.ldb;
   p.c = g.C;
   p.ldc = g.ldc;
-  p.c2 = g.C2;
-  p.ldc2 = g.ldc2;
   p.aux = g.D;
   p.ld_aux = g.ldd;
   p.ns_beta = g.beta;
   p.ns_gamma = g.gamma;
-  p.ns_sym_m = g.sym_m;
-  p.offsets = g.offsets;
+  p.ns_m = g.m;
+  p.ns_sym = g.sym;
   p.K = g.K;
   p.N = g.N;
   p.E = g.E;
-  const int64_t a_span = ((g.R - 1) * g.lda + g.K) * 2;
+  const int64_t a_span = ((R - 1) * g.lda + g.K) * 2;
   const int64_t b_span = g.b_kn ? ((int64_t)(g.K - 1) * g.ldb + g.N) * 2 : ((int64_t)(g.N - 1) * g.ldb + g.K) * 2;
   ZMOE_REQUIRE(a_span <= 0x7fff0000LL && b_span <= 0x7fff0000LL, ZMOE_ERR_SHAPE, "ns_gemm: operand spans 2 GiB");
   p.a_bytes = (uint32_t)a_span;
   p.b_bytes = (uint32_t)b_span;
-  if (use_big_tiles(g.R, g.E, g.N)) {
+  auto tiles = [&](int64_t b) {
+    const int64_t nm = cdiv(g.m, b);
+    return g.E * (g.sym ? nm * (nm + 1) / 2 : nm * cdiv(g.N, b));
+  };
+  // The rule of rows_form, over this launch's own tiles. Five steps, us, on 256 x 256 tiles / by the
+  // rule: 4 x 1024 x 1024 460 / 300, 8 x 1024 x 1536 550 / 436, 16 x 512 x 768 363 / 247,
+  // 24 x 648 x 1000 573 / 509; on 128 x 128 / by the rule: 64 x 1024 x 1024 2364 / 1988,
+  // 64 x 512 x 1024 708 / 635.
+  if (g.m >= 256 && g.N >= 256 && !fewer_rounds_128(tiles(256), tiles(128))) {
     p.n_tiles = (int)cdiv(g.N, 256);
-    return g.b_kn ? launch_rows_bf16<256, 256, true, EPI_NS>(p, g.R, s)
-                  : launch_rows_bf16<256, 256, false, EPI_NS>(p, g.R, s);
+    return g.b_kn ? launch_rows_bf16<256, 256, true, EPI_NS>(p, R, s)
+                  : launch_rows_bf16<256, 256, false, EPI_NS>(p, R, s);
   }
   p.n_tiles = (int)cdiv(g.N, 128);
-  return g.b_kn ? launch_rows_bf16<128, 128, true, EPI_NS>(p, g.R, s)
-                : launch_rows_bf16<128, 128, false, EPI_NS>(p, g.R, s);
+  return g.b_kn ? launch_rows_bf16<128, 128, true, EPI_NS>(p, R, s)
+                : launch_rows_bf16<128, 128, false, EPI_NS>(p, R, s);
 }
 
 }  // namespace zmoe

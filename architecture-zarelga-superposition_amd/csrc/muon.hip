@@ -3,16 +3,22 @@
 // called at :449 as zeropower_via_newtonschulz5(update, steps)).
 //
 // X [E, m, n] bf16 with m <= n (the caller transposes a tall stack, as muon.py:18-19
-// does with .mT). Per matrix, in bf16 tensor arithmetic (every product and sum
-// rounded to bf16, every GEMM accumulated in fp32 and rounded once):
+// does with .mT). Per matrix, in bf16 tensor arithmetic (every term and sum
+// rounded to bf16, every GEMM accumulated in fp32 and rounded once, after its scalar):
 //   X = X / (||X||_F + 1e-7)
-//   repeat steps:  A = X X^T;  B = b A + (c A) A;  X = a X + B X
+//   repeat steps:  A = X X^T;  B = b A + c (A A);  X = a X + B X
 // The three GEMMs of a step are the grouped rows kernel with one "expert" per
-// matrix: A = X X^T reads its right operand as nn.Linear-style rows of X; (cA) A
-// and B X read A and X as [K][N]. Their epilogues form cA (a second output of the
-// first GEMM) and the b A and a X sums, so each step is three launches and no
+// matrix: A = X X^T reads its right operand as nn.Linear-style rows of X; A A
+// and B X read A and X as [K][N]. Their epilogues scale the sums (c (A A), not (c A) A:
+// one rounding fewer) and add b A and a X, so each step is three launches and no
 // elementwise passes. A and B are symmetric, so their GEMMs run only the tiles on
 // or above the diagonal and write each off-diagonal tile's mirror as well.
+//
+// A step at 64 x 1024 x 1024 was 161 + 159 + 141 us, 3 + 3 + 4 rounds of 256 x 256 tiles:
+// the symmetric products took 53 us per round against 35 for B X, on a second output of
+// every tile (cA, 134 MB) and on a mirror read as 16-bit words in 8-way bank conflicts.
+// Without the former and with 32-bit reads: 101 + 118 + 137 us. A round of B X is 22 us of
+// MFMAs and, not overlapped with them, 256 KB of D and output per CU (12 us).
 //
 // The Frobenius norm is a deterministic two-pass reduction: fp32 partial sums
 // of squares per (matrix, slice), then every slice block sums its matrix's
@@ -23,11 +29,6 @@ namespace zmoe {
 
 constexpr int kNsThreads = 256;
 constexpr int kNsMaxSlices = 64;
-
-__global__ void ns_offsets_kernel(int64_t* off, int E, int64_t m) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < E) off[e] = (int64_t)(e + 1) * m;
-}
 
 // partial[e * P + s] = sum of x^2 over slice s of matrix e (chunks of 8 bf16)
 __global__ __launch_bounds__(kNsThreads) void ns_sumsq_kernel(const uint16_t* __restrict__ X, int64_t per_chunks,
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(kNsThreads) void ns_scale_kernel(const uint16_t* __
 }
 
 struct NsLayout {
-  size_t off_offsets, off_partial, off_a, off_p, off_b, off_x, total;
+  size_t off_partial, off_a, off_b, off_x, total;
   int P;
   int64_t slice_chunks;
 };
@@ -101,13 +102,9 @@ NsLayout ns_layout(int64_t E, int64_t m, int64_t n) {
   L.P = P;
   L.slice_chunks = cdiv(per_chunks, P);
   size_t o = 0;
-  L.off_offsets = o;
-  o += align256((size_t)E * 8);
   L.off_partial = o;
   o += align256((size_t)E * P * 4);
   L.off_a = o;
-  o += align256((size_t)(E * m * m) * 2);
-  L.off_p = o;
   o += align256((size_t)(E * m * m) * 2);
   L.off_b = o;
   o += align256((size_t)(E * m * m) * 2);
@@ -144,16 +141,11 @@ namespace {
 int ns_pass(uint16_t* Xuser, int64_t Ec, int64_t m, int64_t n, int steps, float a, float b, float c, char* ws,
             hipStream_t s) {
   const NsLayout L = ns_layout(Ec, m, n);
-  int64_t* offsets = reinterpret_cast<int64_t*>(ws + L.off_offsets);
   float* partial = reinterpret_cast<float*>(ws + L.off_partial);
   uint16_t* Abuf = reinterpret_cast<uint16_t*>(ws + L.off_a);
-  uint16_t* Pbuf = reinterpret_cast<uint16_t*>(ws + L.off_p);
   uint16_t* Bbuf = reinterpret_cast<uint16_t*>(ws + L.off_b);
   uint16_t* Xtmp = reinterpret_cast<uint16_t*>(ws + L.off_x);
 
-  hipLaunchKernelGGL(ns_offsets_kernel, dim3((unsigned)cdiv(Ec, 256)), dim3(256), 0, s, offsets, (int)Ec, m);
-  int rc = check_launch("newton_schulz5 offsets");
-  if (rc) return rc;
   // the normalised X goes where the step count makes the last step land in X
   uint16_t* cur = (steps % 2 == 1) ? Xtmp : Xuser;
   uint16_t* nxt = (steps % 2 == 1) ? Xuser : Xtmp;
@@ -161,43 +153,42 @@ int ns_pass(uint16_t* Xuser, int64_t Ec, int64_t m, int64_t n, int steps, float 
   const dim3 grid((unsigned)L.P, (unsigned)Ec);
   hipLaunchKernelGGL(ns_sumsq_kernel, grid, dim3(kNsThreads), 0, s, Xuser, per_chunks, L.slice_chunks, L.P,
                      partial);
-  rc = check_launch("newton_schulz5 norm");
+  int rc = check_launch("newton_schulz5 norm");
   if (rc) return rc;
   hipLaunchKernelGGL(ns_scale_kernel, grid, dim3(kNsThreads), 0, s, Xuser, cur, per_chunks, L.slice_chunks, L.P,
                      partial);
   rc = check_launch("newton_schulz5 scale");
   if (rc) return rc;
 
-  const int64_t R = Ec * m;
   for (int it = 0; it < steps; ++it) {
-    // A = X X^T, and cA as a second output
+    // A = X X^T
     NsGemm g1{};
     g1.A = cur; g1.lda = n;
     g1.B = cur; g1.b_estride = m * n; g1.ldb = n; g1.b_kn = false;
-    g1.offsets = offsets; g1.R = R; g1.K = (int)n; g1.N = (int)m; g1.E = (int)Ec;
+    g1.m = (int)m; g1.K = (int)n; g1.N = (int)m; g1.E = (int)Ec;
     g1.C = Abuf; g1.ldc = m;
-    g1.C2 = Pbuf; g1.ldc2 = m; g1.gamma = c;
-    g1.sym_m = (int)m;  // X X^T is symmetric: upper-triangle tiles plus their mirror
+    g1.gamma = 1.f;
+    g1.sym = true;  // X X^T is symmetric: upper-triangle tiles plus their mirror
     rc = ns_gemm(g1, s);
     if (rc) return rc;
-    // B = (cA) A + bA, A read as [K][N] (its columns), so the product does not rely on
+    // B = c (A A) + bA, A read as [K][N] (its columns), so the product does not rely on
     // the rounded A being exactly symmetric
     NsGemm g2{};
-    g2.A = Pbuf; g2.lda = m;
+    g2.A = Abuf; g2.lda = m;
     g2.B = Abuf; g2.b_estride = m * m; g2.ldb = m; g2.b_kn = true;
-    g2.offsets = offsets; g2.R = R; g2.K = (int)m; g2.N = (int)m; g2.E = (int)Ec;
+    g2.m = (int)m; g2.K = (int)m; g2.N = (int)m; g2.E = (int)Ec;
     g2.C = Bbuf; g2.ldc = m;
-    g2.D = Abuf; g2.ldd = m; g2.beta = b;
-    g2.sym_m = (int)m;  // (cA) A + bA is symmetric (polynomial in the symmetric A)
+    g2.D = Abuf; g2.ldd = m; g2.beta = b; g2.gamma = c;
+    g2.sym = true;  // c (A A) + bA is symmetric (polynomial in the symmetric A)
     rc = ns_gemm(g2, s);
     if (rc) return rc;
     // X' = B X + aX
     NsGemm g3{};
     g3.A = Bbuf; g3.lda = m;
     g3.B = cur; g3.b_estride = m * n; g3.ldb = n; g3.b_kn = true;
-    g3.offsets = offsets; g3.R = R; g3.K = (int)m; g3.N = (int)n; g3.E = (int)Ec;
+    g3.m = (int)m; g3.K = (int)m; g3.N = (int)n; g3.E = (int)Ec;
     g3.C = nxt; g3.ldc = n;
-    g3.D = cur; g3.ldd = n; g3.beta = a;
+    g3.D = cur; g3.ldd = n; g3.beta = a; g3.gamma = 1.f;
     rc = ns_gemm(g3, s);
     if (rc) return rc;
     uint16_t* t = cur;

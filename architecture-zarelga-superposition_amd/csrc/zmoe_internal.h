@@ -98,29 +98,25 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 
 // ---------------------------------------------------------------- grouped GEMM, Newton-Schulz epilogue
-// C rows [R, N] (bf16; expert e owns rows offsets[e-1] .. offsets[e] - 1) = A rows [R, K] @ B_e,
+// C rows [E * m, N] (bf16; matrix e owns rows e * m .. e * m + m - 1) = A rows [E * m, K] @ B_e,
 // where B_e sits at B + e * b_estride elements as [N][K] (K contiguous; b_kn false) or
-// [K][N] (N contiguous; b_kn true). Epilogue (t = bf16(acc)): C = bf16(t + bf16(beta * D))
-// when D is given, else t; C2 = bf16(gamma * t) when C2 is given. D and C2 share C's rows.
+// [K][N] (N contiguous; b_kn true). Epilogue (t = bf16(gamma * acc)): C = bf16(t + bf16(beta * D))
+// when D is given, else t. D shares C's rows.
 struct NsGemm {
   const void* A;
   int64_t lda;
   const void* B;
   int64_t b_estride, ldb;
   bool b_kn;
-  const int64_t* offsets;
-  int64_t R;
-  int K, N, E;
+  int m, K, N, E;
   void* C;
   int64_t ldc;
   const void* D;
   int64_t ldd;
   float beta;
-  void* C2;
-  int64_t ldc2;
   float gamma;
-  int sym_m;  // > 0: each expert's output is a symmetric sym_m x sym_m matrix (N == sym_m, uniform
-              // rows): only the tiles on or above the diagonal run and they write their mirror
+  bool sym;  // each matrix's output is symmetric (N == m): only the tiles on or above the
+             // diagonal run and they write their mirror
 };
 int ns_gemm(const NsGemm& g, hipStream_t s);
 

@@ -397,8 +397,9 @@ int zmoe_rmsnorm_rows_backward(const void* dY, const void* X, int64_t x_stride, 
  * the orthogonalisation inside the MuonMD step on 3-D expert weights
  * (muon.py:399-508, called at :449). X [E, m, n] bf16, contiguous, m <= n (the
  * caller transposes a tall stack first, as muon.py:18-19 does), updated in place:
- *   X = X / (||X||_F + 1e-7);  repeat steps: A = X X^T; B = b A + (c A) A; X = a X + B X
- * with bf16 rounding after every product and sum, as in bf16 tensor arithmetic.
+ *   X = X / (||X||_F + 1e-7);  repeat steps: A = X X^T; B = b A + c (A A); X = a X + B X
+ * with every GEMM accumulated in fp32 and rounded to bf16 once, after its scalar, and
+ * every other product and sum rounded to bf16.
  * Any E: the stack runs in passes of at most min(1024, (2 GiB - 64 KiB) / (2 m n))
  * matrices over one pass-sized workspace (one matrix must span less than that).
  * Workspace: zmoe_newton_schulz5_workspace_bytes(E, m, n), 256-byte aligned (0 when

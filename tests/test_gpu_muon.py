@@ -63,6 +63,22 @@ def test_steps_match_oracle(hip_device, shape, steps):
         assert err <= REL_FRO[steps], (shape, steps, e, err)
 
 
+# Enough matrices that 256 x 256 tiles take fewer rounds than 128 x 128 ones: for the symmetric
+# products (first shape: 3 x 3 tiles, the last ones 8 rows; B X on 128 x 128), for B X (second:
+# symmetric products on 128 x 128), for both (third)
+@pytest.mark.parametrize("shape", [(40, 520, 520), (30, 520, 776), (64, 512, 512)])
+@pytest.mark.parametrize("steps", [1, 2])
+def test_large_tiles_match_oracle(hip_device, shape, steps):
+    from zmoe import ops
+
+    G = make_stack(shape, 31 + steps, hip_device)
+    got = ops.newton_schulz5(G, steps)
+    for e in (0, shape[0] // 2, shape[0] - 1):
+        ref = O.newton_schulz5(G[e].cpu().numpy()[None], steps)[0]
+        err = rel_fro(got[e].float().cpu().numpy(), ref)
+        assert err <= REL_FRO[steps], (shape, steps, e, err)
+
+
 def test_input_untouched_and_dropin_name(hip_device):
     from zmoe.muon import zeropower_via_newtonschulz5
 
