@@ -228,6 +228,24 @@ Tensors glu_w1_forward(const Tensor& x, const Tensor& W1, const Tensor& se, cons
   return op.call(x, W1, se, ss, off, k, scale);
 }
 
+Tensor glu_act_forward(const Tensor& x, const Tensor& W1, const Tensor& ss, const Tensor& off, int64_t k,
+                       const Opt& scale) {
+  if (x.is_cuda() && known(x) && rows2(x, x) && flat(W1, x, x.scalar_type()) && W1.dim() == 3 && k > 0 && fits_int(k) &&
+      W1.size(2) == x.size(1) && W1.size(1) % 2 == 0 && fits_int(W1.size(0))) {
+    const int64_t T = x.size(0), E = W1.size(0), f = W1.size(1) / 2, R = T * k;
+    if (index(ss, x, R) && index(off, x, E) && (!scale || (flat(*scale, x, at::kFloat) && scale->numel() == R))) {
+      const c10::DeviceGuard guard(x.device());
+      Tensor A = empty({R, f}, x);
+      if (zmoe_glu_act_forward(raw(x), x.stride(0), raw(W1), ids(ss), ids(off), T, x.size(1), f, (int)E, (int)k,
+                               code(x), scale ? ptr<const float>(*scale) : nullptr, raw(A), stream_of(x)) == ZMOE_OK)
+        return A;
+    }
+  }
+  static const auto op = general<Tensor(const Tensor&, const Tensor&, const Tensor&, const Tensor&, c10::SymInt,
+                                        const Opt&)>("zmoe::glu_act_forward");
+  return op.call(x, W1, ss, off, k, scale);
+}
+
 // out [R, N] = the grouped product; false where the general form has to run.
 bool grouped_into(const Tensor& X, const Tensor& W, const Opt& b, const Tensor& se, const Tensor& ss, int64_t k,
                   bool xg, bool yg, const Tensor& off, const Tensor& out) {
@@ -639,6 +657,9 @@ TORCH_LIBRARY(zmoe_eager, m) {
   ZMOE_EAGER(glu_w1_forward,
              "(Tensor x, Tensor W1, Tensor sorted_expert_idxs, Tensor sorted_scattered_idxs, Tensor expert_offsets, "
              "int k, Tensor? row_scale) -> Tensor[]");
+  ZMOE_EAGER(glu_act_forward,
+             "(Tensor x, Tensor W1, Tensor sorted_scattered_idxs, Tensor expert_offsets, int k, Tensor? row_scale) "
+             "-> Tensor");
   ZMOE_EAGER(grouped_mm,
              "(Tensor X, Tensor W, Tensor sorted_expert_idxs, Tensor sorted_scattered_idxs, int k, bool x_grouped, "
              "bool y_grouped, Tensor expert_offsets, str region) -> Tensor");

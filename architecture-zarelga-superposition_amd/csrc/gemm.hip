@@ -559,8 +559,10 @@ __device__ __forceinline__ void rows_epilogue(const RowsParams& p, char* smem, c
         unpack_chunk(gv, g, T{});
 #pragma unroll
         for (int q = 0; q < VEC; ++q) a[q] = silu_f(g[q]) * h[q];
-        *reinterpret_cast<uint4*>(C + orow * p.ldc + jj) = hv;
-        *reinterpret_cast<uint4*>(C + orow * p.ldc + p.half + jj) = gv;
+        if (C != nullptr) {
+          *reinterpret_cast<uint4*>(C + orow * p.ldc + jj) = hv;
+          *reinterpret_cast<uint4*>(C + orow * p.ldc + p.half + jj) = gv;
+        }
         *reinterpret_cast<uint4*>(A2 + orow * p.ldc2 + jj) = pack_chunk(a, T{});
       }
     }
@@ -1637,8 +1639,10 @@ __device__ __forceinline__ void rows_epilogue_bf16(const RowsParams& p, char* st
 #pragma unroll
             for (int q = 0; q < VEC; ++q) a[q] = rs * (silu_f(gt[q]) * h[q]);
             const int64_t o = orow[u];
-            st_out(C + o * p.ldc + jj, hv[u]);
-            st_out(C + o * p.ldc + p.half + jj, gv[u]);
+            if (C != nullptr) {
+              st_out(C + o * p.ldc + jj, hv[u]);
+              st_out(C + o * p.ldc + p.half + jj, gv[u]);
+            }
             st_out(A2 + o * p.ldc2 + jj, pack_chunk(a, uint16_t{}));
           }
         }
@@ -2719,8 +2723,10 @@ __global__ __launch_bounds__(256, (KSPLIT > 1 ? 4 : 1)) void stream_rows_kernel(
             gt[u] = to_f32(bf16_bits(acc[4 * (q + 2) + u]));
             a[u] = rs * (silu_f(gt[u]) * h[u]);
           }
-          *reinterpret_cast<uint2*>(C + o * ldc + pr) = pack4_bf16(h);
-          *reinterpret_cast<uint2*>(C + o * ldc + width + pr) = pack4_bf16(gt);
+          if (C != nullptr) {
+            *reinterpret_cast<uint2*>(C + o * ldc + pr) = pack4_bf16(h);
+            *reinterpret_cast<uint2*>(C + o * ldc + width + pr) = pack4_bf16(gt);
+          }
           *reinterpret_cast<uint2*>(C2 + o * ldc2 + pr) = pack4_bf16(a);
         }
       } else {
@@ -2976,7 +2982,7 @@ extern "C" int zmoe_scatter2scatter(const void* X, int64_t x_stride_m, const voi
 namespace {
 int glu_w1_forward_impl(const void* X, int64_t x_stride_m, const void* W1, const int64_t* sorted_scattered_idxs,
                         const int64_t* expert_offsets, int64_t T, int64_t d, int64_t f, int E, int k, int dtype,
-                        const float* row_scale, void* H, void* A, void* stream) {
+                        const float* row_scale, bool keep_h, void* H, void* A, void* stream) {
   ZMOE_REQUIRE(dtype_ok(dtype), ZMOE_ERR_DTYPE, "glu_w1_forward: dtype %d", dtype);
   ZMOE_REQUIRE(T >= 0 && d >= 1 && f >= 1 && E >= 1 && E <= kGemmMaxE && k >= 1, ZMOE_ERR_SHAPE,
                "glu_w1_forward: bad sizes");
@@ -2984,7 +2990,7 @@ int glu_w1_forward_impl(const void* X, int64_t x_stride_m, const void* W1, const
   ZMOE_REQUIRE(T < kMaxRows && T * k < kMaxRows, ZMOE_ERR_SHAPE, "glu_w1_forward: T*k must be below 2^31");
   const int64_t R = T * k;
   if (R == 0) return ZMOE_OK;
-  ZMOE_REQUIRE(X && W1 && H && A && sorted_scattered_idxs && expert_offsets, ZMOE_ERR_NULL,
+  ZMOE_REQUIRE(X && W1 && (H || !keep_h) && A && sorted_scattered_idxs && expert_offsets, ZMOE_ERR_NULL,
                "glu_w1_forward: null pointer");
   const int v = vec_elems(dtype);
   ZMOE_REQUIRE(d % v == 0 && f % v == 0 && ok_rows(dtype, X, x_stride_m) && aligned16(W1) && aligned16(H) &&
@@ -3023,7 +3029,7 @@ extern "C" int zmoe_glu_w1_forward(const void* X, int64_t x_stride_m, const void
                                    int dtype, void* H, void* A, void* stream) {
   (void)sorted_expert_idxs;
   return glu_w1_forward_impl(X, x_stride_m, W1, sorted_scattered_idxs, expert_offsets, T, d, f, E, k, dtype, nullptr,
-                             H, A, stream);
+                             true, H, A, stream);
 }
 
 extern "C" int zmoe_glu_w1_forward_scaled(const void* X, int64_t x_stride_m, const void* W1,
@@ -3035,7 +3041,22 @@ extern "C" int zmoe_glu_w1_forward_scaled(const void* X, int64_t x_stride_m, con
   ZMOE_REQUIRE(dtype == ZMOE_DTYPE_BF16, ZMOE_ERR_DTYPE, "glu_w1_forward_scaled: bf16 only (dtype %d)", dtype);
   ZMOE_REQUIRE(T <= 0 || k <= 0 || row_scale != nullptr, ZMOE_ERR_NULL, "glu_w1_forward_scaled: null row_scale");
   return glu_w1_forward_impl(X, x_stride_m, W1, sorted_scattered_idxs, expert_offsets, T, d, f, E, k, dtype,
-                             row_scale, H, A, stream);
+                             row_scale, true, H, A, stream);
+}
+
+// Without H: the launch is tile for tile the same, but its epilogue writes a third of the bytes. The
+// epilogue of a 256 x 256 tile is not overlapped with MFMAs (one workgroup per CU), and a CU's share
+// of the memory rate is about 20 GB/s, so at d = 1024, E = 64, k = 8, f = 512, T = 16384 (a tile:
+// 22 us of MFMAs at most, 128 KB of H, 64 KB of A) the whole forward is 538 -> 504 us; T = 509 at
+// d = 2048, E = 128, f = 768 270 -> 264, T = 2011 470 -> 456.
+extern "C" int zmoe_glu_act_forward(const void* X, int64_t x_stride_m, const void* W1,
+                                    const int64_t* sorted_scattered_idxs, const int64_t* expert_offsets, int64_t T,
+                                    int64_t d, int64_t f, int E, int k, int dtype, const float* row_scale, void* A,
+                                    void* stream) {
+  ZMOE_REQUIRE(dtype == ZMOE_DTYPE_BF16 || row_scale == nullptr, ZMOE_ERR_DTYPE,
+               "glu_act_forward: row_scale with bf16 only (dtype %d)", dtype);
+  return glu_w1_forward_impl(X, x_stride_m, W1, sorted_scattered_idxs, expert_offsets, T, d, f, E, k, dtype,
+                             row_scale, false, nullptr, A, stream);
 }
 
 extern "C" int zmoe_glu_stream_shared_ok(int64_t T, int64_t d, int64_t f, int64_t fs, int E, int k) {

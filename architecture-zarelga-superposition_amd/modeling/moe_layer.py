@@ -13,7 +13,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from scattermoe.mlp import GLUMLP
+from scattermoe.mlp import GLUMLP, _records_graph
 from zmoe import functional as _zf
 from zmoe import library as _zl
 
@@ -52,8 +52,8 @@ class _FusedMoELayer(torch.autograd.Function):
     adds over [T, d]).
 
     (x [T, d], gate weight, expert_biases, W1, W2, shared gate/up/down weights, k, E,
-    pad_rows, pad_total) -> (out, topk_idx [T, k], expert_offsets [E]); out is [T, d], or
-    with pad_rows (int64 [T]) the padded [pad_total, d] whose row pad_rows[t] is token t's.
+    pad_rows, pad_total, backward) -> (out, topk_idx [T, k], expert_offsets [E]); with backward
+    False (a call that records no graph) no pre-activations are kept; out is [T, d], or with pad_rows (int64 [T]) the padded [pad_total, d] whose row pad_rows[t] is token t's.
     Every launch is a ``zmoe::`` custom op, so torch.compile traces through the function
     without a graph break.
 
@@ -67,7 +67,7 @@ class _FusedMoELayer(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, gate_w, expert_biases, W1, W2, Ws_gate, Ws_up, Ws_down, k: int, E: int, pad_rows=None,
-                pad_total: int = 0):
+                pad_total: int = 0, backward: bool = True):
         bf = torch.bfloat16
         ctx.f32_grads = W1.dtype == torch.float32
         ctx.x_dtype = x.dtype
@@ -93,7 +93,10 @@ class _FusedMoELayer(torch.autograd.Function):
             As = _zl.swiglu(Hs)
             S = F.linear(As, Ws_down)                                                # expert_layer.py:23-24
             se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
-            H, A_s = _zl.glu_w1_forward(x, W1, se, ss, off, k, w_sorted)             # A_s = w * A
+            if backward:
+                H, A_s = _zl.glu_w1_forward(x, W1, se, ss, off, k, w_sorted)         # A_s = w * A
+            else:
+                H, A_s = None, _zl.glu_act_forward(x, W1, ss, off, k, w_sorted)
             Y_s = _zl.grouped_mm(A_s, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
                                  "scatter2scatter")                                  # = w * Y
         out = _zl.combine(Y_s, None, k, S, pad_rows, pad_total)                      # moe_layer.py:48-56
@@ -106,7 +109,7 @@ class _FusedMoELayer(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout, d_idx, d_off):
         if dout is None:  # out took no part in the loss
-            return (None,) * 12
+            return (None,) * 13
         x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3 = ctx.saved_tensors
         W3 = w3[0] if len(w3) == 1 else torch.cat(w3, dim=0)  # [up | gate | router]
         k, E, fs = ctx.k, ctx.E, ctx.fs
@@ -135,7 +138,7 @@ class _FusedMoELayer(torch.autograd.Function):
         dx = _zl.sum_k(dXe, k, dx_dense, ctx.x_dtype == torch.float32)  # fp32 input: the fp32 sum
         part = (lambda a, b: None) if dW3 is None else (lambda a, b: dW3[a:b])
         return (dx, part(2 * fs, 2 * fs + E), None, dW1, dW2, part(fs, 2 * fs), part(0, fs), dWs_down,
-                None, None, None, None)
+                None, None, None, None, None)
 
 
 class MoELayer(nn.Module):
@@ -216,8 +219,8 @@ class MoELayer(nn.Module):
                 x = normed.reshape(-1, h)
             else:
                 x = flat if unpad_indices is None else index_first_axis(flat, unpad_indices)
-            out, topk_idx, offsets = _FusedMoELayer.apply(x, ws[0], self.gate.expert_biases, *ws[1:],
-                                                          self.gate.top_k, self.routed_experts.num_experts, *pad)
+            ins = (x, ws[0], self.gate.expert_biases, *ws[1:], self.gate.top_k, self.routed_experts.num_experts, *pad)
+            out, topk_idx, offsets = _FusedMoELayer.apply(*ins, _records_graph(ins))
             self.routed_experts.last_expert_offsets = offsets
             if unpad_indices is None:
                 return out.view(bsz, seq_len, h), topk_idx.view(bsz, seq_len, -1)

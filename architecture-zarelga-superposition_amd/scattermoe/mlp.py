@@ -36,22 +36,31 @@ def _fused_widths_ok(d: int, f: int, dtype: torch.dtype) -> bool:
     return d % v == 0 and f % v == 0
 
 
+def _records_graph(args) -> bool:
+    """Whether an autograd function applied to ``args`` here is differentiated through."""
+    return torch.is_grad_enabled() and any(isinstance(a, torch.Tensor) and a.requires_grad for a in args)
+
+
 class GLUExpertsFunction(torch.autograd.Function):
     """y = sum_j gates[:, j] * W2[e_j] silu(W1g[e_j] x) * (W1h[e_j] x) for every token.
 
     (x, gates, expert_idxs, W1, W2, k, num_experts, residual=None, pad_rows=None,
-    pad_total=0) -> (y, expert_offsets). ``residual`` [T, d] is added in the combine pass
-    (moe_layer.py:53 adds the shared expert's output); with ``pad_rows`` the output is the
-    padded [pad_total, d] (moe_layer.py:55-56). ``expert_offsets`` is the sort's (not
+    pad_total=0, backward=True) -> (y, expert_offsets). ``residual`` [T, d] is added in the
+    combine pass (moe_layer.py:53 adds the shared expert's output); with ``pad_rows`` the
+    output is the padded [pad_total, d] (moe_layer.py:55-56). ``backward=False`` (a call that
+    records no graph) keeps no pre-activations. ``expert_offsets`` is the sort's (not
     differentiable). Every launch is a ``zmoe::`` custom op, so torch.compile traces
     through this function without a graph break.
     """
 
     @staticmethod
     def forward(ctx, x, gates, expert_idxs, W1, W2, k: int, num_experts: int, residual=None, pad_rows=None,
-                pad_total: int = 0):
+                pad_total: int = 0, backward: bool = True):
         se, ss, off, inv = _zl.flatten_sort_count(expert_idxs, num_experts)
-        H, A = _zl.glu_w1_forward(x, W1, se, ss, off, k, None)                   # mlp.py:80-86
+        if backward:
+            H, A = _zl.glu_w1_forward(x, W1, se, ss, off, k, None)               # mlp.py:80-86
+        else:
+            H, A = None, _zl.glu_act_forward(x, W1, ss, off, k, None)
         Y = _zl.grouped_mm(A, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
                            "scatter2scatter")                                    # mlp.py:87-93
         out = _zl.combine(Y, gates, k, residual, pad_rows, pad_total)            # parallel_experts.py:50-52
@@ -66,7 +75,7 @@ class GLUExpertsFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dout, d_off):
         if dout is None:  # out took no part in the loss
-            return (None,) * 10
+            return (None,) * 11
         x, gates, W1, W2, se, ss, off, inv, H, A, Y, pad_rows = ctx.saved_tensors
         k, E = ctx.k, ctx.num_experts
         dout = dout.to(x.dtype)
@@ -79,7 +88,7 @@ class GLUExpertsFunction(torch.autograd.Function):
         d_res = None
         if ctx.has_residual and ctx.needs_input_grad[7]:
             d_res = dout if pad_rows is None else dout.index_select(0, pad_rows)
-        return dx, d_gates.to(gates.dtype), None, dW1, dW2, None, None, d_res, None, None
+        return dx, d_gates.to(gates.dtype), None, dW1, dW2, None, None, d_res, None, None, None
 
 
 class MLP(nn.Module):
@@ -143,9 +152,9 @@ class GLUMLP(nn.Module):
             dtype = _compute_dtype(x)
             res = None if residual is None else residual.reshape(-1, residual.shape[-1]).to(dtype)
             rows, total = (None, 0) if pad is None else (pad[0], int(pad[1]))
-            y, self.last_expert_offsets = GLUExpertsFunction.apply(
-                x.to(dtype), expert_p, expert_idxs, self.experts.compute_weight(dtype),
-                self.output_experts.compute_weight(dtype), self.top_k, self.num_experts, res, rows, total)
+            ins = (x.to(dtype), expert_p, expert_idxs, self.experts.compute_weight(dtype),
+                   self.output_experts.compute_weight(dtype), self.top_k, self.num_experts, res, rows, total)
+            y, self.last_expert_offsets = GLUExpertsFunction.apply(*ins, _records_graph(ins))
             return y if pad is not None else y.view(*x_shape[:-1], y.size(-1))
         sorted_expert_idxs, sorted_scattered_idxs, expert_offsets = flatten_sort_count(
             expert_idxs, num_experts=self.num_experts)

@@ -55,6 +55,7 @@ SIGNATURES = {
     "zmoe_dense_wgrad": (I32, [P, I64, P, I64, I64, I64, I64, I32, I32, I32, P, P, SZ, P]),
     "zmoe_rowwise_sum_product": (I32, [P, I32, P, I32, I64, I32, I64, P, I32, P]),
     "zmoe_glu_w1_forward": (I32, [P, I64, P, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P]),
+    "zmoe_glu_act_forward": (I32, [P, I64, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P]),
     "zmoe_glu_w1_forward_scaled": (I32, [P, I64, P, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P, P]),
     "zmoe_glu_stream_shared_ok": (I32, [I64, I64, I64, I64, I32, I32]),
     "zmoe_glu_w1_forward_shared": (I32, [P, P, P, P, I64, I64, I64, I32, I32, P, P, P, P, P, I64, P, P, P]),

@@ -215,6 +215,18 @@ def _(x, W1, sorted_expert_idxs, sorted_scattered_idxs, expert_offsets, k, row_s
     return [_empty((R, two_f), x), _empty((R, two_f // 2), x)]
 
 
+@layer_op("glu_act_forward")
+def glu_act_forward(x: torch.Tensor, W1: torch.Tensor, sorted_scattered_idxs: torch.Tensor,
+                    expert_offsets: torch.Tensor, k: int, row_scale: Optional[torch.Tensor]) -> torch.Tensor:
+    """``glu_w1_forward``'s A alone, for a forward whose backward will not run."""
+    return _z.glu_act_forward(x, W1, sorted_scattered_idxs, expert_offsets, k, row_scale)
+
+
+@glu_act_forward.register_fake
+def _(x, W1, sorted_scattered_idxs, expert_offsets, k, row_scale):
+    return _empty((x.shape[0] * k, W1.shape[1] // 2), x)
+
+
 @layer_op("grouped_mm")
 def grouped_mm(X: torch.Tensor, W: torch.Tensor, sorted_expert_idxs: torch.Tensor,
                sorted_scattered_idxs: torch.Tensor, k: int, x_grouped: bool, y_grouped: bool,

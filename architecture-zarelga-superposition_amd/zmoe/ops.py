@@ -459,6 +459,25 @@ def glu_w1_forward(x: torch.Tensor, W1: torch.Tensor, sorted_expert_idxs, sorted
     return H, A
 
 
+def glu_act_forward(x: torch.Tensor, W1: torch.Tensor, sorted_scattered_idxs, expert_offsets, k: int,
+                    row_scale: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``glu_w1_forward``'s A [R, f] alone: H, which only a backward reads, is not written."""
+    dev = _require_cuda(x, W1, row_scale)
+    x = _rows(x)
+    W1 = W1.contiguous()
+    E, two_f, d = W1.shape
+    T, f = x.shape[0], two_f // 2
+    A = torch.empty((T * k, f), dtype=x.dtype, device=dev)
+    if row_scale is not None:
+        row_scale = row_scale.reshape(-1).contiguous()
+        if row_scale.dtype != torch.float32 or row_scale.numel() != T * k:
+            raise ValueError("glu_w1_forward: row_scale must be float32 with T*k entries")
+    with profiling.region("glu_w1_forward", dev):
+        L.call("zmoe_glu_act_forward", _ptr(x), x.stride(0), _ptr(W1), _ptr(sorted_scattered_idxs),
+               _ptr(expert_offsets), T, d, f, E, k, _dtype_code(x), _ptr(row_scale), _ptr(A), _stream(dev))
+    return A
+
+
 def glu_stream_shared_ok(T: int, d: int, f: int, fs: int, E: int, k: int) -> bool:
     """Whether ``glu_shared_forward`` takes these sizes (zmoe_glu_stream_shared_ok, in Python so that
     tracing can follow it): bf16 layers of few rows per expert."""

@@ -246,6 +246,13 @@ int zmoe_glu_w1_forward_scaled(const void* X, int64_t x_stride_m, const void* W1
                                int64_t f, int E, int k, int dtype, const float* row_scale,
                                void* H, void* A, void* stream);
 
+/* The activations of the two above without H, for a forward whose backward will not run:
+ * row_scale null, or (bf16 only) [R] f32. */
+int zmoe_glu_act_forward(const void* X, int64_t x_stride_m, const void* W1,
+                         const int64_t* sorted_scattered_idxs, const int64_t* expert_offsets,
+                         int64_t T, int64_t d, int64_t f, int E, int k, int dtype,
+                         const float* row_scale, void* A, void* stream);
+
 /* Small batches (few rows per expert, bf16): the two forward launches of the routed experts with
  * the shared expert's products (expert_layer.py:23-24) in the same launches. ok returns 1 for the
  * sizes they take (T * k <= 8 E; d, f and fs multiples of 64), else 0 and they return

@@ -402,6 +402,61 @@ def test_glu_w1_forward_scaled(hip_device, T, d, f, E, k, skew):
     assert_close(np64(A), ref.astype(np.float64), **TOL[torch.bfloat16], what="scaled A")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("T,d,f,E,k", [(32, 256, 256, 32, 8),       # weight streaming
+                                       (1000, 64, 136, 64, 2),      # 64 x 128 tiles; f32: few tiles
+                                       (600, 72, 136, 8, 2),        # 128 x 128
+                                       (1290, 64, 512, 128, 8),     # 128 x 256
+                                       (2100, 64, 512, 128, 8)])    # 256 x 256; f32: many tiles
+def test_glu_act_forward(hip_device, dtype, T, d, f, E, k):
+    """The activations without H: bit for bit glu_w1_forward's, on every tile form, from the
+    wrapper and from both registrations of the op."""
+    from zmoe import library, ops
+
+    idx, se, ss, off, _ = _routing(T, E, k, 0.2, hip_device, seed=T + f)
+    g = gen(T + d + f)
+    x = torch.randn(T, d, generator=g).to(dtype).to(hip_device)
+    W1 = (torch.randn(E, 2 * f, d, generator=g) / d ** 0.5).to(dtype).to(hip_device)
+    rs = (torch.rand(T * k, generator=g) + 0.05).to(hip_device)
+    for scale in (None, rs) if dtype == torch.bfloat16 else (None,):
+        _, A = ops.glu_w1_forward(x, W1, se, ss, off, k, row_scale=scale)
+        assert torch.equal(ops.glu_act_forward(x, W1, ss, off, k, scale), A)
+        with torch.no_grad():
+            assert torch.equal(torch.ops.zmoe.glu_act_forward(x, W1, ss, off, k, scale), A)
+            assert torch.equal(library.glu_act_forward(x, W1, ss, off, k, scale), A)   # the native one
+    if dtype == torch.float32:
+        with pytest.raises(ValueError):
+            ops.glu_act_forward(x, W1, ss, off, k, rs)
+
+
+@pytest.mark.parametrize("T", [700, 40])
+def test_layer_without_graph_matches(hip_device, T):
+    """The layer and the GLU experts under no_grad (no pre-activations kept) give bit for bit
+    what they give when they record a graph, and a graph is recorded when one input needs it."""
+    from modeling.model_config import ModelConfig
+    from modeling.moe_layer import MoELayer
+
+    torch.manual_seed(T)
+    cfg = ModelConfig(hidden_size=128, intermediate_size=64, n_experts=17, n_shared_experts=1, n_experts_per_token=4)
+    layer = MoELayer(cfg).to(hip_device).to(torch.bfloat16)
+    x = torch.randn(1, T, 128, generator=gen(T)).to(torch.bfloat16).to(hip_device)
+    out, idx = layer(x)
+    with torch.no_grad():
+        out0, idx0 = layer(x)
+    assert out.requires_grad and not out0.requires_grad
+    assert torch.equal(out, out0) and torch.equal(idx, idx0)
+    glu = layer.routed_experts
+    p = torch.rand(T, 4, generator=gen(T + 1)).to(hip_device)
+    y = glu(x[0], p, idx.view(T, 4))
+    with torch.no_grad():
+        assert torch.equal(glu(x[0], p, idx.view(T, 4)), y)
+    layer.requires_grad_(False)
+    assert torch.equal(layer(x)[0], out)                       # grad mode on, nothing to differentiate
+    xg = x.clone().requires_grad_(True)
+    layer(xg)[0].sum().backward()
+    assert torch.isfinite(xg.grad).all() and xg.grad.abs().sum() > 0
+
+
 @pytest.mark.parametrize("gather,k", [(False, 2), (True, 2), (True, 3), (True, 6)])
 def test_group_bwd_w_small_expert_split(hip_device, gather, k):
     """bf16 weight grads with 256 x 256 tiles and fewer than 1024 rows per expert on average:
