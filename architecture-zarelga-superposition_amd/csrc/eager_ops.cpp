@@ -505,6 +505,43 @@ Tensor cast_bf16(const Tensor& src) {
   return op.call(src);
 }
 
+Tensors cast_bf16_packed(at::TensorList srcs, int64_t cat_from) {
+  const int64_t n = (int64_t)srcs.size();
+  if (cat_from >= 0 && cat_from < n && n <= ZMOE_CAST_MAX_SEGMENTS && srcs[0].is_cuda()) {
+    const Tensor& x = srcs[0];
+    bool ok = true;
+    int64_t rows = 0;
+    for (int64_t i = 0; i < n; ++i) {
+      ok = ok && flat(srcs[i], x, at::kFloat) && srcs[i].dim() >= 1;
+      if (ok && i >= cat_from) {
+        ok = srcs[i].sizes().slice(1) == srcs[cat_from].sizes().slice(1);
+        rows += srcs[i].size(0);
+      }
+    }
+    if (ok) {
+      const c10::DeviceGuard guard(x.device());
+      Tensors out;
+      const float* src[ZMOE_CAST_MAX_SEGMENTS];
+      int64_t count[ZMOE_CAST_MAX_SEGMENTS];
+      void* dst[ZMOE_CAST_MAX_SEGMENTS];
+      for (int64_t i = 0; i < cat_from; ++i) out.push_back(empty(srcs[i].sizes(), x, at::kBFloat16));
+      auto shape = srcs[cat_from].sizes().vec();
+      shape[0] = rows;
+      out.push_back(empty(shape, x, at::kBFloat16));
+      int64_t at = 0;
+      for (int64_t i = 0; i < n; ++i) {
+        src[i] = ptr<const float>(srcs[i]);
+        count[i] = srcs[i].numel();
+        dst[i] = i < cat_from ? raw(out[i]) : static_cast<char*>(raw(out[cat_from])) + 2 * at;
+        if (i >= cat_from) at += count[i];
+      }
+      if (zmoe_cast_f32_bf16_segments(src, count, dst, (int)n, stream_of(x)) == ZMOE_OK) return out;
+    }
+  }
+  static const auto op = general<Tensors(at::TensorList, c10::SymInt)>("zmoe::cast_bf16_packed");
+  return op.call(srcs, cat_from);
+}
+
 Tensor swiglu(const Tensor& H) {
   if (H.is_cuda() && known(H) && H.dim() == 2 && H.is_contiguous()) {
     const c10::DeviceGuard guard(H.device());
@@ -680,6 +717,7 @@ TORCH_LIBRARY(zmoe_eager, m) {
              "(Tensor Y, Tensor grad_out, Tensor gates, Tensor inverse, Tensor? grad_rows) -> Tensor[]");
   ZMOE_EAGER(sum_k, "(Tensor Xe, int k, Tensor? add0, bool out_f32=False) -> Tensor");
   ZMOE_EAGER(cast_bf16, "(Tensor src) -> Tensor");
+  ZMOE_EAGER(cast_bf16_packed, "(Tensor[] srcs, int cat_from) -> Tensor[]");
   ZMOE_EAGER(swiglu, "(Tensor H) -> Tensor");
   ZMOE_EAGER(swiglu_backward, "(Tensor dA, Tensor H) -> Tensor");
   ZMOE_EAGER(swiglu_backward_gates, "(Tensor dA, Tensor H, Tensor row_scale, Tensor slot_of_row) -> Tensor[]");

@@ -279,6 +279,35 @@ __global__ __launch_bounds__(256) void cast_f32_bf16_kernel(const float* __restr
   if (blockIdx.x == 0 && threadIdx.x < n - 8 * nv) dst[8 * nv + threadIdx.x] = bf16_bits(src[8 * nv + threadIdx.x]);
 }
 
+// Several casts in one launch: block b belongs to the segment i with first[i] <= b < first[i + 1],
+// where it does what block b - first[i] of a launch of that segment alone does. The copies of a
+// small layer's fp32 weights are bound by launches: d = 512, E = 32, f = 160, 6.5k tokens, seven
+// tensors with three of them concatenated 15 us, as six launches (three of these casts, two of
+// torch's and a concatenation) 31 us, and the layer's step, bound by the host's calls, 682 -> 665.
+struct CastSegments {
+  const float* src[ZMOE_CAST_MAX_SEGMENTS];
+  uint16_t* dst[ZMOE_CAST_MAX_SEGMENTS];
+  int64_t n[ZMOE_CAST_MAX_SEGMENTS];
+  uint32_t first[ZMOE_CAST_MAX_SEGMENTS + 1];
+};
+
+__global__ __launch_bounds__(256) void cast_segments_kernel(const CastSegments g, int segments) {
+  int s = 0;
+  for (int i = 1; i < segments; ++i) s = blockIdx.x >= g.first[i] ? i : s;
+  const float* src = g.src[s];
+  uint16_t* dst = g.dst[s];
+  const int64_t n = g.n[s], nv = n / 8;
+  const uint32_t b = blockIdx.x - g.first[s];
+  const int64_t i = (int64_t)b * 256 + threadIdx.x;
+  if (i < nv) {
+    float v[8];
+    unpack_chunk(ld16_stream(src + 8 * i), v, float{});
+    unpack_chunk(ld16_stream(src + 8 * i + 4), v + 4, float{});
+    st16(dst + 8 * i, pack_chunk(v, uint16_t{}));
+  }
+  if (b == 0 && threadIdx.x < n - 8 * nv) dst[8 * nv + threadIdx.x] = bf16_bits(src[8 * nv + threadIdx.x]);
+}
+
 // ------------------------------------------------------------------ padded copies
 // dst [batch, drows, dcols] (contiguous) = src[b, r, c] (strides sbs, srs, 1) where r < rows and
 // c < cols, else 0: one pass each way between rows of any width and the 16-byte rows that the
@@ -596,6 +625,36 @@ extern "C" int zmoe_cast_f32_bf16(const float* src, int64_t n, void* dst, void* 
   hipLaunchKernelGGL(cast_f32_bf16_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), src, n,
                      (uint16_t*)dst);
   return check_launch("cast_f32_bf16");
+}
+
+extern "C" int zmoe_cast_f32_bf16_segments(const float* const* src, const int64_t* n, void* const* dst, int segments,
+                                           void* stream) {
+  ZMOE_REQUIRE(segments >= 0 && segments <= ZMOE_CAST_MAX_SEGMENTS, ZMOE_ERR_SHAPE,
+               "cast_f32_bf16_segments: 0 to %d segments (%d)", ZMOE_CAST_MAX_SEGMENTS, segments);
+  ZMOE_REQUIRE(segments == 0 || (src && n && dst), ZMOE_ERR_NULL, "cast_f32_bf16_segments: null pointer");
+  CastSegments g{};
+  int used = 0;
+  int64_t blocks = 0;
+  for (int i = 0; i < segments; ++i) {
+    ZMOE_REQUIRE(n[i] >= 0, ZMOE_ERR_SHAPE, "cast_f32_bf16_segments: n < 0");
+    if (n[i] == 0) continue;
+    ZMOE_REQUIRE(src[i] && dst[i], ZMOE_ERR_NULL, "cast_f32_bf16_segments: null pointer");
+    ZMOE_REQUIRE(aligned16(src[i]) && aligned16(dst[i]), ZMOE_ERR_ALIGN,
+                 "cast_f32_bf16_segments: pointers must be 16-byte aligned");
+    g.src[used] = src[i];
+    g.dst[used] = static_cast<uint16_t*>(dst[i]);
+    g.n[used] = n[i];
+    g.first[used] = (uint32_t)blocks;
+    const int64_t chunks = n[i] / 8 > 0 ? n[i] / 8 : 1;
+    ZMOE_REQUIRE(chunks < ((int64_t)1 << 39), ZMOE_ERR_SHAPE, "cast_f32_bf16_segments: n too large");
+    blocks += cdiv(chunks, 256);
+    ZMOE_REQUIRE(blocks < (int64_t)0x7fffffff, ZMOE_ERR_SHAPE, "cast_f32_bf16_segments: n too large");
+    ++used;
+  }
+  if (used == 0) return ZMOE_OK;
+  g.first[used] = (uint32_t)blocks;
+  hipLaunchKernelGGL(cast_segments_kernel, dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), g, used);
+  return check_launch("cast_f32_bf16_segments");
 }
 
 extern "C" int zmoe_copy_pad(const void* src, int64_t src_stride_b, int64_t src_stride_r, int64_t batch, int64_t rows,

@@ -71,22 +71,31 @@ class _FusedMoELayer(torch.autograd.Function):
         bf = torch.bfloat16
         ctx.f32_grads = W1.dtype == torch.float32
         ctx.x_dtype = x.dtype
-        # bf16 compute copies of fp32 operands (one HIP pass each)
-        cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731
-        x, W1, W2 = cast(x), cast(W1), cast(W2)
-        Ws_down = Ws_down.to(bf)
         fs = Ws_up.shape[0]
+        W3 = None  # [up | gate | router] rows in one operand, [2fs + E, d]; rows :2fs = [up | gate]
+        if all(t.dtype == torch.float32 for t in (W1, W2, Ws_down, Ws_up, Ws_gate, gate_w)):
+            # bf16 compute copies of fp32 operands (one HIP pass)
+            xs = () if x.dtype == bf else (x,)
+            *xs, W1, W2, Ws_down, W3 = _zl.cast_bf16_packed([*xs, W1, W2, Ws_down, Ws_up, Ws_gate, gate_w],
+                                                            len(xs) + 3)
+            x = xs[0] if xs else x
+        else:
+            cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731
+            x, W1, W2 = cast(x), cast(W1), cast(W2)
+            Ws_down = Ws_down.to(bf)
         if _zl.glu_stream_shared_ok(x.shape[0], x.shape[1], W2.shape[2], fs, E, k):
             # few rows per expert: the launches stream weights, and the shared expert's products
             # ride in the routed experts' two (W3 below is only formed if there is a backward)
-            w3 = (Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf))
+            if W3 is None:
+                w3 = (Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf))
+            else:
+                w3 = (W3[:fs], W3[fs:2 * fs], W3[2 * fs:])
             logits = F.linear(x, w3[2])                                              # moe_gate.py:26
             idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
             se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
             H, A_s, Y_s, Hs, As, S = _zl.glu_shared_forward(x, W1, W2, ss, off, k, w_sorted, w3[0], w3[1], Ws_down)
         else:
-            # [up | gate | router] rows in one operand (cast with the concatenation)
-            w3 = (torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf),)  # [2fs + E, d]; rows :2fs = [up | gate]
+            w3 = (torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf) if W3 is None else W3,)
             logits = F.linear(x, w3[0][2 * fs:])                                     # moe_gate.py:26
             idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
             Hs = F.linear(x, w3[0][:2 * fs])
@@ -100,6 +109,8 @@ class _FusedMoELayer(torch.autograd.Function):
             Y_s = _zl.grouped_mm(A_s, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
                                  "scatter2scatter")                                  # = w * Y
         out = _zl.combine(Y_s, None, k, S, pad_rows, pad_total)                      # moe_layer.py:48-56
+        if W3 is not None:
+            w3 = (W3,)
         ctx.save_for_backward(x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3)
         ctx.k, ctx.E, ctx.fs = k, E, fs
         ctx.mark_non_differentiable(idx, off)

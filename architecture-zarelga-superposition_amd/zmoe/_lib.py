@@ -69,6 +69,7 @@ SIGNATURES = {
     "zmoe_combine_backward_rows": (I32, [P, P, P, I64, P, P, I64, I32, I64, I32, P, P, P]),
     "zmoe_sum_k": (I32, [P, I64, I32, I64, I32, P, P, I32, P, P]),
     "zmoe_cast_f32_bf16": (I32, [P, I64, P, P]),
+    "zmoe_cast_f32_bf16_segments": (I32, [P, P, P, I32, P]),
     "zmoe_copy_pad": (I32, [P, I64, I64, I64, I64, I64, I32, P, I64, I64, P]),
     "zmoe_swiglu": (I32, [P, I64, I64, I32, P, P]),
     "zmoe_swiglu_backward": (I32, [P, P, I64, I64, I32, P, I64, P]),

@@ -359,6 +359,20 @@ def _(src):
     return _empty(src.shape, src, torch.bfloat16)
 
 
+@layer_op("cast_bf16_packed")
+def cast_bf16_packed(srcs: List[torch.Tensor], cat_from: int) -> List[torch.Tensor]:
+    """``cast_bf16`` of ``srcs[:cat_from]``, and of ``srcs[cat_from:]`` concatenated along dim 0."""
+    return list(_z.cast_bf16_packed(srcs, cat_from))
+
+
+@cast_bf16_packed.register_fake
+def _(srcs, cat_from):
+    tail = srcs[cat_from:]
+    rows = sum(s.shape[0] for s in tail)
+    return ([_empty(s.shape, s, torch.bfloat16) for s in srcs[:cat_from]]
+            + [_empty((rows, *tail[0].shape[1:]), tail[0], torch.bfloat16)])
+
+
 @layer_op("swiglu")
 def swiglu(H: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up for H = [up | gate] (mlp.py:86, expert_layer.py:23-24)."""

@@ -8,6 +8,7 @@ implementation: unsupported inputs raise.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -656,6 +657,32 @@ def cast_bf16(src: torch.Tensor) -> torch.Tensor:
     out = torch.empty(src.shape, dtype=torch.bfloat16, device=dev)
     with profiling.region("cast_bf16", dev):
         L.call("zmoe_cast_f32_bf16", _ptr(src), src.numel(), _ptr(out), _stream(dev))
+    return out
+
+
+def cast_bf16_packed(srcs, cat_from: int):
+    """The bf16 copies of fp32 tensors, in one HIP pass: ``cast_bf16`` of each of
+    ``srcs[:cat_from]``, then that of ``srcs[cat_from:]`` concatenated along dim 0."""
+    dev = _require_cuda(*srcs)
+    if any(s.dtype != torch.float32 for s in srcs):
+        raise ValueError("cast_bf16_packed: float32 inputs expected")
+    srcs = [s.contiguous() for s in srcs]
+    tail = srcs[cat_from:]
+    out = [torch.empty(s.shape, dtype=torch.bfloat16, device=dev) for s in srcs[:cat_from]]
+    rows = sum(s.shape[0] for s in tail)
+    out.append(torch.empty((rows, *tail[0].shape[1:]), dtype=torch.bfloat16, device=dev))
+    dst, at = [o.data_ptr() for o in out[:-1]], out[-1].data_ptr()
+    for s in tail:
+        if s.shape[1:] != tail[0].shape[1:]:
+            raise ValueError("cast_bf16_packed: the concatenated tensors must agree past dim 0")
+        dst.append(at)
+        at += 2 * s.numel()
+    n = len(srcs)
+    if n > 8 or any(p % 16 for p in dst) or any(s.data_ptr() % 16 for s in srcs):
+        return [cast_bf16(s) for s in srcs[:cat_from]] + [torch.cat(tail, dim=0).to(torch.bfloat16)]
+    with profiling.region("cast_bf16", dev):
+        L.call("zmoe_cast_f32_bf16_segments", (ctypes.c_void_p * n)(*(s.data_ptr() for s in srcs)),
+               (ctypes.c_int64 * n)(*(s.numel() for s in srcs)), (ctypes.c_void_p * n)(*dst), n, _stream(dev))
     return out
 
 

@@ -342,6 +342,12 @@ int zmoe_sum_k(const void* Xe, int64_t T, int k, int64_t d, int dtype,
  * even, NaN kept. src and dst 16-byte aligned. */
 int zmoe_cast_f32_bf16(const float* src, int64_t n, void* dst, void* stream);
 
+/* Up to ZMOE_CAST_MAX_SEGMENTS such copies in one launch: dst[i] = bf16 of src[i]'s n[i] elements
+ * (the three arrays are read on the host, before the call returns). */
+#define ZMOE_CAST_MAX_SEGMENTS 8
+int zmoe_cast_f32_bf16_segments(const float* const* src, const int64_t* n, void* const* dst, int segments,
+                                void* stream);
+
 /* dst [batch, dst_rows, dst_cols] (contiguous) = src[b, r, c] where r < rows and c < cols, else
  * 0; src has strides (src_stride_b, src_stride_r, 1). The padded copies that rows of a width
  * the other entry points do not take (not whole 16-byte chunks) go through, and back. Pointers

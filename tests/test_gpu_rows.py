@@ -121,6 +121,31 @@ def test_cast_bf16_matches_torch(hip_device, n):
     assert torch.equal(gi[~nan], ri[~nan])
 
 
+# one-block and many-block segments, tails of 1 to 7 elements, an empty segment, one segment of the
+# concatenation that leaves the next unaligned (the general form), and eight and nine segments
+@pytest.mark.parametrize("shapes,cat_from", [([(3, 8), (5, 8)], 0),
+                                             ([(7,), (2048,), (2049, 3), (6, 16), (10, 16), (1, 16)], 3),
+                                             ([(0, 24), (513, 24), (0, 24), (9, 24)], 1),
+                                             ([(40, 33), (3, 5), (4, 5)], 1),
+                                             ([(k, 16) for k in range(1, 9)], 5),
+                                             ([(k, 16) for k in range(1, 10)], 5)])
+def test_cast_bf16_packed(hip_device, shapes, cat_from):
+    """Bit for bit torch's casts and the cast of the concatenation, from every form of the op."""
+    from zmoe import library, ops
+
+    srcs = [torch.randn(*s, generator=gen(i)).to(hip_device) for i, s in enumerate(shapes)]
+    srcs[-1].view(-1)[:2] = torch.tensor([float("inf"), float("nan")])
+    want = [s.to(torch.bfloat16) for s in srcs[:cat_from]] + [torch.cat(srcs[cat_from:]).to(torch.bfloat16)]
+    with torch.no_grad():
+        forms = [ops.cast_bf16_packed(srcs, cat_from), torch.ops.zmoe.cast_bf16_packed(srcs, cat_from),
+                 library.cast_bf16_packed(srcs, cat_from)]
+    for got in forms:
+        assert len(got) == len(want)
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and a.dtype == b.dtype
+            assert torch.equal(a.nan_to_num(7.0), b.nan_to_num(7.0)) and torch.equal(a.isnan(), b.isnan())
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_swiglu(hip_device, dtype):
     from zmoe import ops
