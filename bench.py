@@ -56,14 +56,14 @@ GEMM_OPS = ("glu_w1_forward", "scatter2scatter", "glu_w2_backward_dh", "group_bw
 # one after the other): when those differ, the line reports traffic null and says why.
 TRAFFIC_C3_PROFILE = "profiles/grouped_gemm_c3_hbm_bytes.md"
 TRAFFIC_C3_SOURCES = ("gemm.hip", "zmoe_internal.h")  # what the grouped GEMM kernels compile from
-TRAFFIC_C3_GEMM_SHA256 = "d38eed6a4335a73af29503a97c1226584f471d8cc58f3fd5205c9aaf7c53e814"
+TRAFFIC_C3_GEMM_SHA256 = "6a8781b83020dd4922df24bfad290a25517cb04d3b21e522fbf2cec7394d72d7"
 TRAFFIC_C3 = {
-    "glu_w1_forward#0": 6035677760,
-    "scatter2scatter#0": 2891170624,
-    "glu_w2_backward_dh#0": 2458364202,
-    "scatter2scatter#1": 5833844736,
-    "group_bwd_w#0": 2165850346,
-    "group_bwd_w#1": 3661097280,
+    "glu_w1_forward#0": 6090792544,
+    "scatter2scatter#0": 2875663040,
+    "glu_w2_backward_dh#0": 2496369301,
+    "scatter2scatter#1": 5726834901,
+    "group_bwd_w#0": 2166642133,
+    "group_bwd_w#1": 3670652715,
 }
 ROW_OPS = ("route_topk", "flatten_sort_count", "combine", "combine_backward", "combine_backward_scale",
            "swiglu_backward_gates", "sum_k")
