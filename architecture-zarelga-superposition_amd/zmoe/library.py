@@ -13,13 +13,13 @@ ctypes) on the current stream.
 
 from __future__ import annotations
 
-import functools
 import inspect
 import os
 import threading
 from typing import List, Optional
 
 import torch
+from torch.utils._device import DeviceContext
 
 from . import _lib as L
 from . import ops as _z
@@ -28,73 +28,77 @@ from . import profiling
 _I64 = torch.int64
 _F32 = torch.float32
 
-_eager_fakes = []   # (name, fake implementation) to register once the native ops are loaded
+_eager_loaded = False
 _eager_lock = threading.Lock()
 
 
 def _load_eager():
     """The native ops (csrc/eager_ops.cpp), loaded once; there is no fallback if they are missing."""
-    global _eager_fakes
+    global _eager_loaded
     with _eager_lock:
-        if _eager_fakes is not None:
+        if not _eager_loaded:
             L.load()  # the C ABI library they call
             if not os.path.exists(L.EAGER_PATH):
                 raise ImportError(f"{os.path.basename(L.EAGER_PATH)} not found at {L.EAGER_PATH}; build it first "
                                   "(python architecture-zarelga-superposition_amd/build_lib.py)")
             torch.ops.load_library(L.EAGER_PATH)
-            for name, fake in _eager_fakes:
-                torch.library.register_fake(f"zmoe_eager::{name}", fake)
-            _eager_fakes = None
+            _eager_loaded = True
 
 
-def layer_op(name: str, mutates_args=()):
-    """``torch.library.custom_op("zmoe::<name>")``, with the native ``zmoe_eager::<name>`` of
-    csrc/eager_ops.cpp for eager calls with gradients off.
+# Argument types that a native op takes. Others go to the custom_op: fake tensors and other subclasses
+# with a __torch_dispatch__ or __torch_function__ of their own, and symbolic sizes.
+_plain = frozenset((torch.Tensor, torch.nn.Parameter, int, bool, float, str, list, tuple, type(None))).issuperset
+
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_tracing, _functorch = torch._C._get_tracing_state, torch._C._functorch.peek_interpreter_stack
+_compiling, _grad_enabled, _forward_ad = torch.compiler.is_compiling, torch.is_grad_enabled, torch.autograd.forward_ad
+
+
+def _watched_by_function_mode() -> bool:
+    """Whether a torch-function mode is active besides a default device's, which watches no op."""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(_function_modes()))
+
+
+class LayerOp(torch.library.CustomOpDef):
+    """The custom op ``zmoe::<name>``, whose eager calls with gradients off run the native
+    ``zmoe_eager::<name>`` of csrc/eager_ops.cpp.
 
     The layer calls its ops from inside autograd functions, where grad mode is off and there is
     nothing to record; a small layer's step is bound by the host time of its ~25 calls, most of
-    it custom_op's Python (autograd kernel, redispatch, alias check) and the wrapper's. The
-    native op is an ordinary dispatcher kernel, so modes, fake tensors and profilers see it. With
+    it custom_op's Python (autograd kernel, redispatch, alias check) and the wrapper's. With
     grad mode on (a caller outside an autograd function, or a backward with create_graph) the
-    call goes to the custom_op, which refuses a backward through it; while compiling too, so
-    compiled graphs hold the zmoe:: names, with a symbolic size (the native ops take integers),
-    and while zmoe.profiling times single launches."""
+    call goes to the custom_op, which refuses a backward through it. So does a call that is
+    observed by what knows the ops by their zmoe:: names or has rules registered on them (a
+    compiler or tracer, a dispatch or function mode, a functorch transform, forward-mode AD), and
+    one that zmoe.profiling times."""
+
+    def __call__(self, *args, **kwargs):
+        if (_compiling() or _grad_enabled() or kwargs or _dispatch_modes() or _functorch() is not None
+                or _forward_ad._current_level >= 0 or _tracing() is not None or profiling.active()
+                or not _plain(map(type, args)) or (_function_modes() and _watched_by_function_mode())
+                or (self._lists and not all(_plain(map(type, args[i])) for i in self._lists if i < len(args)))):
+            return super().__call__(*args, **kwargs)
+        if self._native is None:
+            _load_eager()
+            self._native = getattr(torch.ops.zmoe_eager, self._name).default
+        out = self._native(*args)
+        for i in self._mutated:  # as custom_op does: autograd sees that the tensor changed
+            if i < len(args) and args[i] is not None:
+                torch.autograd.graph.increment_version(args[i])
+        return out
+
+
+def layer_op(name: str, mutates_args=()):
+    """Decorator: ``torch.library.custom_op("zmoe::<name>")`` as a ``LayerOp``."""
 
     def wrap(fn):
-        custom = torch.library.custom_op(f"zmoe::{name}", mutates_args=mutates_args)(fn)
-        params = tuple(inspect.signature(fn).parameters)
-        mutated = tuple(params.index(m) for m in mutates_args)
-        native = None
-
-        @functools.wraps(fn)
-        def call(*args, **kwargs):
-            nonlocal native
-            if (kwargs or torch.is_grad_enabled() or torch.compiler.is_compiling() or profiling.active()
-                    or torch.SymInt in map(type, args)):
-                return custom(*args, **kwargs)
-            if native is None:
-                _load_eager()
-                native = getattr(torch.ops.zmoe_eager, name).default
-            out = native(*args)
-            for i in mutated:  # as custom_op does: autograd sees that the tensor changed
-                if i < len(args) and args[i] is not None:
-                    torch.autograd.graph.increment_version(args[i])
-            return out
-
-        def register_fake(fake):
-            custom.register_fake(fake)
-            with _eager_lock:
-                if _eager_fakes is None:  # the native ops are loaded already
-                    torch.library.register_fake(f"zmoe_eager::{name}", fake)
-                else:
-                    _eager_fakes.append((name, fake))
-            return fake
-
-        call.register_fake = register_fake
-        for method in ("register_kernel", "register_autograd", "register_vmap", "register_torch_dispatch",
-                       "set_kernel_enabled"):
-            setattr(call, method, getattr(custom, method))
-        return call
+        op = torch.library.custom_op(f"zmoe::{name}", mutates_args=mutates_args)(fn)
+        op.__class__ = LayerOp
+        op._native = None
+        params = inspect.signature(fn).parameters
+        op._mutated = tuple(i for i, p in enumerate(params) if p in mutates_args)
+        op._lists = tuple(i for i, p in enumerate(params.values()) if str(p.annotation).startswith("List["))
+        return op
 
     return wrap
 
