@@ -83,22 +83,24 @@ class _FusedMoELayer(torch.autograd.Function):
             cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731
             x, W1, W2 = cast(x), cast(W1), cast(W2)
             Ws_down = Ws_down.to(bf)
-        if _zl.glu_stream_shared_ok(x.shape[0], x.shape[1], W2.shape[2], fs, E, k):
+        streamed = _zl.glu_stream_shared_ok(x.shape[0], x.shape[1], W2.shape[2], fs, E, k)
+        if W3 is None and (backward or not streamed):
+            W3 = torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf)
+        if streamed:
             # few rows per expert: the launches stream weights, and the shared expert's products
-            # ride in the routed experts' two (W3 below is only formed if there is a backward)
+            # ride in the routed experts' two, which take the parts of W3 (only a backward needs it)
             if W3 is None:
-                w3 = (Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf))
+                up, gate, router = Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf)
             else:
-                w3 = (W3[:fs], W3[fs:2 * fs], W3[2 * fs:])
-            logits = F.linear(x, w3[2])                                              # moe_gate.py:26
+                up, gate, router = W3[:fs], W3[fs:2 * fs], W3[2 * fs:]
+            logits = F.linear(x, router)                                             # moe_gate.py:26
             idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
             se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
-            H, A_s, Y_s, Hs, As, S = _zl.glu_shared_forward(x, W1, W2, ss, off, k, w_sorted, w3[0], w3[1], Ws_down)
+            H, A_s, Y_s, Hs, As, S = _zl.glu_shared_forward(x, W1, W2, ss, off, k, w_sorted, up, gate, Ws_down)
         else:
-            w3 = (torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf) if W3 is None else W3,)
-            logits = F.linear(x, w3[0][2 * fs:])                                     # moe_gate.py:26
+            logits = F.linear(x, W3[2 * fs:])                                        # moe_gate.py:26
             idx, w, p = _zl.route_topk(logits, expert_biases, k, True)
-            Hs = F.linear(x, w3[0][:2 * fs])
+            Hs = F.linear(x, W3[:2 * fs])
             As = _zl.swiglu(Hs)
             S = F.linear(As, Ws_down)                                                # expert_layer.py:23-24
             se, ss, off, inv, w_sorted = _zl.flatten_sort_count_weights(idx, w, E)   # mlp.py:76-77
@@ -109,9 +111,7 @@ class _FusedMoELayer(torch.autograd.Function):
             Y_s = _zl.grouped_mm(A_s, W2.permute(0, 2, 1), se, ss, 1, True, False, off,
                                  "scatter2scatter")                                  # = w * Y
         out = _zl.combine(Y_s, None, k, S, pad_rows, pad_total)                      # moe_layer.py:48-56
-        if W3 is not None:
-            w3 = (W3,)
-        ctx.save_for_backward(x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3)
+        ctx.save_for_backward(x, W1, W2, W3, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows)
         ctx.k, ctx.E, ctx.fs = k, E, fs
         ctx.mark_non_differentiable(idx, off)
         ctx.set_materialize_grads(False)  # no zero-filled grads for idx and off (two fill launches)
@@ -121,8 +121,7 @@ class _FusedMoELayer(torch.autograd.Function):
     def backward(ctx, dout, d_idx, d_off):
         if dout is None:  # out took no part in the loss
             return (None,) * 13
-        x, W1, W2, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows, *w3 = ctx.saved_tensors
-        W3 = w3[0] if len(w3) == 1 else torch.cat(w3, dim=0)  # [up | gate | router]
+        x, W1, W2, W3, Ws_down, Hs, As, p, idx, w_sorted, se, ss, off, H, A_s, pad_rows = ctx.saved_tensors
         k, E, fs = ctx.k, ctx.E, ctx.fs
         need = ctx.needs_input_grad
         f32 = ctx.f32_grads  # fp32 weight grads from the accumulators (fp32 master weights)

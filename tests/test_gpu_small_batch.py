@@ -1,0 +1,59 @@
+"""The layer at few rows per expert, where its forward streams the routed and the shared experts'
+weights in two launches (zmoe_glu_stream_shared_ok): against the oracle with its backward, and what the
+route owes its callers."""
+
+import pytest
+import torch
+
+from helpers import gen
+
+pytestmark = pytest.mark.gpu
+
+
+def _streams(T, d, f, fs, E, k):
+    from zmoe import library as zl
+
+    return zl.glu_stream_shared_ok(T, d, f, fs, E, k)
+
+
+def _layer(dev, dtype, d=128, E=64, k=4, f=64, n_shared=1, seed=0):
+    from modeling.model_config import ModelConfig
+    from modeling.moe_layer import MoELayer
+
+    torch.manual_seed(seed)
+    cfg = ModelConfig(hidden_size=d, intermediate_size=f, n_experts=E + n_shared, n_shared_experts=n_shared,
+                      n_experts_per_token=k)
+    layer = MoELayer(cfg).to(dev).to(dtype)
+    layer.gate.expert_biases.data = (0.1 * torch.randn(E)).to(dev)
+    return layer
+
+
+def _step(layer, x, dout, between=None, **kw):
+    """(out, dx, weight grads by name) of one step; ``between`` runs after the forward."""
+    layer.zero_grad(set_to_none=True)
+    x = x.clone().requires_grad_(True)
+    out, idx = layer(x, **kw)
+    if between is not None:
+        with torch.no_grad():
+            between()
+    out.backward(dout)
+    return out.detach(), x.grad, {n: p.grad.clone() for n, p in layer.named_parameters()}
+
+
+def _equal(a, b):
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+    for n in a[2]:
+        assert torch.equal(a[2][n], b[2][n]), n
+
+
+def test_weights_edited_between_forward_and_backward(hip_device):
+    """The backward takes the shared expert's up and gate and the router as the forward saw them."""
+    T, dt = 16, torch.bfloat16
+    assert _streams(T, 128, 64, 64, 64, 4)
+    layer = _layer(hip_device, dt)
+    x = torch.randn(1, T, 128, generator=gen(1)).to(dt).to(hip_device)
+    dout = torch.randn(1, T, 128, generator=gen(2)).to(dt).to(hip_device)
+    ref = _step(layer, x, dout)
+    se = layer.shared_experts
+    _equal(_step(layer, x, dout, lambda: [w.mul_(2) for w in (layer.gate.weight, se.up_proj.weight,
+                                                              se.gate_proj.weight)]), ref)
