@@ -55,6 +55,12 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
     return t if t.stride(1) == 1 else t.contiguous()
 
 
+def _on16(t: torch.Tensor) -> torch.Tensor:
+    """``t`` contiguous from a 16-byte boundary (a copy where it is not: a view into a flat buffer)."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _idx64(t: torch.Tensor) -> torch.Tensor:
     t = t.reshape(-1)
     if t.dtype != torch.int64:
@@ -492,10 +498,11 @@ def glu_shared_forward(x: torch.Tensor, W1: torch.Tensor, W2: torch.Tensor, sort
                        W_gate: torch.Tensor, W_down: torch.Tensor):
     """The routed and the shared experts' forward on the weight-streaming path, two launches (bf16,
     sizes of ``glu_stream_shared_ok``): (H [R, 2f], A [R, f] scaled by ``row_scale``, Y [R, d] in slot
-    order, Hs [T, 2fs] = [up | gate], As [T, fs], S [T, d])."""
+    order, Hs [T, 2fs] = [up | gate], As [T, fs], S [T, d]). The shared expert's weights may start at
+    any element, as the library GEMMs that take them elsewhere allow."""
     dev = _require_cuda(x, W1, W2, sorted_scattered_idxs, expert_offsets, row_scale, W_up, W_gate, W_down)
     x, W1, W2 = x.contiguous(), W1.contiguous(), W2.contiguous()
-    W_up, W_gate, W_down = W_up.contiguous(), W_gate.contiguous(), W_down.contiguous()
+    W_up, W_gate, W_down = _on16(W_up), _on16(W_gate), _on16(W_down)
     if any(t.dtype != torch.bfloat16 for t in (x, W1, W2, W_up, W_gate, W_down)):
         raise ValueError("glu_shared_forward: bf16 operands only")
     T, d = x.shape

@@ -57,3 +57,35 @@ def test_weights_edited_between_forward_and_backward(hip_device):
     se = layer.shared_experts
     _equal(_step(layer, x, dout, lambda: [w.mul_(2) for w in (layer.gate.weight, se.up_proj.weight,
                                                               se.gate_proj.weight)]), ref)
+
+
+def _off16(layer, names):
+    """The named weights as parameters that start one element into a buffer of their own."""
+    for n in names:
+        mod = layer.get_submodule(n.rpartition(".")[0])
+        w = mod.weight.detach()
+        buf = torch.empty(w.numel() + 1, dtype=w.dtype, device=w.device)
+        view = buf[1:].view(w.shape)
+        view.copy_(w)
+        mod.weight = torch.nn.Parameter(view)
+        assert mod.weight.data_ptr() % 16
+
+
+SHARED = tuple(f"shared_experts.{p}_proj.weight" for p in ("up", "gate", "down"))
+
+
+def test_shared_weights_off_16_bytes(hip_device):
+    """A shared expert whose weights are views into a flat buffer: taken, with the same bits; the
+    routed experts' weights are still refused there, as they are at every size."""
+    T, dt = 8, torch.bfloat16
+    assert _streams(T, 128, 64, 64, 64, 4)
+    x = torch.randn(1, T, 128, generator=gen(3)).to(dt).to(hip_device)
+    layer = _layer(hip_device, dt).requires_grad_(False)
+    ref = layer(x)[0]
+    for names in (SHARED[:1], SHARED[1:2], SHARED[2:], SHARED):
+        layer = _layer(hip_device, dt).requires_grad_(False)
+        _off16(layer, names)
+        assert torch.equal(layer(x)[0], ref)
+    _off16(layer, ("routed_experts.experts.weight",))
+    with pytest.raises(ValueError):
+        layer(x)
