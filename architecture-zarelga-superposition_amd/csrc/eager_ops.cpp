@@ -505,7 +505,7 @@ Tensor cast_bf16(const Tensor& src) {
   return op.call(src);
 }
 
-Tensors cast_bf16_packed(at::TensorList srcs, int64_t cat_from) {
+Tensors cast_bf16_packed(at::TensorList srcs, int64_t cat_from, int64_t any_from) {
   const int64_t n = (int64_t)srcs.size();
   if (cat_from >= 0 && cat_from < n && n <= ZMOE_CAST_MAX_SEGMENTS && srcs[0].is_cuda()) {
     const Tensor& x = srcs[0];
@@ -538,8 +538,8 @@ Tensors cast_bf16_packed(at::TensorList srcs, int64_t cat_from) {
       if (zmoe_cast_f32_bf16_segments(src, count, dst, (int)n, stream_of(x)) == ZMOE_OK) return out;
     }
   }
-  static const auto op = general<Tensors(at::TensorList, c10::SymInt)>("zmoe::cast_bf16_packed");
-  return op.call(srcs, cat_from);
+  static const auto op = general<Tensors(at::TensorList, c10::SymInt, c10::SymInt)>("zmoe::cast_bf16_packed");
+  return op.call(srcs, cat_from, any_from);
 }
 
 Tensor swiglu(const Tensor& H) {
@@ -717,7 +717,7 @@ TORCH_LIBRARY(zmoe_eager, m) {
              "(Tensor Y, Tensor grad_out, Tensor gates, Tensor inverse, Tensor? grad_rows) -> Tensor[]");
   ZMOE_EAGER(sum_k, "(Tensor Xe, int k, Tensor? add0, bool out_f32=False) -> Tensor");
   ZMOE_EAGER(cast_bf16, "(Tensor src) -> Tensor");
-  ZMOE_EAGER(cast_bf16_packed, "(Tensor[] srcs, int cat_from) -> Tensor[]");
+  ZMOE_EAGER(cast_bf16_packed, "(Tensor[] srcs, int cat_from, int any_from=-1) -> Tensor[]");
   ZMOE_EAGER(swiglu, "(Tensor H) -> Tensor");
   ZMOE_EAGER(swiglu_backward, "(Tensor dA, Tensor H) -> Tensor");
   ZMOE_EAGER(swiglu_backward_gates, "(Tensor dA, Tensor H, Tensor row_scale, Tensor slot_of_row) -> Tensor[]");

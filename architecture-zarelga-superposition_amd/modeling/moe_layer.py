@@ -74,10 +74,10 @@ class _FusedMoELayer(torch.autograd.Function):
         fs = Ws_up.shape[0]
         W3 = None  # [up | gate | router] rows in one operand, [2fs + E, d]; rows :2fs = [up | gate]
         if all(t.dtype == torch.float32 for t in (W1, W2, Ws_down, Ws_up, Ws_gate, gate_w)):
-            # bf16 compute copies of fp32 operands (one HIP pass)
+            # bf16 compute copies of fp32 operands (one HIP pass; the dense weights may start anywhere)
             xs = () if x.dtype == bf else (x,)
             *xs, W1, W2, Ws_down, W3 = _zl.cast_bf16_packed([*xs, W1, W2, Ws_down, Ws_up, Ws_gate, gate_w],
-                                                            len(xs) + 3)
+                                                            len(xs) + 3, len(xs) + 2)
             x = xs[0] if xs else x
         else:
             cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731

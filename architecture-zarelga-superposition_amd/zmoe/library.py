@@ -364,13 +364,14 @@ def _(src):
 
 
 @layer_op("cast_bf16_packed")
-def cast_bf16_packed(srcs: List[torch.Tensor], cat_from: int) -> List[torch.Tensor]:
-    """``cast_bf16`` of ``srcs[:cat_from]``, and of ``srcs[cat_from:]`` concatenated along dim 0."""
-    return list(_z.cast_bf16_packed(srcs, cat_from))
+def cast_bf16_packed(srcs: List[torch.Tensor], cat_from: int, any_from: int = -1) -> List[torch.Tensor]:
+    """``cast_bf16`` of ``srcs[:cat_from]``, and of ``srcs[cat_from:]`` concatenated along dim 0;
+    ``srcs[any_from:]`` (-1: the concatenated ones) may start at any element."""
+    return list(_z.cast_bf16_packed(srcs, cat_from, any_from))
 
 
 @cast_bf16_packed.register_fake
-def _(srcs, cat_from):
+def _(srcs, cat_from, any_from=-1):
     tail = srcs[cat_from:]
     rows = sum(s.shape[0] for s in tail)
     return ([_empty(s.shape, s, torch.bfloat16) for s in srcs[:cat_from]]

@@ -667,13 +667,16 @@ def cast_bf16(src: torch.Tensor) -> torch.Tensor:
     return out
 
 
-def cast_bf16_packed(srcs, cat_from: int):
+def cast_bf16_packed(srcs, cat_from: int, any_from: int = -1):
     """The bf16 copies of fp32 tensors, in one HIP pass: ``cast_bf16`` of each of
-    ``srcs[:cat_from]``, then that of ``srcs[cat_from:]`` concatenated along dim 0."""
+    ``srcs[:cat_from]``, then that of ``srcs[cat_from:]`` concatenated along dim 0. Those from
+    ``any_from`` on (-1: from ``cat_from``) may start at any element, and are copied where that is
+    not on 16 bytes; the others have to start on 16 bytes, as ``cast_bf16``'s."""
+    any_from = cat_from if any_from < 0 else any_from
     dev = _require_cuda(*srcs)
     if any(s.dtype != torch.float32 for s in srcs):
         raise ValueError("cast_bf16_packed: float32 inputs expected")
-    srcs = [s.contiguous() for s in srcs]
+    srcs = [s.contiguous() for s in srcs[:any_from]] + [_on16(s) for s in srcs[any_from:]]
     tail = srcs[cat_from:]
     out = [torch.empty(s.shape, dtype=torch.bfloat16, device=dev) for s in srcs[:cat_from]]
     rows = sum(s.shape[0] for s in tail)
@@ -685,7 +688,7 @@ def cast_bf16_packed(srcs, cat_from: int):
         dst.append(at)
         at += 2 * s.numel()
     n = len(srcs)
-    if n > 8 or any(p % 16 for p in dst) or any(s.data_ptr() % 16 for s in srcs):
+    if n > 8 or any(p % 16 for p in dst):
         return [cast_bf16(s) for s in srcs[:cat_from]] + [torch.cat(tail, dim=0).to(torch.bfloat16)]
     with profiling.region("cast_bf16", dev):
         L.call("zmoe_cast_f32_bf16_segments", (ctypes.c_void_p * n)(*(s.data_ptr() for s in srcs)),

@@ -28,11 +28,12 @@ def _layer(dev, dtype, d=128, E=64, k=4, f=64, n_shared=1, seed=0):
     return layer
 
 
-def _step(layer, x, dout, between=None, **kw):
+def _step(layer, x, dout, between=None, autocast=False, **kw):
     """(out, dx, weight grads by name) of one step; ``between`` runs after the forward."""
     layer.zero_grad(set_to_none=True)
     x = x.clone().requires_grad_(True)
-    out, idx = layer(x, **kw)
+    with torch.autocast("cuda", dtype=torch.bfloat16, enabled=autocast):
+        out, idx = layer(x, **kw)
     if between is not None:
         with torch.no_grad():
             between()
@@ -89,3 +90,22 @@ def test_shared_weights_off_16_bytes(hip_device):
     _off16(layer, ("routed_experts.experts.weight",))
     with pytest.raises(ValueError):
         layer(x)
+
+
+@pytest.mark.parametrize("T", [16, 300])   # the streaming route, and the other
+def test_fp32_shared_weights_off_16_bytes(hip_device, T):
+    """fp32 weights under bf16 autocast: the dense ones (shared expert, router) may start at any
+    element, in the forward and the backward; the routed experts' are refused, as they always were."""
+    assert _streams(T, 128, 64, 64, 64, 4) == (T == 16)
+    x = torch.randn(1, T, 128, generator=gen(4)).to(hip_device)
+    dout = torch.randn(1, T, 128, generator=gen(5)).to(torch.bfloat16).to(hip_device)
+    ref = _step(_layer(hip_device, torch.float32), x, dout, autocast=True)
+    for names in (SHARED[2:], ("gate.weight",), (*SHARED, "gate.weight")):
+        layer = _layer(hip_device, torch.float32)
+        _off16(layer, names)
+        _equal(_step(layer, x, dout, autocast=True), ref)
+    for name in ("routed_experts.experts.weight", "routed_experts.output_experts.weight"):
+        layer = _layer(hip_device, torch.float32)
+        _off16(layer, (name,))
+        with pytest.raises(ValueError):
+            _step(layer, x, dout, autocast=True)
