@@ -314,14 +314,15 @@ __global__ __launch_bounds__(256) void cast_segments_kernel(const CastSegments g
 // other kernels take. A wave walks 64 16-byte chunks of a destination row, 4 rows per block, so
 // both sides are contiguous; rows that do not start on 16 bytes use the same loads and stores
 // unaligned (global memory takes any alignment of the element), the last partial chunk of a row
-// goes by elements. Bound by HBM and the launch: 16 bf16 [1030, 510] matrices into [1032, 512] in
-// 8.8 us (3.8 TB/s); as a zero fill and a strided copy 24-27 us, 47-51 us where it also transposed.
+// goes by elements. The blocks run over y and z, so that any number of rows is one launch. Bound by
+// HBM and the launch: 16 bf16 [1030, 510] matrices into [1032, 512] in 6.7 us, 256 of them in 124
+// (as a zero fill and a strided copy 21 and 213 us; a launch per matrix took 692 us for the 256).
 template <typename T>
 __global__ __launch_bounds__(kRowThreads) void copy_pad_kernel(const T* __restrict__ src, int64_t sbs, int64_t srs,
                                                                int64_t rows, int64_t cols, T* __restrict__ dst,
                                                                int64_t drows, int64_t dcols, int64_t total_rows) {
   constexpr int VN = 16 / sizeof(T);
-  const int64_t row = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int64_t row = ((int64_t)blockIdx.z * gridDim.y + blockIdx.y) * 4 + (threadIdx.x >> 6);
   const int64_t c0 = ((int64_t)blockIdx.x * 64 + (threadIdx.x & 63)) * VN;
   if (row >= total_rows || c0 >= dcols) return;
   const int64_t b = row / drows, r = row - b * drows;
@@ -669,35 +670,16 @@ extern "C" int zmoe_copy_pad(const void* src, int64_t src_stride_b, int64_t src_
   ZMOE_REQUIRE(dst_rows <= kMax / batch, ZMOE_ERR_SHAPE, "copy_pad: sizes too large");
   const int64_t total = batch * dst_rows;
   const int64_t nch = cdiv(dst_cols, 16 / dtype_size(dtype));
-  const int64_t rows_per_launch = 4 * 65535;  // grid.y
+  const int64_t blocks = cdiv(total, 4);
+  const int64_t gy = blocks < 65535 ? blocks : 65535;
+  const dim3 grid((unsigned)cdiv(nch, 64), (unsigned)gy, (unsigned)cdiv(blocks, gy));
   hipStream_t s = as_stream(stream);
-  // a launch takes whole batches of rows only when one launch is not enough, so that (batch, row)
-  // stay a plain division: larger copies go row block by row block of one batch
-  if (total <= rows_per_launch) {
-    const dim3 grid((unsigned)cdiv(nch, 64), (unsigned)cdiv(total, 4));
-    if (dtype == ZMOE_DTYPE_BF16)
-      hipLaunchKernelGGL(copy_pad_kernel<uint16_t>, grid, dim3(kRowThreads), 0, s, (const uint16_t*)src, src_stride_b,
-                         src_stride_r, rows, cols, (uint16_t*)dst, dst_rows, dst_cols, total);
-    else
-      hipLaunchKernelGGL(copy_pad_kernel<float>, grid, dim3(kRowThreads), 0, s, (const float*)src, src_stride_b,
-                         src_stride_r, rows, cols, (float*)dst, dst_rows, dst_cols, total);
-    return check_launch("copy_pad");
-  }
-  const int64_t es = dtype_size(dtype);
-  for (int64_t b = 0; b < batch; ++b)
-    for (int64_t r0 = 0; r0 < dst_rows; r0 += rows_per_launch) {
-      const int64_t n = dst_rows - r0 < rows_per_launch ? dst_rows - r0 : rows_per_launch;
-      const int64_t live = rows > r0 ? rows - r0 : 0;
-      const char* sp = static_cast<const char*>(src) + (b * src_stride_b + r0 * src_stride_r) * es;
-      char* dp = static_cast<char*>(dst) + (b * dst_rows + r0) * dst_cols * es;
-      const dim3 grid((unsigned)cdiv(nch, 64), (unsigned)cdiv(n, 4));
-      if (dtype == ZMOE_DTYPE_BF16)
-        hipLaunchKernelGGL(copy_pad_kernel<uint16_t>, grid, dim3(kRowThreads), 0, s, (const uint16_t*)sp, 0,
-                           src_stride_r, live, cols, (uint16_t*)dp, n, dst_cols, n);
-      else
-        hipLaunchKernelGGL(copy_pad_kernel<float>, grid, dim3(kRowThreads), 0, s, (const float*)sp, 0, src_stride_r,
-                           live, cols, (float*)dp, n, dst_cols, n);
-    }
+  if (dtype == ZMOE_DTYPE_BF16)
+    hipLaunchKernelGGL(copy_pad_kernel<uint16_t>, grid, dim3(kRowThreads), 0, s, (const uint16_t*)src, src_stride_b,
+                       src_stride_r, rows, cols, (uint16_t*)dst, dst_rows, dst_cols, total);
+  else
+    hipLaunchKernelGGL(copy_pad_kernel<float>, grid, dim3(kRowThreads), 0, s, (const float*)src, src_stride_b,
+                       src_stride_r, rows, cols, (float*)dst, dst_rows, dst_cols, total);
   return check_launch("copy_pad");
 }
 

@@ -176,6 +176,30 @@ def test_copy_pad(hip_device, dtype, batch, rows, cols, drows, dcols):
     assert torch.equal(out, ref)
 
 
+def test_copy_pad_is_one_launch(hip_device):
+    """Any number of rows goes in one launch (also many small matrices: a captured graph's nodes)."""
+    import ctypes
+
+    from zmoe import _lib, ops
+
+    src = torch.randn(300, 1001, 5, device=hip_device)
+    out = torch.empty(300, 1002, 8, device=hip_device)       # 300600 rows, more than a grid's y takes by fours
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        ops.copy_pad(src, 1002, 8, out)
+    nodes = ctypes.c_size_t(0)
+    # (the library's handle resolves the runtime that it is linked to)
+    rc = _lib.load().hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(nodes))
+    assert rc == 0 and nodes.value == 1
+    graph.instantiate()
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[:, :1001, :5], src)
+        assert not out[:, 1001:].any() and not out[:, :, 5:].any()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("N", [8, 32, 40, 64, 136])
 def test_bias_grad_row_counts(hip_device, dtype, N):
