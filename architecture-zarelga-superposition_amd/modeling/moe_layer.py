@@ -83,11 +83,12 @@ class _FusedMoELayer(torch.autograd.Function):
             cast = lambda t: t if t.dtype == bf else _zl.cast_bf16(t)  # noqa: E731
             x, W1, W2 = cast(x), cast(W1), cast(W2)
             Ws_down = Ws_down.to(bf)
-        streamed = _zl.glu_stream_shared_ok(x.shape[0], x.shape[1], W2.shape[2], fs, E, k)
+        (T, d), f = x.shape, W2.shape[2]
+        streamed = _zl.glu_stream_shared_ok(T, d, f, fs, E, k) and _zl.glu_stream_shared_pays(T, d, fs)
         if W3 is None and (backward or not streamed):
             W3 = torch.cat([Ws_up, Ws_gate, gate_w], dim=0).to(bf)
         if streamed:
-            # few rows per expert: the launches stream weights, and the shared expert's products
+            # few rows per expert, few tokens: the launches stream weights, and the shared expert's products
             # ride in the routed experts' two, which take the parts of W3 (only a backward needs it)
             if W3 is None:
                 up, gate, router = Ws_up.to(bf), Ws_gate.to(bf), gate_w.to(bf)

@@ -182,6 +182,7 @@ def _(expert_idxs, weights, num_experts):
 
 # ------------------------------------------------------------------ grouped GEMMs
 glu_stream_shared_ok = _z.glu_stream_shared_ok
+glu_stream_shared_pays = _z.glu_stream_shared_pays
 
 
 @layer_op("glu_shared_forward")

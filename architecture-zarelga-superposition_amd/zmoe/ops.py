@@ -493,6 +493,21 @@ def glu_stream_shared_ok(T: int, d: int, f: int, fs: int, E: int, k: int) -> boo
             and max(T * d, T * k * f, T * fs, 2 * f * d) <= span and max(d, f, fs) < 1 << 24)
 
 
+def glu_stream_shared_pays(T: int, d: int, fs: int) -> bool:
+    """Whether the shared expert, which has all T tokens, is better off in the streaming launches than
+    in library GEMMs beside them. There its weights are streamed once per group of 32 tokens, from L2
+    after the first: about 0.5 us per group and million weights (3 fs d of them), against 12-18 us and
+    the library's own reads, more where only it needs the weights concatenated. T is large where k is
+    small. The routed and shared products, in the launches / library / library and concatenation, us:
+    d = 2048, fs = 1536, E = 256, k = 1: 262 / 284 / 298 at T = 192 (the last inside the rule), 402 / 378 /
+    391 at 384, 738 / 522 / 535 at 2048; d = 1024, fs = 1024, E = 1024, k = 1: 200 / 208 / 217 at 384,
+    405 / 383 / 393 at 1024, 1009 / 667 / 675 at 8192; d = 512, fs = 384: 125 / 125 / 132 at 2048, 210 /
+    167 / 173 at 8192; d = 7168, fs = 2048, E = 64, k = 2: 989 / 1011 / 1059 at 96, 1062 / 1044 / 1088 at
+    128, 1213 / 1114 / 1160 at 256."""
+    groups = (T + 31) // 32
+    return (2 * groups - 5) * fs * d <= 3 << 23
+
+
 def glu_shared_forward(x: torch.Tensor, W1: torch.Tensor, W2: torch.Tensor, sorted_scattered_idxs: torch.Tensor,
                        expert_offsets: torch.Tensor, k: int, row_scale: torch.Tensor, W_up: torch.Tensor,
                        W_gate: torch.Tensor, W_down: torch.Tensor):

@@ -256,8 +256,9 @@ int zmoe_glu_act_forward(const void* X, int64_t x_stride_m, const void* W1,
 /* Small batches (few rows per expert, bf16): the two forward launches of the routed experts with
  * the shared expert's products (expert_layer.py:23-24) in the same launches. ok returns 1 for the
  * sizes they take (T * k <= 8 E; d, f and fs multiples of 64), else 0 and they return
- * ZMOE_ERR_SHAPE. Contiguous operands: X [T, d], W_up and W_gate [fs, d], W_down [d, fs]; H, A, Y as
- * zmoe_glu_w1_forward_scaled's and zmoe_scatter2scatter's (Y in slot order); Hs [T, 2 fs] = [up |
+ * ZMOE_ERR_SHAPE; they pay while the shared expert has few groups of 32 tokens (the layer asks for
+ * (2 ceil(T / 32) - 5) fs d <= 3 * 2^23). Contiguous operands: X [T, d], W_up and W_gate [fs, d],
+ * W_down [d, fs]; H, A, Y as zmoe_glu_w1_forward_scaled's and zmoe_scatter2scatter's (Y in slot order); Hs [T, 2 fs] = [up |
  * gate], As [T, fs] = silu(gate) * up, S [T, d] = As W_down^T. */
 int zmoe_glu_stream_shared_ok(int64_t T, int64_t d, int64_t f, int64_t fs, int E, int k);
 int zmoe_glu_w1_forward_shared(const void* X, const void* W1, const int64_t* sorted_scattered_idxs,

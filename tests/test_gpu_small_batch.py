@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 def _streams(T, d, f, fs, E, k):
     from zmoe import library as zl
 
-    return zl.glu_stream_shared_ok(T, d, f, fs, E, k)
+    return zl.glu_stream_shared_ok(T, d, f, fs, E, k) and zl.glu_stream_shared_pays(T, d, fs)
 
 
 def _layer(dev, dtype, d=128, E=64, k=4, f=64, n_shared=1, seed=0):
@@ -109,3 +109,18 @@ def test_fp32_shared_weights_off_16_bytes(hip_device, T):
         _off16(layer, (name,))
         with pytest.raises(ValueError):
             _step(layer, x, dout, autocast=True)
+
+
+@pytest.mark.parametrize("T", [192, 193])
+def test_shared_expert_leaves_the_launches(hip_device, T, monkeypatch):
+    """Few rows per routed expert, but so many tokens that the shared expert is better off in library
+    GEMMs: the layer takes those (d = 2048, a shared width of 1536: from seven groups of 32 tokens)."""
+    from test_gpu_layer import run_and_compare
+    from zmoe import library as zl
+
+    calls = []
+    real = zl.glu_shared_forward
+    monkeypatch.setattr(zl, "glu_shared_forward", lambda *a: calls.append(1) or real(*a))
+    assert T * 1 <= 8 * 32
+    run_and_compare(T, 2048, 32, 1, 64, 24, torch.bfloat16, hip_device)
+    assert len(calls) == (T == 192)
