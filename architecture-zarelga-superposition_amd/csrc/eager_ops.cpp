@@ -377,36 +377,19 @@ Tensor group_bwd_w_gather_dy(const Tensor& DY, const Tensor& gather, int64_t div
   return op.call(DY, gather, div, X, off, E, out_f32);
 }
 
-// The split count of zmoe.ops.dense_wgrad_splits (the same cost model and tie order).
-int dense_wgrad_splits(int64_t M, int64_t N, int64_t K) {
-  const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  const int64_t tile = (M >= 256 && N >= 256 && K >= 256) ? 256 : 128;
-  const int64_t tiles = cdiv(N, tile) * cdiv(K, tile);
-  int best = 1;
-  double least = 0;
-  for (int s = 1; s <= 64; ++s) {
-    if (s > 1 && M / s < 1024) continue;
-    const double extra = s == 1 ? 0.0 : 2.0 * s * N * K * 4 / 5.0e6;
-    const double cost = (double)cdiv(tiles * s, 256) * ((double)cdiv(M, 64 * s) * 1.6 + 11.0) + extra;
-    if (s == 1 || cost < least) {
-      least = cost;
-      best = s;
-    }
-  }
-  return best;
-}
-
 Tensor dense_wgrad(const Tensor& DY, const Tensor& X, bool out_f32) {
   if (DY.is_cuda() && known(DY) && rows2(DY, DY) && rows2(X, DY) && X.size(0) == DY.size(0)) {
     const c10::DeviceGuard guard(DY.device());
     const int64_t M = DY.size(0), N = DY.size(1), K = X.size(1);
-    const int splits = dense_wgrad_splits(M, N, K);
-    Tensor dW = empty({N, K}, DY, wgrad_dtype(DY, out_f32));
-    const size_t bytes = zmoe_dense_wgrad_workspace_bytes(N, K, DY.scalar_type() == at::kBFloat16 ? splits : 0);
-    Tensor ws = workspace(bytes, DY);
-    if (zmoe_dense_wgrad(raw(DY), DY.stride(0), raw(X), X.stride(0), M, N, K, code(DY), code(dW), splits, raw(dW),
-                         raw(ws), bytes, stream_of(DY)) == ZMOE_OK)
-      return dW;
+    int splits = 0;
+    if (zmoe_dense_wgrad_splits(M, N, K, 256, &splits) == ZMOE_OK) {
+      Tensor dW = empty({N, K}, DY, wgrad_dtype(DY, out_f32));
+      const size_t bytes = zmoe_dense_wgrad_workspace_bytes(N, K, DY.scalar_type() == at::kBFloat16 ? splits : 0);
+      Tensor ws = workspace(bytes, DY);
+      if (zmoe_dense_wgrad(raw(DY), DY.stride(0), raw(X), X.stride(0), M, N, K, code(DY), code(dW), splits, raw(dW),
+                           raw(ws), bytes, stream_of(DY)) == ZMOE_OK)
+        return dW;
+    }
   }
   static const auto op = general<Tensor(const Tensor&, const Tensor&, bool)>("zmoe::dense_wgrad");
   return op.call(DY, X, out_f32);

@@ -52,6 +52,7 @@ SIGNATURES = {
     "zmoe_group_bwd_w": (I32, [P, I64, P, I64, P, I32, P, I64, I64, I64, I32, I32, I32, P, P, P]),
     "zmoe_group_bwd_w_gather_dy": (I32, [P, I64, P, I32, P, I64, P, I64, I64, I64, I32, I32, I32, P, P]),
     "zmoe_dense_wgrad_workspace_bytes": (SZ, [I64, I64, I32]),
+    "zmoe_dense_wgrad_splits": (I32, [I64, I64, I64, I32, P]),
     "zmoe_dense_wgrad": (I32, [P, I64, P, I64, I64, I64, I64, I32, I32, I32, P, P, SZ, P]),
     "zmoe_rowwise_sum_product": (I32, [P, I32, P, I32, I64, I32, I64, P, I32, P]),
     "zmoe_glu_w1_forward": (I32, [P, I64, P, P, P, P, I64, I64, I64, I32, I32, I32, P, P, P]),

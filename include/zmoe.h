@@ -200,9 +200,12 @@ int zmoe_group_bwd_w_gather_dy(const void* DY, int64_t dy_stride_m,
  * split into `splits` ranges computed by the grouped wgrad kernel into fp32
  * partials, then summed in a fixed order and rounded once (deterministic).
  * workspace: zmoe_dense_wgrad_workspace_bytes(N, K, splits) bytes, 16-byte
- * aligned (0 for sizes dense_wgrad rejects: N or K >= 2^30, splits > 64). fp32 runs unsplit. out_dtype: `dtype`, or F32 for BF16 operands
- * (the fp32 sum written unrounded: fp32 master weights under bf16 autocast).
+ * aligned (0 for sizes dense_wgrad rejects: N or K >= 2^30, splits > 64). fp32 runs unsplit.
+ * out_dtype: `dtype`, or F32 for BF16 operands (the fp32 sum written unrounded: fp32 master
+ * weights under bf16 autocast). zmoe_dense_wgrad_splits stores the split count to use on `cus`
+ * compute units (256) into *splits; a host function.
  * ------------------------------------------------------------------------- */
+int zmoe_dense_wgrad_splits(int64_t M, int64_t N, int64_t K, int cus, int* splits);
 size_t zmoe_dense_wgrad_workspace_bytes(int64_t N, int64_t K, int splits);
 int zmoe_dense_wgrad(const void* DY, int64_t dy_stride_m, const void* X,
                      int64_t x_stride_m, int64_t M, int64_t N, int64_t K,

@@ -116,6 +116,30 @@ def test_dense_wgrad_workspace_holds_every_split_offset():
     assert rc == 2
 
 
+def test_dense_wgrad_splits_is_one_rule():
+    """The library's split count (what both forms of the dense weight grad use) is the least cost of
+    its model, the smaller count on ties, and sizes that dense_wgrad rejects are refused."""
+    from zmoe import _lib, ops
+
+    lib = _lib.load()
+
+    def cost(M, N, K, cus, s):
+        tile = 256 if min(M, N, K) >= 256 else 128
+        tiles = -(-N // tile) * -(-K // tile)
+        return -(-tiles * s // cus) * (-(-M // (64 * s)) * 1.6 + 11.0) + (0.0 if s == 1 else 2.0 * s * N * K * 4 / 5.0e6)
+
+    got = ctypes.c_int(0)
+    for M in (0, 1, 1023, 2047, 2048, 3000, 8190, 16383, 32768, 65536, 1 << 20):
+        for N, K in ((8, 256), (640, 512), (2048, 2176), (3072, 2048), (7168, 2048), (255, 4096), (16384, 16384)):
+            for cus in (256, 304):
+                want = min((s for s in range(1, 65) if s == 1 or M // s >= 1024), key=lambda s: cost(M, N, K, cus, s))
+                assert lib.zmoe_dense_wgrad_splits(M, N, K, cus, ctypes.byref(got)) == 0 and got.value == want
+                assert ops.dense_wgrad_splits(M, N, K, cus) == want
+    for bad in ((-1, 8, 8, 256), (1 << 31, 8, 8, 256), (8, 1 << 30, 8, 256), (8, 8, 1 << 30, 256), (8, 8, 8, 0)):
+        assert lib.zmoe_dense_wgrad_splits(*bad, ctypes.byref(got)) == 2
+    assert lib.zmoe_dense_wgrad_splits(8, 8, 8, 256, None) == 1
+
+
 def test_newton_schulz_workspace_is_sized_for_one_pass():
     """Stacks of any length run in passes of at most 1024 matrices spanning under 2 GiB,
     so the workspace of a long stack equals that of one full pass."""
