@@ -2806,7 +2806,9 @@ inline bool fewer_rounds_128(int64_t tiles256, int64_t tiles128) {
   return 20 * cdiv(tiles128, 512) < 29 * cdiv(tiles256, 256);
 }
 enum RowsForm { ROWS_128x128, ROWS_64x128, ROWS_128x256, ROWS_256x256 };
-inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t nt256, int64_t nt128, bool b_kn) {
+// (cols: the launch's output columns, or its pairs for SwiGLU, whose N is twice those)
+inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t cols, bool swiglu, bool b_kn) {
+  const int64_t nt256 = cdiv(cols, swiglu ? 128 : 256), nt128 = cdiv(cols, swiglu ? 64 : 128);
   if (R >= (int64_t)E * 256 && N >= 256) {
     return fewer_rounds_128(rows_tiles(R, E, 256) * nt256, rows_tiles(R, E, 128) * nt128) ? ROWS_128x128
                                                                                           : ROWS_256x256;
@@ -2829,10 +2831,9 @@ int dispatch_rows(int dtype, RowsParams p, int64_t R, int bn_for_tiles_div, hipS
     // contiguous the n-tiles are, so the tiles sharing B columns run together (measured
     // at C3: W2 forward 3%, W1 input grad 2% faster; n-major W1 forward 1% slower)
     p.n_major = p.a_rows == nullptr ? 1 : 0;
-    const int64_t nt256 = cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 128 : 256);
-    const int64_t nt128 = cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? 64 : 128);
-    const RowsForm form = rows_form(R, p.E, p.N, p.K, nt256, nt128, B_KN);
-    p.n_tiles = (int)(form == ROWS_256x256 || form == ROWS_128x256 ? nt256 : nt128);
+    const RowsForm form = rows_form(R, p.E, p.N, p.K, bn_for_tiles_div, EPI == EPI_SWIGLU, B_KN);
+    const int bn = form == ROWS_256x256 || form == ROWS_128x256 ? 256 : 128;
+    p.n_tiles = (int)cdiv(bn_for_tiles_div, EPI == EPI_SWIGLU ? bn / 2 : bn);
     switch (form) {
       case ROWS_256x256: return launch_rows_bf16<256, 256, B_KN, EPI>(p, R, s);
       case ROWS_128x256: return launch_rows_bf16<128, 256, B_KN, EPI>(p, R, s);
@@ -2917,6 +2918,20 @@ bool ok_rows(int dtype, const void* ptr, int64_t ld) {
 }
 
 }  // namespace
+
+extern "C" int zmoe_rows_gemm_tile(int64_t R, int64_t N, int64_t K, int E, int swiglu, int w_kn, int* bm, int* bn) {
+  ZMOE_REQUIRE(R >= 0 && R < kMaxRows && N >= 1 && K >= 1 && N < (1 << 30) && K < (1 << 30) && E >= 1 &&
+                   E <= kGemmMaxE,
+               ZMOE_ERR_SHAPE, "rows_gemm_tile: bad sizes (R=%lld N=%lld K=%lld E=%d)", (long long)R, (long long)N,
+               (long long)K, E);
+  ZMOE_REQUIRE(bm && bn, ZMOE_ERR_NULL, "rows_gemm_tile: null pointer");
+  *bm = *bn = 0;
+  if (!w_kn && use_stream(R, E, K)) return ZMOE_OK;
+  const RowsForm form = rows_form(R, E, N, K, swiglu ? N / 2 : N, swiglu != 0, w_kn != 0);
+  *bm = form == ROWS_64x128 ? 64 : (form == ROWS_256x256 ? 256 : 128);
+  *bn = form == ROWS_256x256 || form == ROWS_128x256 ? 256 : 128;
+  return ZMOE_OK;
+}
 
 extern "C" int zmoe_scatter2scatter(const void* X, int64_t x_stride_m, const void* W, int64_t w_stride_e,
                                     int64_t w_stride_k, int64_t w_stride_n, const void* b, int64_t b_stride_e,

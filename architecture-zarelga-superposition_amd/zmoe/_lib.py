@@ -47,6 +47,7 @@ SIGNATURES = {
     "zmoe_flatten_sort_count_noalloc": (I32, [P, I64, I32, P, P, P, P, P, P]),
     "zmoe_offsets_from_sorted": (I32, [P, I64, I32, P, P]),
     "zmoe_group": (I32, [P, I64, I64, I32, P, I64, I32, P, I32, P, I64, P]),
+    "zmoe_rows_gemm_tile": (I32, [I64, I64, I64, I32, I32, I32, P, P]),
     "zmoe_scatter2scatter": (I32, [P, I64, P, I64, I64, I64, P, I64, P, P, P, I64, I64, I64, I32, I32, I32, I32,
                                    I32, P, I64, P]),
     "zmoe_group_bwd_w": (I32, [P, I64, P, I64, P, I32, P, I64, I64, I64, I32, I32, I32, P, P, P]),

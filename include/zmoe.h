@@ -163,6 +163,11 @@ int zmoe_scatter2scatter(const void* X, int64_t x_stride_m, const void* W,
                          int64_t N, int E, int k, int x_grouped, int y_grouped,
                          int dtype, void* Y, int64_t y_stride_m, void* stream);
 
+/* The rows x columns of a tile of the bf16 launch for R sorted rows, N columns (the SwiGLU forward: 2f)
+ * and depth K; w_kn: W has unit stride along N (the input grads'). 0 x 0: the weight-streaming kernel
+ * (no bias). A host function: nothing is launched. */
+int zmoe_rows_gemm_tile(int64_t R, int64_t N, int64_t K, int E, int swiglu, int w_kn, int* bm, int* bn);
+
 /* ---------------------------------------------------------------------------
  * group_bwd_W — scattermoe/kernels/ops.py:263-438 (grouped weight gradient):
  *   DWt[e, n, c] = sum_{i in expert e} DY[i, n] * Xrow(i)[c]

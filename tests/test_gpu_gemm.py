@@ -429,13 +429,16 @@ def test_glu_act_forward(hip_device, dtype, T, d, f, E, k):
             ops.glu_act_forward(x, W1, ss, off, k, rs)
 
 
-@pytest.mark.parametrize("T", [700, 40])
+@pytest.mark.parametrize("T", [700, 40, 32])   # 32: the small-batch route
 def test_layer_without_graph_matches(hip_device, T):
-    """The layer and the GLU experts under no_grad (no pre-activations kept) give bit for bit
-    what they give when they record a graph, and a graph is recorded when one input needs it."""
+    """The layer and the GLU experts under no_grad (no pre-activations kept by the grouped launches)
+    give bit for bit what they give when they record a graph, and a graph is recorded when one input
+    needs it."""
     from modeling.model_config import ModelConfig
     from modeling.moe_layer import MoELayer
+    from zmoe import ops
 
+    assert ops.glu_stream_shared_ok(T, 128, 64, 64, 16, 4) == (T == 32)
     torch.manual_seed(T)
     cfg = ModelConfig(hidden_size=128, intermediate_size=64, n_experts=17, n_shared_experts=1, n_experts_per_token=4)
     layer = MoELayer(cfg).to(hip_device).to(torch.bfloat16)
@@ -623,12 +626,12 @@ def test_f32_tile_sizes(hip_device, d, f):
 
 
 # (rows per expert, N, f): each tile size of the bf16 rows launches at its own row counts, K of 1, 2
-# and 4 stages (the 3-stage rings' edges)
+# and 4 stages (the 3-stage rings' edges); test_rows_tile_forms asserts every launch's tile
 _FORM_COUNTS = {
     "64x128": (np.array([0, 1, 17, 63, 64, 65, 127, 128, 129, 0, 5, 8]), 264, 200),       # <= 52 rows on average
-    "128x256": (np.array([0, 1, 63, 64, 65, 127, 128, 129, 257, 60, 40, 30] * 8), 1000, 504),  # 52-112, >= 384 pairs
-    "256x256 few rows": (np.array([0, 3, 64, 65, 128, 129, 255, 256, 257, 190, 120, 100] * 8), 1000, 504),
-    "256x256": (SMALL_TILE_COUNTS, 1928, 960),  # one round of 256 x 256, two of 128 x 128
+    "128x256": (np.array([0, 1, 63, 64, 65, 127, 128, 129, 257, 60, 40, 30] * 8), 1000, 1000),  # 52-112, >= 384 pairs
+    "256x256 few rows": (np.array([0, 3, 64, 65, 128, 129, 255, 256, 257, 190, 120, 100] * 8), 1000, 1000),
+    "256x256": (SMALL_TILE_COUNTS, 1928, 1928),  # one round (SwiGLU: two) of 256 x 256, two (three) of 128 x 128
 }
 
 
@@ -637,7 +640,9 @@ _FORM_COUNTS = {
 def test_rows_tile_forms(hip_device, form, K):
     """bf16 rows launches at sizes that the dispatch sends to each tile size: both weight layouts,
     gathered and grouped A, scattered output, bias, the (scaled) SwiGLU forward and its backward."""
-    from zmoe import ops
+    import ctypes
+
+    from zmoe import _lib, ops
 
     counts, N, f = _FORM_COUNTS[form]
     k, dt = 2, torch.bfloat16
@@ -645,6 +650,10 @@ def test_rows_tile_forms(hip_device, form, K):
         counts = counts.copy()
         counts[-1] += 1
     E, R = len(counts), int(counts.sum())
+    for cols, swiglu, kn in ((N, 0, 0), (N, 0, 1), (2 * f, 1, 0), (f, 0, 1)):
+        bm, bn = ctypes.c_int(-1), ctypes.c_int(-1)
+        assert _lib.load().zmoe_rows_gemm_tile(R, cols, K, E, swiglu, kn, ctypes.byref(bm), ctypes.byref(bn)) == 0
+        assert f"{bm.value}x{bn.value}" == form.split()[0], (cols, swiglu, kn)
     se, ss, off = _fixed_routing(counts, k, hip_device, seed=23)
     sn, en = ss.cpu().numpy(), se.cpu().numpy()
     g = gen(R + N + K)
