@@ -5,7 +5,7 @@ route owes its callers."""
 import pytest
 import torch
 
-from helpers import gen
+from helpers import assert_close, gen, np64
 
 pytestmark = pytest.mark.gpu
 
@@ -45,6 +45,45 @@ def _equal(a, b):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
     for n in a[2]:
         assert torch.equal(a[2][n], b[2][n]), n
+
+
+@pytest.mark.parametrize("T,n_shared", [(1, 1), (16, 1), (33, 2), (128, 2)])   # one to four groups of 32 tokens
+def test_layer_against_oracle(hip_device, T, n_shared):
+    """Forward and backward on the streaming route (bf16), every grad."""
+    from test_gpu_layer import run_and_compare
+
+    d, E, k, f = 128, 64, 4, 64
+    assert _streams(T, d, f, n_shared * f, E, k)
+    run_and_compare(T, d, E, k, f, n_shared, torch.bfloat16, hip_device)
+
+
+@pytest.mark.parametrize("pad", [False, True])
+@pytest.mark.parametrize("T", [16, 33])
+def test_fp32_masters_match_bf16_layer(hip_device, T, pad):
+    """fp32 weights and input under bf16 autocast on the streaming route, with and without unpad
+    indices: the bf16 layer's output bit for bit, its input grad's fp32 sum, and fp32 weight grads
+    that round to its own but for rare accumulation flips (the bf16 layer itself: the oracle, above)."""
+    l32, l16 = _layer(hip_device, torch.float32), _layer(hip_device, torch.float32)
+    l16.load_state_dict(l32.state_dict())
+    bias = l32.gate.expert_biases.data.clone()
+    l16 = l16.to(torch.bfloat16)
+    l16.gate.expert_biases.data = bias
+    kw, n = {}, T
+    if pad:
+        kw["unpad_indices"] = torch.tensor([i for i in range(T) if i % 5 != 2], device=hip_device)
+        n = kw["unpad_indices"].numel()
+    assert _streams(n, 128, 64, 64, 64, 4)
+    x = torch.randn(1, T, 128, generator=gen(6)).to(torch.bfloat16).to(hip_device)
+    dout = torch.randn(1, T, 128, generator=gen(7)).to(torch.bfloat16).to(hip_device)
+    o32, dx32, g32 = _step(l32, x.float(), dout, autocast=True, **kw)
+    o16, dx16, g16 = _step(l16, x, dout, **kw)
+    assert torch.equal(o32, o16)
+    assert dx32.dtype == torch.float32 and torch.equal(dx32.to(torch.bfloat16), dx16)
+    for name, g in g32.items():
+        r = g.to(torch.bfloat16)
+        assert g.dtype == torch.float32 and g16[name].abs().sum() > 0, name
+        assert (r == g16[name]).float().mean().item() >= 0.99, name
+        assert_close(np64(r), np64(g16[name]), rtol=2 ** -7, atol=1e-6, what=name)
 
 
 def test_weights_edited_between_forward_and_backward(hip_device):
