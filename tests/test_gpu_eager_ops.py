@@ -1,7 +1,10 @@
 """The native dispatcher kernels of the layer's ops (csrc/eager_ops.cpp, zmoe_eager::) against the
 ops' general form (zmoe::, the Python wrappers): the same bits for the operands the layer passes,
 for strided rows, other index and gate dtypes and widths that need padding, the same errors, and
-the general form where a backward through the op has to be refused."""
+the general form where a backward through the op has to be refused. That an op runs natively is shown
+by taking the general form's functions away."""
+
+import threading
 
 import pytest
 import torch
@@ -82,9 +85,21 @@ def _same(a, b):
         assert torch.equal(u, v)
 
 
+def _no_general_form(monkeypatch):
+    """Every function that the general forms are made of fails."""
+    from zmoe import ops as zops
+
+    def gone(*args, **kwargs):
+        raise AssertionError("the general form ran")
+
+    for n, v in list(vars(zops).items()):
+        if callable(v) and getattr(v, "__module__", None) == zops.__name__:
+            monkeypatch.setattr(zops, n, gone)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("d,f", [(D, F), (D + 3, F + 1)])
-def test_native_op_equals_general(hip_device, dtype, d, f):
+def test_native_op_equals_general(hip_device, dtype, d, f, monkeypatch):
     from zmoe import library as zl
 
     for key, args in _ops(hip_device, dtype, d, f).items():
@@ -96,7 +111,8 @@ def test_native_op_equals_general(hip_device, dtype, d, f):
             with pytest.raises(ValueError), torch.no_grad():
                 native(*args)
             continue
-        with torch.no_grad():
+        with torch.no_grad(), monkeypatch.context() as m:
+            _no_general_form(m)
             _same(native(*args), ref)
 
 
@@ -129,6 +145,75 @@ def test_native_op_conversions_and_refusals(hip_device):
     leaf = Y.clone().requires_grad_(True)
     with pytest.raises(RuntimeError):   # no formula: refused, not silently dropped
         zl.sum_k(leaf, k, None, False).sum().backward()
+
+
+def _off(t, by=1):
+    """A copy of ``t`` that starts ``by`` elements into a buffer."""
+    buf = torch.empty(t.numel() + by, dtype=t.dtype, device=t.device)
+    view = buf[by:].view(t.shape)
+    view.copy_(t)
+    return view
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_native_op_operands_off_16_bytes(hip_device, dtype, monkeypatch):
+    """Rows have to start on 16 bytes in both forms; per-row floats, a norm's weight and the router's
+    logits need not, natively."""
+    from zmoe import library as zl
+
+    ops = _ops(hip_device, dtype, D, F)
+    for key in ("swiglu", "swiglu_backward", "swiglu_backward_gates", "combine", "sum_k", "rmsnorm_rows",
+                "glu_w1_forward", "grouped_mm", "group_bwd_w", "dense_wgrad", "cast_bf16"):
+        if key in ops:
+            args = (_off(ops[key][0]), *ops[key][1:])
+            for form in (getattr(zl, key), getattr(torch.ops.zmoe, key)):
+                with pytest.raises(ValueError), torch.no_grad():
+                    form(*args)
+    for key, at in (("route_topk", 0), ("combine", 1), ("swiglu_backward_gates", 2), ("flatten_sort_count_weights", 1),
+                    ("rmsnorm_rows", 1), ("rmsnorm_rows_backward", 4), ("rmsnorm_rows_backward", 3)):
+        args = ops[key]
+        ref = getattr(torch.ops.zmoe, key)(*args)
+        with torch.no_grad(), monkeypatch.context() as m:
+            _no_general_form(m)
+            _same(getattr(zl, key)(*args[:at], _off(args[at]), *args[at + 1:]), ref)
+
+
+def test_native_ops_on_streams_and_threads(hip_device):
+    """An op runs on the caller's current stream, after what is queued there, also from several
+    threads at once."""
+    from zmoe import library as zl
+
+    cases = []
+    for key, args in _ops(hip_device, torch.bfloat16, D, F).items():
+        cases.append((key, getattr(zl, _name(key)), args, getattr(torch.ops.zmoe, _name(key))(*args)))
+    torch.cuda.synchronize()
+    failed = []
+
+    def work():
+        stream = torch.cuda.Stream()
+        try:
+            with torch.no_grad(), torch.cuda.stream(stream):
+                for key, native, args, ref in cases:
+                    # the floating operands arrive late, on this stream
+                    late = [torch.zeros_like(a) if isinstance(a, torch.Tensor) and a.is_floating_point() else a
+                            for a in args]
+                    torch.cuda._sleep(2_000_000)
+                    for a, b in zip(late, args):
+                        if a is not b:
+                            a.copy_(b)
+                    got = native(*late)
+                    stream.synchronize()
+                    _same(got, ref)
+        except Exception as e:  # reported by the main thread
+            failed.append((key, e))
+
+    work()
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
 
 
 def test_native_mutating_ops(hip_device):
