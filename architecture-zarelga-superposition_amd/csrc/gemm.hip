@@ -2801,7 +2801,12 @@ inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
 //  * From 256 rows on, whichever needs less time in whole rounds over the CUs (one 256 x 256 or two
 //    128 x 128 workgroups each, a round of the former 1.45x the latter's): d = 512, E = 32, f = 160,
 //    410 rows: W1 21 / 17 on 128 x 128; d = 2048, E = 32, f = 768: dA 93 / 73 at 600 rows, but
-//    51 / 65 at 410; from a few rounds on 256 x 256, whose loads have twice the reuse.
+//    51 / 65 at 410; from a few rounds on 256 x 256, whose loads have twice the reuse. The rows per expert
+//    are not known here, and an even routing and a skewed one (half a partial tile per expert) can come
+//    to different rounds, so 128 x 128 has to win under both (420 rows, E = 64, d = 1024, f = 512: even 2
+//    rounds of 256 x 256, the estimate 3: W1 88 / 68 on 256 x 256 with an even routing, dA 44 / 54 under
+//    a Zipf(1.1) skew; over 300 launches of K = 256 to 2048 at 300-2048 rows the two together are never
+//    slower than 256 x 256 alone, the estimate alone up to 1.37x).
 inline bool fewer_rounds_128(int64_t tiles256, int64_t tiles128) {
   return 20 * cdiv(tiles128, 512) < 29 * cdiv(tiles256, 256);
 }
@@ -2810,8 +2815,10 @@ enum RowsForm { ROWS_128x128, ROWS_64x128, ROWS_128x256, ROWS_256x256 };
 inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t cols, bool swiglu, bool b_kn) {
   const int64_t nt256 = cdiv(cols, swiglu ? 128 : 256), nt128 = cdiv(cols, swiglu ? 64 : 128);
   if (R >= (int64_t)E * 256 && N >= 256) {
-    return fewer_rounds_128(rows_tiles(R, E, 256) * nt256, rows_tiles(R, E, 128) * nt128) ? ROWS_128x128
-                                                                                          : ROWS_256x256;
+    const int64_t mean = cdiv(R, E);
+    const bool few = fewer_rounds_128(rows_tiles(R, E, 256) * nt256, rows_tiles(R, E, 128) * nt128) &&
+                     fewer_rounds_128(E * cdiv(mean, 256) * nt256, E * cdiv(mean, 128) * nt128);
+    return few ? ROWS_128x128 : ROWS_256x256;
   }
   const bool many = N >= 256 && E * nt256 >= 384;
   if (many && R >= (int64_t)E * 112) return ROWS_256x256;

@@ -140,6 +140,30 @@ def test_dense_wgrad_splits_is_one_rule():
     assert lib.zmoe_dense_wgrad_splits(8, 8, 8, 256, None) == 1
 
 
+def _rows_tile(rows, N, K, E, swiglu=0, w_kn=0):
+    from zmoe import _lib
+
+    bm, bn = ctypes.c_int(-1), ctypes.c_int(-1)
+    assert _lib.load().zmoe_rows_gemm_tile(rows * E, N, K, E, swiglu, w_kn, ctypes.byref(bm), ctypes.byref(bn)) == 0
+    return bm.value, bn.value
+
+
+def test_rows_tile_from_256_rows():
+    """128 x 128 tiles only where they take fewer rounds over the CUs under an even routing too: at 420
+    rows an expert has two 256-row tiles, which the estimate with half a partial tile each puts at more
+    than 2.1 (measured with even experts, us, 128 x 128 / 256 x 256, at each size)."""
+    for N, K, E, swiglu, kn in ((1024, 1024, 64, 1, 0),    # 88 / 68
+                                (1024, 512, 64, 0, 0),     # 55 / 45
+                                (512, 1024, 64, 0, 1),     # 45 / 35
+                                (1024, 2048, 64, 0, 1),    # 157 / 115
+                                (2048, 1024, 32, 1, 0)):   # 89 / 68
+        assert _rows_tile(420, N, K, E, swiglu, kn) == (256, 256), (N, K, E)
+    assert _rows_tile(410, 320, 512, 32, 1) == (128, 128)           # 17 / 21
+    assert _rows_tile(600, 768, 2048, 32, 0, 1) == (128, 128)       # 73 / 93
+    assert _rows_tile(410, 768, 2048, 32, 0, 1) == (256, 256)       # 65 / 51
+    assert _rows_tile(2048, 1536, 2048, 128, 1) == (256, 256)
+
+
 def test_newton_schulz_workspace_is_sized_for_one_pass():
     """Stacks of any length run in passes of at most 1024 matrices spanning under 2 GiB,
     so the workspace of a long stack equals that of one full pass."""
