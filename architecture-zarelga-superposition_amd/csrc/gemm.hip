@@ -2797,7 +2797,9 @@ inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
 //    but at 96: 222 / 210). Between the two, 128 x 256 ring tiles (d = 7168, 96 rows: W1 682 / 742
 //    on 128 x 128, W1 input grad 686 / 752). Both need enough tiles: d = 1024, E = 64 has 256
 //    (expert, 256-column) pairs for W1, and under a Zipf(1.1) skew at 126 rows 256 x 256 takes 61,
-//    128 x 128 49.
+//    128 x 128 49. From 384 pairs 128 x 256, from 512 (two rounds) 256 x 256: E = 128, N = 768 (384),
+//    128 x 128 / 128 x 256 / 256 x 256: the SwiGLU backward 127 / 118 / 149 at 120 even rows, 165 / 161 /
+//    202 at 180 skewed ones, dA 103 / 92 / 118 and 136 / 131 / 148 (but 129 / 130 / 101 at 120 skewed).
 //  * From 256 rows on, whichever needs less time in whole rounds over the CUs (one 256 x 256 or two
 //    128 x 128 workgroups each, a round of the former 1.45x the latter's): d = 512, E = 32, f = 160,
 //    410 rows: W1 21 / 17 on 128 x 128; d = 2048, E = 32, f = 768: dA 93 / 73 at 600 rows, but
@@ -2820,10 +2822,10 @@ inline RowsForm rows_form(int64_t R, int E, int64_t N, int64_t K, int64_t cols, 
                      fewer_rounds_128(E * cdiv(mean, 256) * nt256, E * cdiv(mean, 128) * nt128);
     return few ? ROWS_128x128 : ROWS_256x256;
   }
-  const bool many = N >= 256 && E * nt256 >= 384;
-  if (many && R >= (int64_t)E * 112) return ROWS_256x256;
+  const int64_t pairs = N >= 256 ? E * nt256 : 0;
+  if (pairs >= 512 && R >= (int64_t)E * 112) return ROWS_256x256;
   if (R <= (int64_t)E * 52 && !(b_kn && K > 2048)) return ROWS_64x128;
-  return many ? ROWS_128x256 : ROWS_128x128;
+  return pairs >= 384 ? ROWS_128x256 : ROWS_128x128;
 }
 
 template <bool B_KN, int EPI>

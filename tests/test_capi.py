@@ -164,6 +164,17 @@ def test_rows_tile_from_256_rows():
     assert _rows_tile(2048, 1536, 2048, 128, 1) == (256, 256)
 
 
+def test_rows_tile_below_256_rows():
+    """256 x 256 tiles of one per expert need two rounds' worth of (expert, 256-column) pairs; a round
+    and a half is better off on 128 x 256 tiles."""
+    for rows in (120, 180, 250):
+        assert _rows_tile(rows, 768, 2048, 128, 0, 1) == (128, 256)     # 384 pairs
+        assert _rows_tile(rows, 1024, 2048, 128, 0, 1) == (256, 256)    # 512
+        assert _rows_tile(rows, 512, 2048, 128, 0, 1) == (128, 128)     # 256
+        assert _rows_tile(rows, 1536, 2048, 128, 1, 0) == (256, 256)    # 768 pair-column tiles
+    assert _rows_tile(100, 1024, 2048, 128, 0, 1) == (128, 256)
+
+
 def test_newton_schulz_workspace_is_sized_for_one_pass():
     """Stacks of any length run in passes of at most 1024 matrices spanning under 2 GiB,
     so the workspace of a long stack equals that of one full pass."""
