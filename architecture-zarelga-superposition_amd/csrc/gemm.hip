@@ -13,17 +13,20 @@
 //     wgrad_bf16_kernel / grouped_wgrad_kernel), x rows optionally gathered.
 //
 // bf16 tile machinery (BM x BN = 256 x 256 on 8 waves in a 2x4 grid, two waves per
-// SIMD and 128 x 64 outputs per wave; or 128 x 128 on 4 waves in a 2x2 grid):
+// SIMD and 128 x 64 outputs per wave; 128 x 128 on 4 waves in a 2x2 grid; for rows launches of few
+// rows per expert also 128 x 256 on 8 waves and 64 x 128 on 4, see rows_form):
 //   * Operands go HBM -> LDS with buffer_load_dwordx4 ... lds (no VGPR staging) in
-//     64-deep stages, double-buffered (a rows tile of at most 64 rows: three stages of its
+//     64-deep stages, double-buffered (128 x 256 and 64 x 128 tiles: a ring of three stages,
+//     kloop_ring; a 256 x 256 rows tile of at most 64 rows: three stages of its
 //     64 rows and the weight block, kloop_small), every wave loading its own share: 128-byte
 //     rows with the reduction dimension contiguous (16-byte chunks XOR-swizzled by
 //     row so that each 8- or 16-lane group of a fragment read hits distinct banks), or K-major tiles read with
 //     ds_read_b64_tr_b16 for operands whose reduction dimension is strided. Each
 //     stage has its own scalar buffer descriptor (the k advance and the tail
 //     clipping), so issuing a load costs no vector ALU.
-//   * v_mfma_f32_16x16x32_bf16 on 8 waves (kloop64_m16; the SwiGLU-backward epilogue,
-//     4-wave tiles, the DY-gathered weight grads and the weight grads with the few-rows form
+//   * v_mfma_f32_16x16x32_bf16 on 8 waves and in the ring loops (kloop64_m16, kloop_ring; the
+//     SwiGLU-backward epilogue on 256 x 256 tiles, 128 x 128 tiles, the DY-gathered weight grads and
+//     the weight grads with the few-rows form
 //     inline keep v_mfma_f32_32x32x16_bf16, kloop64), with the B tile as the first operand: each
 //     lane ends up holding 4 consecutive output columns of one output row. Every MFMA
 //     slot of the K loop is pinned with sched_barrier so loads, fragment reads and the
@@ -1888,8 +1891,9 @@ struct WaveGrid {
   __device__ __forceinline__ static int wn0(int wave) { return (wave % GN) * WN; }
 };
 
-// LDS of the bf16 kernels: two operand stages (three short ones in kloop_small), reused by
-// the wave staging areas after the K loop, then the rows kernel's output-row table.
+// LDS of the bf16 kernels: two operand stages (three in the ring loops, 144 KB at 128 x 256, so one
+// workgroup per CU; three short ones in kloop_small), reused by the wave staging areas after the K loop,
+// then the rows kernel's output-row table.
 template <int BM, int BN, int NW = 4>
 constexpr int bf16_stage_bytes() {
   constexpr int loop = (ring_stages(BM, BN, NW) > 0 ? ring_stages(BM, BN, NW) : 2) * (BM + BN) * 64 * 2;
@@ -1992,9 +1996,9 @@ __global__ __launch_bounds__(NW * 64, (NW == 4 && ring_stages(BM, BN, NW) > 0 ? 
 
   const int wave = threadIdx.x >> 6;
   const int wm0 = WG::wm0(wave), wn0 = WG::wn0(wave);
-  // 8 waves run the 16 x 16 x 32 K loop (kloop64_m16; the C3 step 2.8% faster than on 32 x 32 x 16
-  // MFMAs, the Newton-Schulz pass 2.5%), except with the SwiGLU-backward epilogue, which has no
-  // registers left for its extra fragments
+  // The ring loops and 8 waves run 16 x 16 x 32 MFMAs (kloop64_m16: the C3 step 2.8% faster than on 32 x
+  // 32 x 16, the Newton-Schulz pass 2.5%), except 256 x 256 tiles with the SwiGLU-backward epilogue, whose
+  // 128 accumulators a lane leave no registers for the extra fragments (a 128 x 256 tile has 64)
   constexpr int RING = ring_stages(BM, BN, NW);
   constexpr bool M16 = RING > 0 || (EPI != EPI_SWIGLU_BWD && NW == 8);
   using Acc = typename std::conditional<M16, f32x4_t[4], f32x16_t>::type;
@@ -2541,9 +2545,6 @@ int launch_wgrad_big(const WgradParams& p, hipStream_t s) {
                              bf16_lds_bytes<256, 256, NW>(), 256, 256, p, s, NW * 64);
 }
 
-// Large tiles when the average expert holds enough rows to fill them.
-inline bool use_big_tiles(int64_t R, int E, int64_t N) { return R >= (int64_t)E * 256 && N >= 256; }
-
 // Weight grads under a skewed routing (fewer than 1024 rows per expert on average): the
 // experts holding at most kFewRows rows take the write-bound few-rows form. With X's rows
 // gathered (dW1) it runs inside the 256 x 256 K-loop launch: one launch over every expert,
@@ -2596,7 +2597,8 @@ struct StreamShared {
 };
 
 template <int EPI, int KSPLIT>
-__global__ __launch_bounds__(256, (KSPLIT > 1 ? 4 : 1)) void stream_rows_kernel(RowsParams p, StreamShared sh, int wtiles_per_e) {
+__global__ __launch_bounds__(256, (KSPLIT > 1 ? 4 : 1)) void stream_rows_kernel(RowsParams p, StreamShared sh,
+                                                                               int wtiles_per_e) {
   __shared__ f32x4_t red[KSPLIT > 1 ? 3 : 1][4][64];
   const int lane = (int)(threadIdx.x & 63), wave = (int)(threadIdx.x >> 6);
   const int tpb = KSPLIT == 1 ? 4 : 1;  // tiles per block
@@ -2786,7 +2788,11 @@ constexpr int64_t kF32SmallTiles = 448;
 inline bool f32_small_tiles(int64_t tiles) { return tiles < kF32SmallTiles; }
 
 // Tile size of a bf16 rows launch from its rows per expert (R / E on average) and its column
-// tiles of 256 and of 128 (nt256, nt128 per expert). All figures in us.
+// tiles of 256 and of 128 (nt256, nt128 per expert). All figures in us. The rows of each expert are
+// known on the device only, so the rule is for an even routing and a Zipf skew of up to about 1.1, where
+// over 700 launches below 256 rows it takes 0.94 of 128 x 128 tiles' time (single ones up to 1.2 of it: d =
+// 1024, E = 64, 16 skewed rows, W1 30 / 25). Where a few experts hold every row the small tiles lose
+// (d = 2048, E = 128, all rows on 8 experts, 30 per expert: W1 48 on 64 x 128, 35 on 128 x 128).
 //  * Up to 52 rows nearly every expert is one tile of 64, and the launch streams weights: 64 x 128
 //    ring tiles, two workgroups per CU, keep more of them in flight (E = 128, d = 2048, f = 768,
 //    against 128 x 128: at 32 rows W1 174 / 198, W2 86 / 96, dA 78 / 90; at 64 rows, where half the
@@ -3302,8 +3308,6 @@ extern "C" int zmoe_glu_w2_backward_dh_gates(const void* dout, int64_t T, int k,
 }
 
 namespace {
-// bf16 weight grads: 256 x 256 tiles when the experts are large enough, 128 x 128 otherwise,
-// and the small experts split off under a skewed routing. DYG: the gather is on DY's rows.
 // 256 x 256 weight-grad tiles (with the few-rows form for experts of at most 64 rows) rather than
 // 128 x 128. A tile's time is mostly its fixed cost (decode, first loads, output) unless its expert
 // has many rows, so the larger tile wins whenever the launch has several per CU, whatever the rows
@@ -3318,6 +3322,8 @@ inline bool use_big_wgrad(int64_t M, int E, int64_t N, int64_t K) {
   return N >= 256 && K >= 256 && (tiles >= 1024 || (M >= (int64_t)E * 256 && tiles > 128));
 }
 
+// bf16 weight grads: 256 x 256 or 128 x 128 tiles (use_big_wgrad), and the small experts split off
+// under a skewed routing. DYG: the gather is on DY's rows.
 template <bool DYG, bool OUT_F32 = false>
 int group_bwd_w_bf16(WgradParams p, int64_t M, int E, int64_t N, int64_t K, hipStream_t s) {
   const bool big = use_big_wgrad(M, E, N, K);
@@ -3564,7 +3570,7 @@ extern "C" int zmoe_dense_wgrad(const void* DY, int64_t dy_stride_m, const void*
   ZMOE_REQUIRE(dy_span <= kMaxSpan && x_span <= kMaxSpan, ZMOE_ERR_SHAPE, "dense_wgrad: DY or X spans more than 2 GiB");
   p.dy_bytes = (uint32_t)dy_span;
   p.x_bytes = (uint32_t)x_span;
-  if (use_big_tiles(M, S, N) && K >= 256)
+  if (M >= (int64_t)S * 256 && N >= 256 && K >= 256)  // enough rows per split to fill the larger tiles
     rc = launch_wgrad_big<0, true>(p, s);
   else
     rc = launch_wgrad_kernel(wgrad_bf16_kernel<128, 128, 0, true>, bf16_lds_bytes<128, 128>(), 128, 128, p, s);

@@ -52,10 +52,12 @@ class _FusedMoELayer(torch.autograd.Function):
     adds over [T, d]).
 
     (x [T, d], gate weight, expert_biases, W1, W2, shared gate/up/down weights, k, E,
-    pad_rows, pad_total, backward) -> (out, topk_idx [T, k], expert_offsets [E]); with backward
-    False (a call that records no graph) no pre-activations are kept; out is [T, d], or with pad_rows (int64 [T]) the padded [pad_total, d] whose row pad_rows[t] is token t's.
-    Every launch is a ``zmoe::`` custom op, so torch.compile traces through the function
-    without a graph break.
+    pad_rows, pad_total, backward) -> (out, topk_idx [T, k], expert_offsets [E]); out is [T, d],
+    or with pad_rows (int64 [T]) the padded [pad_total, d] whose row pad_rows[t] is token t's.
+    With backward False (a call that records no graph) the grouped W1 launch writes no
+    pre-activations and W3 is formed only where the launches read it; the streaming launches of a
+    small batch write theirs either way. Every launch is a ``zmoe::`` custom op, so torch.compile
+    traces through the function without a graph break.
 
     The weights and x may be fp32 (the reference's fp32 master weights and residual stream
     under bf16 autocast, main.py:595, :746): the function then computes on bf16 copies made
