@@ -50,7 +50,7 @@ def _load_eager():
 _plain = frozenset((torch.Tensor, torch.nn.Parameter, int, bool, float, str, list, tuple, type(None))).issuperset
 
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
-_tracing, _functorch = torch._C._get_tracing_state, torch._C._functorch.peek_interpreter_stack
+_tracing, _transforms = torch._C._is_tracing, torch._C._functorch.get_dynamic_layer_stack_depth
 _compiling, _grad_enabled, _forward_ad = torch.compiler.is_compiling, torch.is_grad_enabled, torch.autograd.forward_ad
 
 
@@ -73,8 +73,8 @@ class LayerOp(torch.library.CustomOpDef):
     one that zmoe.profiling times."""
 
     def __call__(self, *args, **kwargs):
-        if (_compiling() or _grad_enabled() or kwargs or _dispatch_modes() or _functorch() is not None
-                or _forward_ad._current_level >= 0 or _tracing() is not None or profiling.active()
+        if (_compiling() or _grad_enabled() or kwargs or _dispatch_modes() or _transforms()
+                or _forward_ad._current_level >= 0 or _tracing() or profiling.active()
                 or not _plain(map(type, args)) or (_function_modes() and _watched_by_function_mode())
                 or (self._lists and not all(_plain(map(type, args[i])) for i in self._lists if i < len(args)))):
             return super().__call__(*args, **kwargs)
