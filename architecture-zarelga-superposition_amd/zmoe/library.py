@@ -80,7 +80,8 @@ class LayerOp(torch.library.CustomOpDef):
             return super().__call__(*args, **kwargs)
         if self._native is None:
             _load_eager()
-            self._native = getattr(torch.ops.zmoe_eager, self._name).default
+            # (the dispatcher's call itself: the overload object's Python __call__ only forwards to it)
+            self._native = getattr(torch.ops.zmoe_eager, self._name).default._op
         out = self._native(*args)
         for i in self._mutated:  # as custom_op does: autograd sees that the tensor changed
             if i < len(args) and args[i] is not None:
