@@ -808,27 +808,27 @@ __global__ __launch_bounds__(kGemmThreads) void grouped_wgrad_kernel(WgradParams
 }
 
 // Db[e, n] = sum over the expert's rows of DY[i, n] (bias grad, off the GLU path). A block takes
-// one expert and 128 bytes of columns (8 16-byte chunks, whole lines); its 128 thread rows sum
-// every 128th row, then the sums are added in a fixed order (within a wave, then across the waves
-// through LDS). Bound by the latency of the row loads, so the rows of a slot are loaded four at a
+// one expert and CH 16-byte chunks of columns; its THREADS / CH thread rows sum
+// every THREADS / CH-th row, then the sums are added in a fixed order (within a wave, then across the
+// waves through LDS). Bound by the latency of the row loads, so the rows of a slot are loaded four at a
 // time. One thread per column over all of an expert's rows took 205 us for 8002 rows of 1032
 // columns in 16 experts (a serial chain of 2-byte loads); this takes 8.2 us, 4.9 at 512 columns.
-constexpr int kBiasThreads = 1024;
-template <typename T>
-__global__ __launch_bounds__(kBiasThreads) void bias_grad_kernel(const T* __restrict__ DY, int64_t lddy,
-                                                                 const int64_t* __restrict__ off, int N,
-                                                                 T* __restrict__ Db) {
+template <typename T, int THREADS, int CH>
+__global__ __launch_bounds__(THREADS) void bias_grad_kernel(const T* __restrict__ DY, int64_t lddy,
+                                                            const int64_t* __restrict__ off, int N,
+                                                            T* __restrict__ Db) {
   constexpr int VN = 16 / sizeof(T);
-  constexpr int SLOTS = kBiasThreads / 8, WAVES = kBiasThreads / 64, U = 4;
-  __shared__ float red[WAVES][8 * VN];
+  constexpr int SLOTS = THREADS / CH, WAVES = THREADS / 64, U = 4;
+  static_assert(CH <= 64 && CH * VN <= THREADS, "a wave holds whole chunk rows; a thread per output column");
+  __shared__ float red[WAVES][CH * VN];
   const int e = blockIdx.y;
-  const int col = ((int)blockIdx.x * 8 + (threadIdx.x & 7)) * VN;
+  const int col = ((int)blockIdx.x * CH + (int)(threadIdx.x % CH)) * VN;
   const int64_t a = e ? off[e - 1] : 0, b = off[e];
   float s[VN];
 #pragma unroll
   for (int u = 0; u < VN; ++u) s[u] = 0.f;
   if (col < N) {
-    for (int64_t i = a + (threadIdx.x >> 3); i < b; i += U * SLOTS) {
+    for (int64_t i = a + threadIdx.x / CH; i < b; i += U * SLOTS) {
       uint4 c[U];
 #pragma unroll
       for (int q = 0; q < U; ++q) {
@@ -847,18 +847,43 @@ __global__ __launch_bounds__(kBiasThreads) void bias_grad_kernel(const T* __rest
 #pragma unroll
   for (int u = 0; u < VN; ++u)
 #pragma unroll
-    for (int o = 8; o < 64; o <<= 1) s[u] += __shfl_xor(s[u], o, 64);
-  if ((threadIdx.x & 63) < 8)
+    for (int o = CH; o < 64; o <<= 1) s[u] += __shfl_xor(s[u], o, 64);
+  if ((threadIdx.x & 63) < CH)
 #pragma unroll
-    for (int u = 0; u < VN; ++u) red[threadIdx.x >> 6][(threadIdx.x & 7) * VN + u] = s[u];
+    for (int u = 0; u < VN; ++u) red[threadIdx.x >> 6][(threadIdx.x & 63) * VN + u] = s[u];
   __syncthreads();
-  if (threadIdx.x >= 8 * VN) return;
-  const int n = (int)blockIdx.x * 8 * VN + (int)threadIdx.x;
+  if (threadIdx.x >= CH * VN) return;
+  const int n = (int)blockIdx.x * CH * VN + (int)threadIdx.x;
   if (n >= N) return;
   float t = 0.f;
 #pragma unroll
   for (int w = 0; w < WAVES; ++w) t += red[w][threadIdx.x];
   Db[(int64_t)e * N + n] = from_f32<T>(t);
+}
+
+// The block's shape. 1024 threads, or 256 where no expert can have more than 128 rows (eight blocks
+// fit on a CU then). On 512 bytes of columns where that still leaves two blocks of 1024 per CU (a block of
+// 128 bytes costs about 2.5 us of waves, loads and barriers, however few its rows), else on 128 (whole
+// lines). With the weight grad's launch, bf16, us, one thread per column / 1024 threads on 128 bytes /
+// this: E = 64, N = 4096, 64 rows 21.9 / 40.3 / 22.3, 8192 rows 63.5 / 51.7 / 38.8; E = 128, N = 1536, 1024
+// rows 33.7 / 45.3 / 33.9; E = 8, N = 64, 40 rows 7.0 / 7.7 / 7.1; E = 16, N = 1032, 8002 rows 145 / 27 / 26;
+// slower only where one of many experts has every row (E = 64, N = 4096, 8192 rows 2055 / 128 / 151).
+template <typename T, int THREADS, int CH>
+void launch_bias_block(const T* DY, int64_t lddy, const int64_t* off, int64_t N, int E, T* Db, hipStream_t s) {
+  const dim3 grid((unsigned)cdiv(N, CH * (16 / (int64_t)sizeof(T))), (unsigned)E);
+  hipLaunchKernelGGL((bias_grad_kernel<T, THREADS, CH>), grid, dim3(THREADS), 0, s, DY, lddy, off, (int)N, Db);
+}
+template <typename T>
+void launch_bias_grad(const T* DY, int64_t lddy, const int64_t* off, int64_t M, int64_t N, int E, T* Db,
+                      hipStream_t s) {
+  const bool wide = E * cdiv(N, 32 * (16 / (int64_t)sizeof(T))) >= 512;
+  if (M <= 128) {
+    if (wide) launch_bias_block<T, 256, 32>(DY, lddy, off, N, E, Db, s);
+    else launch_bias_block<T, 256, 8>(DY, lddy, off, N, E, Db, s);
+  } else {
+    if (wide) launch_bias_block<T, 1024, 32>(DY, lddy, off, N, E, Db, s);
+    else launch_bias_block<T, 1024, 8>(DY, lddy, off, N, E, Db, s);
+  }
 }
 
 
@@ -3478,13 +3503,10 @@ extern "C" int zmoe_group_bwd_w(const void* DY, int64_t dy_stride_m, const void*
                                s);
   }
   if (rc || Db == nullptr) return rc;
-  const dim3 grid((unsigned)cdiv(N, 8 * v), (unsigned)E), block(kBiasThreads);
   if (dtype == ZMOE_DTYPE_BF16)
-    hipLaunchKernelGGL(bias_grad_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)DY, dy_stride_m,
-                       expert_offsets, (int)N, (uint16_t*)Db);
+    launch_bias_grad((const uint16_t*)DY, dy_stride_m, expert_offsets, M, N, E, (uint16_t*)Db, s);
   else
-    hipLaunchKernelGGL(bias_grad_kernel<float>, grid, block, 0, s, (const float*)DY, dy_stride_m, expert_offsets,
-                       (int)N, (float*)Db);
+    launch_bias_grad((const float*)DY, dy_stride_m, expert_offsets, M, N, E, (float*)Db, s);
   return check_launch("bias_grad_kernel");
 }
 

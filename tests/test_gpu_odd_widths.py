@@ -217,3 +217,24 @@ def test_bias_grad_row_counts(hip_device, dtype, N):
     # fp32 sums of up to 1300 terms ~ N(0, 1): 1300 * 2^-24 * sum|terms| bounds any order
     atol = max(TOL[dtype]["atol"], 1300 * 2.0 ** -24 * float(np.abs(np64(DY)).sum(0).max()))
     assert_close(np64(Db), ref, rtol=TOL[dtype]["rtol"], atol=atol, what="bias grad")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("counts,N", [([0, 1, 31, 32, 33, 0, 31], 264), ([0, 128], 8), ([3] * 40, 72),   # <= 128 rows
+                                      ([0, 1, 31, 32, 33, 127, 129, 400] * 16, 1024 + 8),     # wide blocks
+                                      ([257] + [0] * 255, 1024), ([1] * 129, 2000),
+                                      ([0, 33, 1, 0] + [1] * 90, 2000)])                       # both
+def test_bias_grad_block_shapes(hip_device, dtype, counts, N):
+    """The bias grad's other blocks: 256 threads where no expert can have more than 128 rows, and 512
+    bytes of columns where there are many; rows around a slot's four and a block's pass over them."""
+    from zmoe import ops
+
+    off = torch.tensor(np.cumsum(counts), device=hip_device)
+    g = gen(N + len(counts))
+    DY = torch.randn(sum(counts), N, generator=g).to(dtype)
+    X = torch.randn(sum(counts), 16, generator=g).to(dtype)
+    _, Db = ops.group_bwd_w(DY.to(hip_device), X.to(hip_device), off, len(counts), has_bias=True)
+    ref = np.stack([r.sum(0) for r in np.split(np64(DY), np.cumsum(counts)[:-1])])
+    # fp32 sums of n terms: n * 2^-24 * sum|terms| bounds any order
+    atol = max(TOL[dtype]["atol"], max(counts) * 2.0 ** -24 * float(np.abs(np64(DY)).sum(0).max()))
+    assert_close(np64(Db), ref, rtol=TOL[dtype]["rtol"], atol=atol, what="bias grad")
