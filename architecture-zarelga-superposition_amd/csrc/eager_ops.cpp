@@ -1,9 +1,9 @@
 // The layer's device ops as C++ dispatcher kernels (namespace zmoe_eager): what eager calls of
-// zmoe/library.py run with gradients off. Each takes the operands that the layer itself passes
-// (device tensors of one device, bf16 or f32 rows, int64 indices), allocates its outputs with
-// torch and makes one C-ABI call on torch's current stream. Everything else (other dtypes and
-// devices, strides the kernels do not take, bad sizes) goes to the op's general form, the Python
-// wrapper registered as zmoe::<name>, which converts, pads or raises.
+// zmoe/library.py run with gradients off, where no mode, tracer or transform watches. Each takes the
+// operands that the layer itself passes (device tensors of one device, bf16 or f32 rows, int64 indices),
+// allocates its outputs with torch and makes one C-ABI call on torch's current stream. Everything else
+// (other dtypes and devices, strides the kernels do not take, bad sizes) goes to the op's general form,
+// the Python wrapper registered as zmoe::<name>, which converts, pads or raises.
 //
 // Why native: a training step of a small layer is bound by its host work. An op costs ~20-40 us
 // through torch.library.custom_op, the Python wrapper and ctypes, ~8 us here (the training step at

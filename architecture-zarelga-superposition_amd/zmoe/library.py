@@ -8,7 +8,8 @@ functions of ``modeling.moe_layer``, ``scattermoe.mlp`` and ``zmoe.functional``
 call: ``torch.compile`` sees each launch as one opaque node whose output shapes come
 from the fake implementation, so tracing the layer needs no graph break and no host
 sync. Each op runs the ``zmoe.ops`` wrapper of the same name (the C ABI through
-ctypes) on the current stream.
+ctypes) on the current stream, or, in eager calls with gradients off that nothing watches,
+its native form (``LayerOp``).
 """
 
 from __future__ import annotations
