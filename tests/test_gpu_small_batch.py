@@ -163,3 +163,24 @@ def test_shared_expert_leaves_the_launches(hip_device, T, monkeypatch):
     assert T * 1 <= 8 * 32
     run_and_compare(T, 2048, 32, 1, 64, 24, torch.bfloat16, hip_device)
     assert len(calls) == (T == 192)
+
+
+def test_compiled_step_equals_eager(hip_device):
+    """The streaming route under torch.compile with dynamic shapes, at two token counts, and at a third
+    that leaves it."""
+    import torch._dynamo
+
+    layer = _layer(hip_device, torch.bfloat16)
+    torch._dynamo.reset()
+    fn = torch.compile(lambda x: layer(x), backend="aot_eager", dynamic=True, fullgraph=True)
+    for T in (16, 33, 300):
+        assert _streams(T, 128, 64, 64, 64, 4) == (T < 300)
+        x = torch.randn(1, T, 128, generator=gen(T)).to(torch.bfloat16).to(hip_device)
+        dout = torch.randn(1, T, 128, generator=gen(T + 1)).to(torch.bfloat16).to(hip_device)
+        ref = _step(layer, x, dout)
+        xg = x.clone().requires_grad_(True)
+        layer.zero_grad(set_to_none=True)
+        out, _ = fn(xg)
+        out.backward(dout)
+        _equal((out.detach(), xg.grad, {n: p.grad for n, p in layer.named_parameters()}), ref)
+    torch._dynamo.reset()
